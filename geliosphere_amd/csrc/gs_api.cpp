@@ -68,7 +68,7 @@ struct gs_ctx {
     uint64_t cap_border = 0;
     uint32_t *d_bcounts = nullptr;       // batches: 2 * kOrderSimBuckets words per simulation
     uint64_t cap_bcounts = 0;
-    gs::SpillRec *d_spill = nullptr;     // plain runs: two halves of cap_spill records
+    gs::SpillRec *d_spill = nullptr;     // hand-on records: two halves of cap_spill each
     uint64_t cap_spill = 0;
     // launch shape per [plain, batch][model]; zero fields take the defaults
     // (256 threads, the occupancy's blocks per CU, kChunk ids per grab)
@@ -372,13 +372,52 @@ unsigned fold_blocks(uint64_t events) {
 // produce at most one event per particle) to 2^27 x 64 B = 8.6 GB.
 const uint64_t kMaxChunk = 1ull << 27;
 const uint64_t kOrderMinParticles = 4096;   // smaller runs keep id order
-// Tail compaction of plain runs (DevOut::spill): used for 1D F-p, whose
-// lifetimes are heavy-tailed with no energy trend, and for runs of at most
-// kCompactPerLane particles per lane; continuations stop handing on below
-// kCompactMin particles, and after kCompactRounds rounds.
-const uint64_t kCompactPerLane = 16;
-const uint64_t kCompactMin = 1024;
-const int kCompactRounds = 48;
+// Tail launches (tail_kernel): after the throughput launch of a run, or instead
+// of it where the particles fit one lane each at one wave per SIMD.  Launch r
+// has kTailBudget << r cycles, the last one as many as it takes: lifetimes
+// spread over three decades, and a doubling budget repacks the survivors
+// about every time their number has halved.  Every launch is queued beforehand
+// and takes its particle count from the one before on the device; one that
+// finds none ends at once (about 3 us).
+constexpr int kTailRounds = 11;
+constexpr uint32_t kTailBudget = 128;
+
+uint64_t tail_lanes(const gs_ctx *ctx) { return (uint64_t)ctx->n_cu * 4 * gs::kWave; }
+
+// Hand-on records a run of n particles needs per half: one per lane of the
+// throughput launch, or one per particle.
+uint64_t tail_cap(const gs_ctx *ctx, uint64_t n, uint64_t traj_lanes) {
+    return std::max<uint64_t>(1, std::min<uint64_t>(n, std::max(traj_lanes, tail_lanes(ctx))));
+}
+
+// Queues the tail launches of one run on stream s.  fresh_n > 0: the run's
+// particles themselves (no throughput launch ran); otherwise those that the
+// throughput launch handed on to `half0` (counted in counts[0]).  counts: one
+// word per launch, zeroed.
+hipError_t queue_tail(const gs_ctx *ctx, int model, bool batch, const DevParams *sims, uint32_t n_sims,
+                      const uint64_t *offsets, const DevOut &O, uint64_t fresh_n, gs::SpillRec *half0,
+                      gs::SpillRec *half1, uint64_t cap, uint64_t *counts, hipStream_t s) {
+    const uint64_t lanes = tail_lanes(ctx);
+    const uint64_t most = fresh_n ? fresh_n : cap;
+    // workgroups for up to 64 lanes per particle on `lanes`, or one lane each
+    const uint64_t threads = std::min<uint64_t>(most * gs::kWave, std::max(most, lanes));
+    const unsigned grid = (unsigned)((threads + gs::kTailThreads - 1) / gs::kTailThreads);
+    const int rounds = most * gs::kWave <= lanes ? 1 : kTailRounds;   // 64 lanes each at once: no budget
+    for (int r = 0; r < rounds; ++r) {
+        gs::TailArgs A;
+        A.in = r == 0 && fresh_n ? nullptr : (r & 1) ? half1 : half0;
+        A.n_in = counts + r;
+        A.fresh_n = r == 0 ? fresh_n : 0;
+        A.out = r + 1 < rounds ? ((r & 1) ? half0 : half1) : nullptr;
+        A.n_out = counts + r + 1;
+        A.cap = cap;
+        A.budget = kTailBudget << r;
+        A.lanes = (uint32_t)lanes;
+        const hipError_t e = gs_launch_tail(model, batch, sims, n_sims, offsets, O, A, grid, s);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
 
 uint64_t event_room(int model, uint64_t n) {
     if (model == GS_MODEL_1D_FP) return std::max<uint64_t>(n / 16, 1u << 16);
@@ -472,7 +511,7 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
     }
     const size_t nl = launches.size();
     // ---- host staging: params, meta = ev_off[m] | ev_cap[m] | n_events[m] |
-    //      offsets (count+1 per launch) | queues[nl] | cycles[nl]
+    //      offsets (count+1 per launch) | queues[nl] | cycles[nl] | hand-on counts
     ctx->h_params.resize(m);
     uint32_t max_nb = 1, max_nw = 1;
     uint64_t total_room = 0;
@@ -489,7 +528,8 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
     const size_t off_base = 3 * m;
     size_t pos = off_base;
     for (Launch &L : launches) { L.off_pos = pos; pos += L.count + 1; }
-    const size_t q_base = pos, c_base = pos + nl, meta_words = pos + 2 * nl;
+    const size_t q_base = pos, c_base = pos + nl, t_base = pos + 2 * nl;   // queues, cycles, hand-on counts
+    const size_t meta_words = t_base + nl * (kTailRounds + 1);
     ctx->h_meta.assign(meta_words, 0);
     uint64_t eo = 0;
     for (size_t j = 0; j < m; ++j) {
@@ -511,6 +551,14 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
         nv[l] = v;
         perm_total += v;
     }
+    // each launch's slice of the hand-on records
+    std::vector<uint64_t> spill_at(nl), spill_cap(nl);
+    uint64_t spill_total = 0;
+    for (size_t l = 0; l < nl; ++l) {
+        spill_at[l] = spill_total;
+        spill_cap[l] = tail_cap(ctx, nv[l], (uint64_t)launches[l].grid * launches[l].block);
+        spill_total += spill_cap[l];
+    }
     const bool ordered = ctx->order_mode == GS_ORDER_ENERGY;
     gs_status st = ordered ? ensure_batch_order(ctx, std::max<uint64_t>(perm_total, 1),
                                                 2 * (uint64_t)gs::kOrderSimBuckets * m)
@@ -519,6 +567,7 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
     if (st == GS_OK) st = ensure_params(ctx, m);
     if (st == GS_OK) st = ensure_events(ctx, std::max<uint64_t>(total_room, 1));
     if (st == GS_OK) st = ensure_meta(ctx, std::max<size_t>(meta_words, 64));
+    if (st == GS_OK) st = ensure_spill(ctx, spill_total);
     if (st != GS_OK) return st;
     const Layout W = layout(ctx->d_words, m);
     const size_t lds = fold_lds_bytes(max_nb, max_nw);
@@ -528,8 +577,11 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
     // ---- graph (re)build when the layout differs from the cached one
     std::vector<uint64_t> key = {m, nl, (uint64_t)(uintptr_t)ctx->d_words, (uint64_t)(uintptr_t)ctx->d_events,
                                  (uint64_t)(uintptr_t)ctx->d_params, (uint64_t)(uintptr_t)ctx->d_meta, lds, fb,
-                                 ordered, (uint64_t)(uintptr_t)ctx->d_border, (uint64_t)(uintptr_t)ctx->d_bcounts};
-    for (const Launch &L : launches) {
+                                 ordered, (uint64_t)(uintptr_t)ctx->d_border, (uint64_t)(uintptr_t)ctx->d_bcounts,
+                                 (uint64_t)(uintptr_t)ctx->d_spill, ctx->cap_spill};
+    for (size_t l = 0; l < nl; ++l) {
+        const Launch &L = launches[l];
+        key.push_back(nv[l]);   // slices of the permutation and the records, fresh tail launches
         key.push_back((uint64_t)L.model);
         key.push_back(L.count);
         key.push_back(L.grid);
@@ -547,7 +599,7 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
         HIP_TRY(ctx, hipStreamBeginCapture(s0, hipStreamCaptureModeThreadLocal));
         hipError_t e = gs_launch_zero(ctx->d_words, m * words_per_sim(), s0);
         if (e == hipSuccess) e = gs_launch_zero(ctx->d_meta + 2 * m, m, s0);          // n_events
-        if (e == hipSuccess) e = gs_launch_zero(ctx->d_meta + q_base, 2 * nl, s0);    // queues, cycles
+        if (e == hipSuccess) e = gs_launch_zero(ctx->d_meta + q_base, meta_words - q_base, s0);   // queues, cycles, hand-on
         if (e == hipSuccess) e = hipEventRecord(ctx->fork, s0);
         // model groups on up to four streams
         std::vector<int> group_of(nl);
@@ -570,8 +622,9 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
             O.queue = ctx->d_meta + q_base + l;
             O.cycles = ctx->d_meta + c_base + l;
             O.order = nullptr;
-            O.spill = nullptr; O.spill_count = nullptr; O.spill_cap = 0;
-            O.resume = nullptr; O.resume_n = 0;
+            gs::SpillRec *half0 = ctx->d_spill + spill_at[l], *half1 = half0 + ctx->cap_spill;
+            uint64_t *counts = ctx->d_meta + t_base + l * (kTailRounds + 1);
+            O.spill = half0; O.spill_count = counts; O.spill_cap = spill_cap[l];
             O.chunk = L.chunk;
             if (ordered) {
                 e = gs_launch_batch_order(ctx->d_params + L.base, L.count, ctx->d_meta + L.off_pos, nv[l],
@@ -587,8 +640,13 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
             O.ev_off = ctx->d_meta + L.base;
             O.ev_cap = ctx->d_meta + m + L.base;
             O.n_events = ctx->d_meta + 2 * m + L.base;
-            e = gs_launch_traj(L.model, true, ctx->d_params + L.base, L.count, ctx->d_meta + L.off_pos, O,
-                               L.grid, L.block, sg);
+            const bool fresh = nv[l] > 0 && nv[l] <= tail_lanes(ctx);
+            if (!fresh)
+                e = gs_launch_traj(L.model, true, ctx->d_params + L.base, L.count, ctx->d_meta + L.off_pos, O,
+                                   L.grid, L.block, sg);
+            if (e == hipSuccess && nv[l] > 0)
+                e = queue_tail(ctx, L.model, true, ctx->d_params + L.base, L.count, ctx->d_meta + L.off_pos, O,
+                               fresh ? nv[l] : 0, half0, half1, spill_cap[l], counts, sg);
         }
         for (int g = 0; g < 3 && e == hipSuccess; ++g) {
             if (!used[g]) continue;
@@ -599,7 +657,6 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
             DevOut O;
             O.queue = nullptr; O.cycles = nullptr; O.order = nullptr;
             O.spill = nullptr; O.spill_count = nullptr; O.spill_cap = 0;
-            O.resume = nullptr; O.resume_n = 0;
             O.chunk = 0;
             O.g_count = W.count; O.g_digits = W.digits; O.g_stats = W.stats;
             O.events = ctx->d_events;
@@ -661,12 +718,14 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
 }
 
 // Device buffers of one plain run.  meta: [0] event offset (0), [1] event
-// capacity, [2] event count, [3] cycles, [4..5] hand-on counts,
-// [8 .. 8+ST_COUNT_) statistics saved before a chunk.
+// capacity, [2] event count, [3] cycles, [4 .. 4+kTailRounds] hand-on counts,
+// [kMetaSaved ..) statistics saved before a chunk.
 // own = true: the context's buffers, which grow on demand (event region,
 // order permutation, hand-on records).  own = false: fixed buffers (events,
 // order_counts and order of cap_events entries); no exit records, no
 // hand-on, and chunks are cut to fit the fixed event region.
+constexpr int kMetaSaved = 32;
+static_assert(4 + kTailRounds + 1 <= kMetaSaved && kMetaSaved + gs::ST_COUNT_ <= 64, "plain run's meta words");
 struct PlainBufs {
     uint64_t *words;
     DevParams *params;
@@ -703,7 +762,6 @@ gs_status run_plain_core(gs_ctx *ctx, const gs_params &pp, gs_spectrum *out, gs_
     O.cycles = B.meta + 3;
     O.order = nullptr;
     O.spill = nullptr; O.spill_count = nullptr; O.spill_cap = 0;
-    O.resume = nullptr; O.resume_n = 0;
     O.chunk = RS.chunk;
     const uint64_t lanes = (uint64_t)grid * RS.block;
     // largest chunk: 2^27 particles, or what the fixed event region holds
@@ -744,46 +802,29 @@ gs_status run_plain_core(gs_ctx *ctx, const gs_params &pp, gs_spectrum *out, gs_
             O.order = perm;
         }
         // statistics before the chunk, restored if it has to run again
-        HIP_TRY(ctx, hipMemcpyAsync(B.meta + 8, L.stats, gs::ST_COUNT_ * sizeof(uint64_t),
+        HIP_TRY(ctx, hipMemcpyAsync(B.meta + kMetaSaved, L.stats, gs::ST_COUNT_ * sizeof(uint64_t),
                                     hipMemcpyDeviceToDevice, ctx->stream));
         hm[0] = 0;
         hm[1] = cap;
         HIP_TRY(ctx, hipMemcpyAsync(B.meta, hm, 2 * sizeof(uint64_t), hipMemcpyHostToDevice, ctx->stream));
         HIP_TRY(ctx, gs_launch_zero(L.queue, 1, ctx->stream));
-        HIP_TRY(ctx, gs_launch_zero(B.meta + 2, 4, ctx->stream));   // events, cycles, hand-on counts
+        HIP_TRY(ctx, gs_launch_zero(B.meta + 2, 2 + kTailRounds + 1, ctx->stream));   // events, cycles, hand-on counts
         O.events = events;
-        const bool compact = B.own && (q.model == GS_MODEL_1D_FP || q.n_particles <= kCompactPerLane * lanes);
-        if (compact) {
-            st = ensure_spill(ctx, lanes);   // at most one hand-on per lane and launch
+        // the tail needs the context's record buffer
+        const uint64_t cap_tail = tail_cap(ctx, q.n_particles, lanes);
+        const bool fresh = B.own && q.n_particles > 0 && q.n_particles <= tail_lanes(ctx);
+        if (B.own) {
+            st = ensure_spill(ctx, cap_tail);
             if (st != GS_OK) return st;
+            O.spill = ctx->d_spill;
+            O.spill_count = B.meta + 4;
+            O.spill_cap = cap_tail;
         }
-        O.resume = nullptr;
-        O.resume_n = 0;
-        O.spill = compact ? ctx->d_spill : nullptr;
-        O.spill_count = B.meta + 4;
-        O.spill_cap = compact ? ctx->cap_spill : 0;
         HIP_TRY(ctx, hipEventRecord(ctx->ev0, ctx->stream));
-        HIP_TRY(ctx, gs_launch_traj(q.model, false, B.params, 1, nullptr, O, grid, RS.block, ctx->stream));
-        // continuations: the handed-on particles, packed into full waves
-        for (int round = 0, cur = 0; compact; ++round, cur ^= 1) {
-            uint64_t pending = 0;
-            HIP_TRY(ctx, hipMemcpyAsync(&pending, B.meta + 4 + cur, sizeof pending, hipMemcpyDeviceToHost,
-                                        ctx->stream));
-            HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-            pending = std::min(pending, O.spill_cap);   // slots beyond the cap were not handed on
-            if (pending == 0) break;
-            HIP_TRY(ctx, gs_launch_zero(L.queue, 1, ctx->stream));
-            HIP_TRY(ctx, gs_launch_zero(B.meta + 4 + (cur ^ 1), 1, ctx->stream));
-            O.resume = ctx->d_spill + (size_t)cur * ctx->cap_spill;
-            O.resume_n = pending;
-            O.spill = pending > kCompactMin && round + 1 < kCompactRounds
-                          ? ctx->d_spill + (size_t)(cur ^ 1) * ctx->cap_spill : nullptr;
-            O.spill_count = B.meta + 4 + (cur ^ 1);
-            const unsigned g2 = (unsigned)std::min<uint64_t>(grid, (pending + RS.block - 1) / RS.block);
-            HIP_TRY(ctx, gs_launch_traj(q.model, false, B.params, 1, nullptr, O, g2, RS.block, ctx->stream));
-        }
-        O.resume = nullptr;
-        O.spill = nullptr;
+        if (!fresh) HIP_TRY(ctx, gs_launch_traj(q.model, false, B.params, 1, nullptr, O, grid, RS.block, ctx->stream));
+        if (B.own && q.n_particles > 0)
+            HIP_TRY(ctx, queue_tail(ctx, q.model, false, B.params, 1, nullptr, O, fresh ? q.n_particles : 0, ctx->d_spill,
+                                    ctx->d_spill + ctx->cap_spill, cap_tail, B.meta + 4, ctx->stream));
         HIP_TRY(ctx, hipEventRecord(ctx->ev1, ctx->stream));
         uint64_t nev = 0;
         HIP_TRY(ctx, hipMemcpyAsync(&nev, B.meta + 2, sizeof nev, hipMemcpyDeviceToHost, ctx->stream));
@@ -796,7 +837,7 @@ gs_status run_plain_core(gs_ctx *ctx, const gs_params &pp, gs_spectrum *out, gs_
             // the chunk again from the statistics saved before it, with room
             // for its nev events where the limit allows, else as half as
             // many particles.
-            HIP_TRY(ctx, hipMemcpyAsync(L.stats, B.meta + 8, gs::ST_COUNT_ * sizeof(uint64_t),
+            HIP_TRY(ctx, hipMemcpyAsync(L.stats, B.meta + kMetaSaved, gs::ST_COUNT_ * sizeof(uint64_t),
                                         hipMemcpyDeviceToDevice, ctx->stream));
             if (B.own && !grown && nev <= ev_limit) {
                 st = ensure_events(ctx, std::min(nev + nev / 8, ev_limit));

@@ -278,6 +278,25 @@ __device__ void fold_one(const DevParams &P, uint64_t *lds, const DevEvent &e) {
 // emit(t_inj, t_exit, r, theta, sumac) where they happen, so that nothing of
 // an event stays live in registers on the common path.  `trig` is the
 // workgroup's LDS copy of the sin/cos table (the 2D models' sin and cos).
+//
+// fast_step is the same step for a particle to which nothing happens: no exit,
+// end, crossing or reflection (2D: between the polar caps).  It has no branch
+// and updates the state with the same operations, bit for bit; a Watch gathers
+// what tells afterwards whether it was allowed.  A cycle runs fast steps for
+// every lane, tests Watch once, and takes back and repeats with step() the
+// lanes whose Watch says no (run_cycle in gs_kernels.hip).  The tests are
+// conservative: a lane may be repeated although nothing happened to it.
+// What it replaces: per step three or more f64 compares, the step counter and
+// three divergent branches.  A branch on a vector compare costs a lone wave
+// about 50 cycles (measured: a dependent f64 fused multiply-add 6 cycles, with
+// a compare and a branch not taken 63), so the branches took a third of a 1D
+// step there.
+//
+// Radii are watched through the high words of their doubles: unsigned, these
+// grow with a positive double, and those of negative numbers and NaNs lie
+// above all positive ones; max3/min3 take two steps per instruction.
+constexpr uint32_t hi_word(double x) { return (uint32_t)(__builtin_bit_cast(uint64_t, x) >> 32); }
+__device__ __forceinline__ uint32_t hi_of(double x) { return (uint32_t)(fm::double_to_bits(x) >> 32); }
 
 // The 1D models carry momenta in units of T0: P = pc / (q T0 1e9), so that
 // E^2 = P^2 + 1 takes the inline constant 1.0.  K = K0 beta P [GV] enters
@@ -351,6 +370,27 @@ struct Bp {
         }
         return alive;
     }
+    // Nothing happens while 0.31 < r < 99.99 after each step and beta stays
+    // above 0.01: P grows from step to step (V > 0, r > 0), so it is enough that
+    // the first P of the cycle lies above 0.0101 (beta = 0.0100995), and the
+    // last is neither below that nor NaN.
+    struct Watch { uint32_t hmax, hmin; };
+    static constexpr uint32_t kRLo = hi_word(0.31), kRHi = hi_word(99.99), kPLo = hi_word(0.0101), kInf = 0x7ff00000u;
+    __device__ __forceinline__ Watch watch() const { return {0u, 0xffffffffu}; }
+    __device__ __forceinline__ void fast_step(const StepParams &Pm, const double *z, const double *trig, Watch &W) {
+        const double inv_r = fm::rcp(r);
+        const double sK = Pm.sk2dt * w;
+        P = fma(-(Pm.cp * P), inv_r, P);
+        r = r + (sK * fma(sK, inv_r, z[0]) + Pm.vdt);
+        w = P * fm::rsqrt4(fma(P, P, 1.0));
+        const uint32_t h = hi_of(r);
+        W.hmax = max(W.hmax, h);
+        W.hmin = min(W.hmin, h);
+    }
+    __device__ __forceinline__ bool fast_ok(const Watch &W, const Bp &old) const {
+        return W.hmax < kRHi && W.hmin > kRLo && hi_of(old.P) - (kPLo + 1) < kInf - (kPLo + 1) &&
+               hi_of(P) - (kPLo + 1) < kInf - (kPLo + 1);
+    }
 };
 
 // 1D F-p.  State: r, P (units of T0), beta of the last computed T, w =
@@ -419,6 +459,31 @@ struct Fp {
         P = refl ? P : Pn;
         return !stop && rn < 100.0002;
     }
+    // Nothing happens while r stays between 1.01 and 100.00018 (the start of
+    // the cycle included: a crossing looks at both ends of a step; particles
+    // start at 100.0001, one unit of the high word above 100, and end at
+    // 100.0002, three above) and beta stays above 0.01: P falls from step to
+    // step, so the lowest beta is the last one, or, after a reflection before
+    // the cycle (beta then belongs to a discarded P), the first.
+    struct Watch { uint32_t hmax, hmin; };
+    static constexpr uint32_t kRLo = hi_word(1.01), kRHi = hi_word(100.0002);
+    __device__ __forceinline__ Watch watch() const { return {hi_of(r), hi_of(r)}; }
+    __device__ __forceinline__ void fast_step(const StepParams &Pm, const double *z, const double *trig, Watch &W) {
+        const double inv_r = fm::rcp(r);
+        const double sK = Pm.sk2dt * w;
+        P = fma(-(Pm.cp * P), inv_r, P);
+        sumac = fma(Pm.csum, inv_r, sumac);
+        r = r + (sK * fma(sK, inv_r, z[0]) + Pm.vdt);
+        const double q = fm::rsqrt4(fma(P, P, 1.0));
+        w = P * q;
+        beta = w * q;
+        const uint32_t h = hi_of(r);
+        W.hmax = max(W.hmax, h);
+        W.hmin = min(W.hmin, h);
+    }
+    __device__ __forceinline__ bool fast_ok(const Watch &W, const Fp &old) const {
+        return W.hmax < kRHi && W.hmin > kRLo && beta >= 0.01 && old.beta >= 0.01;
+    }
 };
 
 
@@ -441,15 +506,47 @@ struct Sp {
     }
     template <class Emit>
     __device__ __forceinline__ bool step(const StepParams &Pm, const double *z, const double *trig, const Emit &emit) {
-#pragma clang fp contract(fast)
+        advance(Pm, z, trig);
+        theta = fabs(theta);   // theta < 0 -> |theta| (also takes -0 to +0)
+        if (theta > kPi) {
+            asm volatile("");   // emits nothing; a pole crossing is rare: no selects on the common path
+            theta = theta > 2.0 * kPi ? theta - (2.0 * kPi) : (2.0 * kPi) - theta;
+        }
+        r = fabs(r);           // r < 0 -> -r
+        if (r > 100.0) {
+            emit(t_inj, T, r, theta, 0.0);
+            return false;
+        }
+        return r < 100.0;
+    }
+    // Nothing happens while 0 <= r < 100 after each step.  Pole crossings are
+    // part of the fast step (in the Geliosphere model a particle near a pole
+    // crosses it in every second step): fmin(theta, |2 pi - theta|) is step()'s
+    // theta bit for bit.  A NaN theta makes the next r NaN.
+    struct Watch { uint32_t hmax; };
+    static constexpr uint32_t kRHi = hi_word(100.0);
+    __device__ __forceinline__ Watch watch() const { return {0u}; }
+    __device__ __forceinline__ void fast_step(const StepParams &Pm, const double *z, const double *trig, Watch &W) {
+        advance(Pm, z, trig);
+        theta = fmin(fabs(theta), fabs(2.0 * kPi - fabs(theta)));
+        W.hmax = max(W.hmax, hi_of(r));
+    }
+    __device__ __forceinline__ bool fast_ok(const Watch &W, const Sp &old) const { return W.hmax < kRHi; }
+
+    // One Euler step of r, theta and T before the reflections and the exit.
+    // Every fused multiply-add is written out (contraction is off): the 2D
+    // models amplify a last-bit difference into another trajectory, so the
+    // rounding must not depend on what surrounds the inlined step.
+    __device__ __forceinline__ void advance(const StepParams &Pm, const double *z, const double *trig) {
         double s, c;
         fm::sincosd(theta, trig, s, c);
         const double Tp = T + 2.0 * kT0;
         const double Rig = fm::sqrt_nn(T * Tp);
         const double r2 = r * r;
         const double gamma = r * Pm.omega_v * s;
-        const double g2 = gamma * gamma;
-        const double opg = 1.0 + g2;
+        const double opg = fma(gamma, gamma, 1.0);   // 1 + gamma^2
+        const double tpg = fma(gamma, gamma, 2.0);   // 2 + gamma^2
+        const double tmg = 2.0 - gamma * gamma;      // 2 - gamma^2
         double inv_E, inv_r, inv_opg, inv_s;
         fm::rcp4(T + kT0, r, opg, s, inv_E, inv_r, inv_opg, inv_s);
         const double beta = Rig * inv_E;
@@ -469,37 +566,26 @@ struct Sp {
         // = C K0 beta P r [ratio (2 + g^2) / (1+g^2)^1.5 + (1 - ratio) (2 - g^2) / (1+g^2)^2.5],
         // since 5/(3 3.4) = (5/3.4)/3 = C.
         const double krc = kbc * Rig * r;
-        const double dKrr = krc * fma(Pm.ratio * (2.0 + g2), inv_opg15, (1.0 - Pm.ratio) * (2.0 - g2) * inv_opg25);
+        const double dKrr = krc * fma(Pm.ratio * tpg, inv_opg15, (1.0 - Pm.ratio) * tmg * inv_opg25);
         const double sKrr = fm::sqrt_nn(Pm.two_dt * Krr);
         const double sKtt = fm::sqrt_nn(Pm.two_dt * Kper);
         double dr = fma(fma(2.0 * Krr, inv_r, dKrr) - Pm.V, Pm.dt, z[0] * sKrr);
         const double cs = c * inv_s;
         double dth = fma(Kper * cs * inv_r * inv_r * inv_opg, Pm.dt, z[1] * sKtt * inv_r);
-        const double dTkin = -Pm.cp * (Tp * inv_E) * T * inv_r;
         // drifts: sheet angle alphaM + 2 Larmor pi / (180 r), Larmor = (0.0225 / A) P r^2 / sq
         const double sy = fm::sind(fma(Rig * r * inv_sq, (0.0225 / kA) * (kPi / 90.0), Pm.tilt), trig);
         double f, g;
-        fm::sheet_drift<fm::DevOps>(sy, 1.0 - theta * (2.0 / kPi), trig + fm::kBmTrigWords, f, g);
+        fm::sheet_drift<fm::DevOps>(sy, fma(theta, -(2.0 / kPi), 1.0), trig + fm::kBmTrigWords, f, g);
         const double rbg = Rig * beta * r * gamma * inv_opg;
         const double dc = rbg * ((kKonvF * (2.0 / (3.0 * kA))) * f) * inv_opg;
         // (DriftR + DriftSheetR) dt, with fprime = -(2/pi) g
         dr = fma(Pm.poldt, fma(dc, cs, (kKonvF * (1.0 / (3.0 * kA)) * (-2.0 / kPi)) * rbg * g), dr);
         // DriftTheta dt / r
-        dth = fma(-Pm.polthdt * dc * (2.0 + g2), inv_r, dth);
+        dth = fma(-Pm.polthdt * dc * tpg, inv_r, dth);
         r = r + dr;
         theta = theta + dth;
-        theta = fabs(theta);   // theta < 0 -> |theta| (also takes -0 to +0)
-        if (theta > kPi) {
-            asm volatile("");   // emits nothing; a pole crossing is rare: no selects on the common path
-            theta = theta > 2.0 * kPi ? theta - (2.0 * kPi) : (2.0 * kPi) - theta;
-        }
-        T = T - dTkin;
-        r = fabs(r);           // r < 0 -> -r
-        if (r > 100.0) {
-            emit(t_inj, T, r, theta, 0.0);
-            return false;
-        }
-        return r < 100.0;
+        // the energy loss (2/3) V dt (Tp / E) T / r
+        T = fma(Pm.cp * (Tp * inv_E) * T, inv_r, T);
     }
 };
 
@@ -523,7 +609,34 @@ struct Ge {
     }
     template <class Emit>
     __device__ __forceinline__ bool step(const StepParams &Pm, const double *z, const double *trig, const Emit &emit) {
-#pragma clang fp contract(fast)
+        advance(Pm, z, trig);
+        theta = fabs(theta);   // theta < 0 -> |theta| (also takes -0 to +0)
+        if (theta > kPi) {
+            asm volatile("");   // emits nothing; a pole crossing is rare: no selects on the common path
+            theta = theta > 2.0 * kPi ? theta - (2.0 * kPi) : (2.0 * kPi) - theta;
+        }
+        r = fabs(r);           // r < 0 -> -r
+        if (r > 100.0) {
+            emit(t_inj, T, r, theta, 0.0);
+            return false;
+        }
+        return r < 100.0;
+    }
+    // As in Sp.  The polar caps stay branches inside the step: a particle may stay
+    // in one for long, and at 64 lanes a wave has one there in one cycle of five.
+    struct Watch { uint32_t hmax; };
+    static constexpr uint32_t kRHi = hi_word(100.0);
+    __device__ __forceinline__ Watch watch() const { return {0u}; }
+    __device__ __forceinline__ void fast_step(const StepParams &Pm, const double *z, const double *trig, Watch &W) {
+        advance(Pm, z, trig);
+        theta = fmin(fabs(theta), fabs(2.0 * kPi - fabs(theta)));
+        W.hmax = max(W.hmax, hi_of(r));
+    }
+    __device__ __forceinline__ bool fast_ok(const Watch &W, const Ge &old) const { return W.hmax < kRHi; }
+
+    // One Euler step of r, theta and T before the reflections and the exit
+    // (fused multiply-adds written out, as in Sp).
+    __device__ __forceinline__ void advance(const StepParams &Pm, const double *z, const double *trig) {
         // The reference's factors are regrouped so that each per-simulation
         // product is formed once on the host (StepParams ge_*): with
         // C = (5/3.4)/3, kf = 1/(3 (5/3.4)) and kbrc = C K0 beta P,
@@ -559,7 +672,7 @@ struct Ge {
         const double gamma = r * Pm.omega_v * s;
         const double g2 = gamma * gamma;
         const double rd2 = r2 * deltarh2;
-        const double h = rd2 + g2;                    // Cb - 1
+        const double h = fma(r2, deltarh2, g2);       // Cb - 1
         const double Cb = 1.0 + h;
         const double inv_Cb = fm::rcp(Cb);
         const double sqCb = fm::sqrt_nn(Cb);
@@ -568,9 +681,9 @@ struct Ge {
         const double inv_Cb25 = inv_Cb * inv_Cb15;
         const double Rc = fmax(Rig, 0.1);   // P below 0.1 GV counts as 0.1
         const double kbc = Pm.ge_k0c * beta;          // C K0 beta
-        const double Kpar = kbc * Rc * r2 * inv_sqCb;
-        const double Kper = Pm.ratio * Kpar;
-        const double dKc = (Kpar - Kper) * inv_Cb;    // (K_par - K_per) / Cb
+        const double kpr = kbc * Rc * r2;
+        const double Kper = Pm.ratio * (kpr * inv_sqCb);
+        const double dKc = fma(kpr, inv_sqCb, -Kper) * inv_Cb;   // (K_par - K_per) / Cb
         const double Krr = Kper + dKc;
         const double Ktt = fma(rd2, dKc, Kper);
         const double Krt = deltarh * r * dKc;
@@ -599,22 +712,22 @@ struct Ge {
             const double d2 = Pm.delta0_rh * Pm.delta0_rh;
             const double inv_s2 = inv_s * inv_s;
             const double inv_s3 = inv_s2 * inv_s;
-            CKtt = CKtt - r2 * d2 * c * inv_s3;
-            const double dKtt1 = -Pm.ge_a1 * kr2c * CKtt * inv_Cb15;
+            CKtt = fma(-(r2 * d2 * c), inv_s3, CKtt);
+            const double dKtt1 = -(Pm.ge_a1 * kr2c * CKtt * inv_Cb15);
             const double dKtt2 = (Pm.ge_a3 * (1.0 / 3.0)) * kr2c * r2 * d2;
-            const double dKtt3 = -2.0 * c * inv_s3 * kGeKf * inv_Cb15;
             const double dKtt4 = 3.0 * CKtt * inv_s2 * kGeKf * inv_Cb25;
-            dKtt = dKtt1 + dKtt2 * (dKtt3 - dKtt4);
-            dKrtt = -q * r * Pm.delta0_rh * c * inv_s2 * (1.0 - (2.0 * rd2) + (4.0 * g2));
+            // dKtt3 - dKtt4 with dKtt3 = -2 c / s^3 kf / Cb^1.5
+            const double dKtt34 = fma(-2.0 * c * inv_s3 * kGeKf, inv_Cb15, -dKtt4);
+            dKtt = fma(dKtt2, dKtt34, dKtt1);
+            dKrtt = -q * r * Pm.delta0_rh * c * inv_s2 * fma(4.0, g2, fma(-2.0, rd2, 1.0));
         }
-        double dr = fma(fma(fma(Krt, csi, 2.0 * Krr + dKrtt), inv_r, dKrr) - Pm.V, Pm.dt, fma(z[0], B11, z[1] * B12));
-        double dth = fma(fma(fma(Ktt, csi, dKtt), inv_r, 2.0 * Krt) * inv_r + dKrtr, Pm.dt, z[2] * B22);
-        const double dTkin = -Pm.cp * (Tp * inv_E) * T * inv_r;
+        double dr = fma(fma(fma(Krt, csi, fma(2.0, Krr, dKrtt)), inv_r, dKrr) - Pm.V, Pm.dt, fma(z[0], B11, z[1] * B12));
+        double dth = fma(fma(fma(fma(Ktt, csi, dKtt), inv_r, 2.0 * Krt), inv_r, dKrtr), Pm.dt, z[2] * B22);
         // drifts (Kappl 2016 Eq. 26, 32-37 with Cb in place of 1 + gamma^2); sheet
         // angle alphaM + 2 Larmor pi / (180 r), Larmor = (0.0225 / A) P r^2 / sqrt(Cb)
         const double sy = fm::sind(fma(Rig * r * inv_sqCb, (0.0225 / kA) * (kPi / 90.0), Pm.tilt), trig);
         double f, g;
-        fm::sheet_drift<fm::DevOps>(sy, 1.0 - theta * (2.0 / kPi), trig + fm::kBmTrigWords, f, g);
+        fm::sheet_drift<fm::DevOps>(sy, fma(theta, -(2.0 / kPi), 1.0), trig + fm::kBmTrigWords, f, g);
         const double rbg = Rig * beta * r * gamma * inv_Cb;
         const double dc = rbg * ((kKonvF * (2.0 / (3.0 * kA))) * f) * inv_Cb;
         // (DriftR + DriftSheetR) dt, with fprime = -(2/pi) g
@@ -623,18 +736,7 @@ struct Ge {
         dth = fma(-Pm.poldt * dc * (2.0 + g2), inv_r, dth);
         r = r + dr;
         theta = theta + dth;
-        T = T - dTkin;
-        theta = fabs(theta);   // theta < 0 -> |theta| (also takes -0 to +0)
-        if (theta > kPi) {
-            asm volatile("");   // emits nothing; a pole crossing is rare: no selects on the common path
-            theta = theta > 2.0 * kPi ? theta - (2.0 * kPi) : (2.0 * kPi) - theta;
-        }
-        r = fabs(r);           // r < 0 -> -r
-        if (r > 100.0) {
-            emit(t_inj, T, r, theta, 0.0);
-            return false;
-        }
-        return r < 100.0;
+        T = fma(Pm.cp * (Tp * inv_E) * T, inv_r, T);
     }
 };
 

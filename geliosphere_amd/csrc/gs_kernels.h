@@ -105,17 +105,21 @@ struct alignas(64) DevEvent {
 };
 static_assert(sizeof(DevEvent) == 64, "DevEvent is one 64-byte line");
 
-// A live particle handed from one plain launch to the next (see DevOut):
-// the model's state, its id, steps taken and next Philox block.  The
-// counter-based normal stream makes the continuation exact.
+// A live particle handed from one launch to the next (see DevOut): the model's
+// state, its id, the steps taken and its simulation within the launch.  Handed
+// on only between cycles, where the next Philox block is steps / 4 * normals
+// per step; the counter-based normal stream makes the continuation exact.
 struct alignas(64) SpillRec {
     double s[6];
     uint64_t pid;
-    uint32_t steps, blk;
+    uint32_t steps, sim;
 };
 static_assert(sizeof(SpillRec) == 64, "SpillRec is one 64-byte line");
-constexpr int kSpillLanes = 16;      // a wave at or below this many live lanes hands them on
-constexpr uint32_t kSpillMinCycles = 4;   // after at least this many cycles in its launch
+// Cycles a wave of a throughput launch runs on after the ids have run out,
+// before it hands its live particles to the tail launches.
+constexpr uint32_t kDrainCycles = 64;
+// Cycles between two looks at the queue by a wave without an idle lane.
+constexpr uint32_t kQueuePoll = 64;
 
 // Device buffers of a launch over n_sims simulations (plain runs: 1).
 // Per simulation s: histogram count[GS_MAX_BINS], digits[GS_MAX_WEIGHTS][2]
@@ -133,22 +137,33 @@ struct DevOut {
     uint64_t *cycles;         // wave cycles issued by the launch
     const uint32_t *order;    // queue position (plain) or virtual id (batch) -> particle offset
                               // within its simulation (nullptr: identity)
-    // Plain runs only.  Tail compaction: once the queue is exhausted, a wave
-    // with at most kSpillLanes live lanes writes them to spill[*spill_count++]
-    // and exits (spill == nullptr: never).  Slots at or beyond spill_cap are
-    // not written: such particles go on in place.  A continuation launch
-    // takes its particles from resume[0 .. resume_n) instead of the queue of
-    // new ids.
+    // Hand-on: kDrainCycles after the queue is exhausted a wave writes its live
+    // particles to spill[*spill_count ..] and exits (spill == nullptr: never).
+    // spill_cap has room for one particle per lane of the launch.
     SpillRec *spill;
     uint64_t *spill_count;
     uint64_t spill_cap;
-    const SpillRec *resume;
-    uint64_t resume_n;
     // Particle ids a wave takes from the queue per grab (0: kChunk): larger
     // grabs mean fewer queue atomics, smaller ones a finer share-out of the
     // last particles among the waves.
     uint32_t chunk;
 };
+
+// One tail launch (see tail_kernel): live particles in[0 .. *n_in), or, with
+// in == nullptr, the fresh_n new particles of the launch's queue order.  What
+// still lives after `budget` cycles goes to out[*n_out ..) (out == nullptr:
+// none, run to the end).
+struct TailArgs {
+    const SpillRec *in;
+    const uint64_t *n_in;
+    uint64_t fresh_n;
+    SpillRec *out;
+    uint64_t *n_out;
+    uint64_t cap;            // records in `in` and `out`
+    uint32_t budget;
+    uint32_t lanes;          // lanes to spread the particles over (one wave per SIMD)
+};
+constexpr int kTailThreads = 256;
 
 // LDS layout per workgroup: count[n_bins] | digits[n_weights][2][n_bins][16] | stat[ST_COUNT_]
 __host__ __device__ inline int lds_words(int nb, int nw) {
@@ -188,6 +203,11 @@ hipError_t gs_traj_occupancy(int model, bool batch, unsigned block_threads, int 
 hipError_t gs_launch_traj(int model, bool batch, const gs::DevParams *sims, uint32_t n_sims,
                           const uint64_t *offsets, const gs::DevOut &O, unsigned grid,
                           unsigned block_threads, hipStream_t s);
+// One tail launch of `model` over `grid` workgroups of kTailThreads; grid must
+// hold one lane per particle.
+hipError_t gs_launch_tail(int model, bool batch, const gs::DevParams *sims, uint32_t n_sims,
+                          const uint64_t *offsets, const gs::DevOut &O, const gs::TailArgs &A, unsigned grid,
+                          hipStream_t s);
 // Scheduling order of the n = sims->n_particles particles of one plain
 // simulation: perm[0 .. n) receives the offsets 0 .. n-1 in ascending bucket
 // order (within a bucket in no fixed order).  counts: 2 * key.nb words of

@@ -19,6 +19,13 @@
 
 namespace gs {
 
+// Lane 0's value, known to the compiler to be wave-uniform (all 64 lanes must
+// be active).
+__device__ __forceinline__ uint64_t from_lane0(uint64_t v) {
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v), hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    return ((uint64_t)hi << 32) | lo;
+}
+
 // Append one event to its simulation's event region (counted even when the
 // region is full; the host then runs the simulation again with more room).
 __device__ __forceinline__ void emit_event(const DevOut &O, uint64_t pid, uint32_t sim, double t_inj, double t_exit,
@@ -122,7 +129,7 @@ __device__ __forceinline__ void stage_flush(St *st, const DevOut &O, uint32_t mi
     }
     unsigned long long base = 0;
     if (lane == 0) base = atomicAdd((unsigned long long *)&O.n_events[sim], (unsigned long long)c);
-    base = __shfl(base, 0);
+    base = from_lane0(base);
     const uint64_t cap = O.ev_cap[sim];
     uint64_t *g = (uint64_t *)(O.events + O.ev_off[sim]);
     for (uint32_t i = (uint32_t)lane; i < c * kRecWords; i += kWave) {
@@ -145,6 +152,74 @@ __device__ __forceinline__ void flush_sim_stats(const DevOut &O, uint32_t sim, u
     if (capped) atomicAdd(&g[ST_CAP], (unsigned long long)capped);
 }
 
+// Normals of step s of a cycle whose first Philox block is blk: the cycle's
+// normals NPS s .. NPS s + NPS - 1 (used where a cycle is repeated).
+template <int NPS>
+__device__ __forceinline__ void normals_of_step(uint64_t pid, uint32_t blk, int s, uint32_t k0, uint32_t k1,
+                                                const BmTables &bm, double *z) {
+    for (int i = 0; i < NPS; ++i) {
+        const int j = NPS * s + i;
+        double t[4];
+        normal_block(pid, blk + (uint32_t)(j >> 2), k0, k1, bm, t);
+        z[i] = (j & 2) ? ((j & 1) ? t[3] : t[2]) : ((j & 1) ? t[1] : t[0]);
+    }
+}
+
+// What a lane has gathered about its particles.
+struct LaneStats {
+    uint64_t steps;
+    uint32_t particles, nan, cap, max_steps;
+    // The lane's particle has ended after `n` steps.
+    template <class Model>
+    __device__ __forceinline__ void ended(const Model &m, uint32_t n) {
+        steps += n;
+        max_steps = n > max_steps ? n : max_steps;
+        if (isnan(m.r)) ++nan;
+    }
+};
+
+// Plain runs: lane statistics into the workgroup's words, and those into the
+// simulation's.
+__device__ __forceinline__ void flush_lane_stats(uint64_t *stat, const LaneStats &st) {
+    if (st.steps) atomicAdd((unsigned long long *)&stat[ST_STEPS], (unsigned long long)st.steps);
+    if (st.particles) atomicAdd((unsigned long long *)&stat[ST_PARTICLES], (unsigned long long)st.particles);
+    if (st.nan) atomicAdd((unsigned long long *)&stat[ST_NAN], (unsigned long long)st.nan);
+    if (st.cap) atomicAdd((unsigned long long *)&stat[ST_CAP], (unsigned long long)st.cap);
+    if (st.max_steps) atomicMax((unsigned long long *)&stat[ST_MAX_STEPS], (unsigned long long)st.max_steps);
+}
+__device__ __forceinline__ void flush_block_stats(const uint64_t *stat, const DevOut &O) {
+    if (threadIdx.x < ST_COUNT_ && stat[threadIdx.x]) {
+        unsigned long long *g = (unsigned long long *)&O.g_stats[threadIdx.x];
+        if (threadIdx.x == ST_MAX_STEPS) atomicMax(g, (unsigned long long)stat[threadIdx.x]);
+        else atomicAdd(g, (unsigned long long)stat[threadIdx.x]);
+    }
+}
+
+// The cycle of a lane to which something happens (or the step cap comes
+// near): up to kCycleSteps full steps.  Returns whether the particle goes on;
+// `steps` counts the steps taken.
+template <class Model, class Prm, class Normals, class Emit>
+__device__ __forceinline__ bool slow_cycle(Model &m, const Prm &P, const Normals &normals, const double *trig,
+                                           uint32_t cap, uint32_t &steps, LaneStats &st, const Emit &emit) {
+    bool active = true;
+#pragma unroll 1
+    for (int s = 0; s < kCycleSteps; ++s) {
+        double z[Model::kNormals];
+        normals(s, z);
+        if (active) {
+            if (steps >= cap) {
+                ++st.cap;
+                active = false;
+            } else {
+                ++steps;
+                if (!m.step(P, z, trig, emit)) active = false;
+            }
+        }
+    }
+    if (!active) st.ended(m, steps);
+    return active;
+}
+
 // The lanes of one wave integrate particles until the id space is exhausted.
 //
 // kBatch = false: one simulation, parameters read wave-uniformly from sims[0];
@@ -156,6 +231,11 @@ __device__ __forceinline__ void flush_sim_stats(const DevOut &O, uint32_t sim, u
 //   the old one and loads the new one's step parameters, Philox key and step
 //   cap into registers.  A wave only ever moves forward in the id space, so a
 //   lane's simulation index never decreases.
+//
+// A cycle runs fast_step for all lanes (lanes without a particle compute on
+// whatever state they hold, which nothing reads), then repeats it with full
+// steps for the lanes whose Watch asks for that: about 1 in 5000 lane-cycles
+// of a 1D B-p run, 5 % of wave-cycles.
 template <class Model, bool kBatch, class St>
 __device__ void run_lanes(const DevParams *__restrict__ sims, uint32_t n_sims, const uint64_t *off,
                           uint64_t *stat, St *stage, const BmTables &bm, const DevOut &O) {
@@ -164,8 +244,7 @@ __device__ void run_lanes(const DevParams *__restrict__ sims, uint32_t n_sims, c
     const int lane = (int)(threadIdx.x & (kWave - 1));
     const uint64_t lane_lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     const DevParams &P0 = sims[0];
-    const bool resume = !kBatch && O.resume != nullptr;
-    const uint64_t N = kBatch ? off[n_sims] : (resume ? O.resume_n : P0.n_particles);
+    const uint64_t N = kBatch ? off[n_sims] : P0.n_particles;
     const uint64_t grab = O.chunk ? (uint64_t)O.chunk : kChunk;   // ids per queue grab (wave-uniform)
 
     // Per-simulation values (wave-uniform for plain runs, per lane in batches).
@@ -187,18 +266,18 @@ __device__ void run_lanes(const DevParams *__restrict__ sims, uint32_t n_sims, c
     Model m;
     uint64_t pid = 0;
     uint32_t steps = 0, blk = 0;
-    bool active = false, has_particle = false;
+    bool active = false;
     uint64_t q_next = 0, q_end = 0;
     bool exhausted = false;
-    uint64_t my_steps = 0;
-    uint32_t my_particles = 0, my_nan = 0, my_cap = 0, cycles = 0, my_max = 0;
+    LaneStats st{0, 0, 0, 0, 0};
+    uint32_t cycles = 0, drained = 0;
 
     auto emit = [&](double t_inj, double t_exit, double r, double theta, double sumac) {
         stage_event(stage, O, pid, sim, t_inj, t_exit, r, theta, sumac);
     };
-    auto do_step = [&](const double *z) -> bool {
-        if constexpr (kVecParams) return m.step(lp, z, bm.trig, emit);
-        else return m.step(P0, z, bm.trig, emit);
+    auto params = [&]() -> const StepParams & {
+        if constexpr (kVecParams) return lp;
+        else return P0;
     };
 
     for (;;) {
@@ -213,7 +292,7 @@ __device__ void run_lanes(const DevParams *__restrict__ sims, uint32_t n_sims, c
             if (avail < (uint64_t)n_idle) {
                 unsigned long long base = 0;
                 if (lane == 0) base = atomicAdd(queue, (unsigned long long)grab);
-                base = __shfl(base, 0);
+                base = from_lane0(base);
                 if (base >= N) {
                     exhausted = true;
                     q_next = q_end = N;
@@ -231,22 +310,13 @@ __device__ void run_lanes(const DevParams *__restrict__ sims, uint32_t n_sims, c
                 q_next += (uint64_t)n_idle;
             }
             if (take != ~0ull) {
-                // the lane's previous particle ended: its steps, and whether
-                // it stopped on a NaN state
-                if (has_particle) {
-                    my_steps += steps;
-                    my_max = steps > my_max ? steps : my_max;
-                    if (isnan(m.r)) ++my_nan;
-                }
-                has_particle = true;
                 steps = 0;
                 blk = 0;
                 double T;
                 if constexpr (kBatch) {
                     if (take >= sim_hi) {
-                        if (my_particles) flush_sim_stats(O, sim, my_steps, my_particles, my_nan, my_cap);
-                        my_steps = 0;
-                        my_particles = my_nan = my_cap = 0;
+                        if (st.particles) flush_sim_stats(O, sim, st.steps, st.particles, st.nan, st.cap);
+                        st = LaneStats{0, 0, 0, 0, 0};
                         // largest s in [sim, n_sims) with off[s] <= take; off[s+1] > take follows
                         uint32_t lo = sim, hi = n_sims;
                         while (hi - lo > 1) {
@@ -266,57 +336,49 @@ __device__ void run_lanes(const DevParams *__restrict__ sims, uint32_t n_sims, c
                     pid = first + (O.order ? (uint64_t)O.order[take] : take - sim_lo);
                     const DevParams &Q = sims[sim];
                     T = injection_energy(Q, pid);
-                    ++my_particles;
                     active = m.init(lp, T);
-                } else if (resume) {
-                    // a particle handed on by the previous launch
-                    const SpillRec &rec = O.resume[take];
-                    m.load(rec.s);
-                    pid = rec.pid;
-                    steps = rec.steps;
-                    blk = rec.blk;
-                    active = true;
                 } else {
                     pid = first + (O.order ? (uint64_t)O.order[take] : take);
                     T = injection_energy(P0, pid);
-                    ++my_particles;
                     active = m.init(P0, T);
                 }
+                ++st.particles;
             }
         }
-        if constexpr (!kBatch) {
-            // tail compaction: a sparse wave hands its live particles on and exits
-            if (O.spill && exhausted && cycles >= kSpillMinCycles) {
+        if (O.spill) {
+            // A wave whose lanes are all busy learns from the queue itself that
+            // the ids have run out.
+            if (!exhausted && q_next == q_end && cycles % kQueuePoll == kQueuePoll - 1) {
+                const uint64_t head = __hip_atomic_load(queue, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                exhausted = from_lane0(head) >= N;
+            }
+            if (exhausted && ++drained > kDrainCycles) {
                 const uint64_t live = __ballot(active);
-                const int n_live = __popcll(live);
-                if (n_live > 0 && n_live <= kSpillLanes) {
-                    unsigned long long base = 0;
-                    if (lane == 0) base = atomicAdd((unsigned long long *)O.spill_count, (unsigned long long)n_live);
-                    base = __shfl(base, 0);
-                    const uint64_t slot = base + (uint64_t)__popcll(live & lane_lt);
-                    if (active && slot < O.spill_cap) {
-                        SpillRec &rec = O.spill[slot];
-                        m.save(rec.s);
-                        rec.pid = pid;
-                        rec.steps = steps;
-                        rec.blk = blk;
-                        active = false;
-                        has_particle = false;   // its steps are counted where it ends
-                    }
+                unsigned long long base = 0;
+                if (lane == 0 && live)
+                    base = atomicAdd((unsigned long long *)O.spill_count, (unsigned long long)__popcll(live));
+                base = from_lane0(base);
+                const uint64_t slot = base + (uint64_t)__popcll(live & lane_lt);
+                if (active && slot < O.spill_cap) {   // (always: one slot per lane)
+                    SpillRec &rec = O.spill[slot];
+                    m.save(rec.s);
+                    rec.pid = pid;
+                    rec.steps = steps;   // counted where the particle ends
+                    rec.sim = sim;
                 }
+                break;
             }
         }
-        stage_flush<kBatch>(stage, O, kStageFlush);
         if (__ballot(active) == 0) {
             if (exhausted) break;
             continue;
         }
         ++cycles;
         // ---- one cycle: kCycleSteps steps, NPS Philox blocks
+        const Model old = m;
+        typename Model::Watch watch = m.watch();
+        double z1[4] = {0.0, 0.0, 0.0, 0.0};   // 1D: the cycle's four normals, one block
         if constexpr (NPS == 1) {
-            // 1D: the four normals of the cycle come from one block; every
-            // normal's position is known at compile time.
-            double z[4];
             if constexpr (!kBatch && !Model::kLatencyBound) {
                 // wave-uniform Philox key: an empty asm (it emits nothing)
                 // makes the round keys be formed with scalar adds in every
@@ -325,30 +387,9 @@ __device__ void run_lanes(const DevParams *__restrict__ sims, uint32_t n_sims, c
                 // instruction).  A latency-bound model keeps them.
                 asm volatile("" : "+s"(k0), "+s"(k1));
             }
-            normal_block(pid, blk, k0, k1, bm, z);
-            if (__ballot(active && steps + kCycleSteps > cap) == 0) {
-                // no lane can reach its step cap in this cycle
+            normal_block(pid, blk, k0, k1, bm, z1);
 #pragma unroll
-                for (int s = 0; s < kCycleSteps; ++s) {
-                    if (active) {
-                        ++steps;
-                        if (!do_step(&z[s])) active = false;
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int s = 0; s < kCycleSteps; ++s) {
-                    if (active) {
-                        if (steps >= cap) {
-                            ++my_cap;
-                            active = false;
-                        } else {
-                            ++steps;
-                            if (!do_step(&z[s])) active = false;
-                        }
-                    }
-                }
-            }
+            for (int s = 0; s < kCycleSteps; ++s) m.fast_step(params(), &z1[s], bm.trig, watch);
         } else if constexpr (NPS == 2) {
             // 2D SolarProp: one block serves two steps (normals 4k .. 4k+3 of
             // the cycle); the loop over step pairs stays rolled.
@@ -358,17 +399,7 @@ __device__ void run_lanes(const DevParams *__restrict__ sims, uint32_t n_sims, c
                 if constexpr (!kBatch) asm volatile("" : "+s"(k0), "+s"(k1));   // as above
                 normal_block(pid, blk + (uint32_t)(s >> 1), k0, k1, bm, t);
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    if (active) {
-                        if (steps >= cap) {
-                            ++my_cap;
-                            active = false;
-                        } else {
-                            ++steps;
-                            if (!do_step(&t[2 * h])) active = false;
-                        }
-                    }
-                }
+                for (int h = 0; h < 2; ++h) m.fast_step(params(), &t[2 * h], bm.trig, watch);
             }
         } else {
             // 2D Geliosphere: steps stay rolled (the step body is large).
@@ -398,35 +429,39 @@ __device__ void run_lanes(const DevParams *__restrict__ sims, uint32_t n_sims, c
                         c0 = t[1]; c1 = t[2]; c2 = t[3];
                     }
                 }
-                if (active) {
-                    if (steps >= cap) {
-                        ++my_cap;
-                        active = false;
-                    } else {
-                        ++steps;
-                        if (!do_step(z)) active = false;
-                    }
-                }
+                m.fast_step(params(), z, bm.trig, watch);
             }
         }
+        const bool again = active && !(m.fast_ok(watch, old) && cap - steps >= (uint32_t)kCycleSteps);
+        if (__ballot(again)) {
+            if (again) {
+                m = old;
+                double q0 = z1[0], q1 = z1[1], q2 = z1[2], q3 = z1[3];
+                active = slow_cycle(
+                    m, params(),
+                    [&](int s, double *z) {
+                        if constexpr (NPS == 1) {
+                            z[0] = q0;
+                            q0 = q1; q1 = q2; q2 = q3;
+                        } else {
+                            normals_of_step<NPS>(pid, blk, s, k0, k1, bm, z);
+                        }
+                    },
+                    bm.trig, cap, steps, st, emit);
+                steps -= (uint32_t)kCycleSteps;   // added below (a particle that ended is counted already)
+            }
+            stage_flush<kBatch>(stage, O, kStageFlush);
+        }
+        steps += (uint32_t)kCycleSteps;
         blk += (uint32_t)NPS;
-    }
-    if (has_particle) {
-        my_steps += steps;
-        my_max = steps > my_max ? steps : my_max;
-        if (isnan(m.r)) ++my_nan;
     }
     stage_flush<kBatch>(stage, O, 1);
     if constexpr (kBatch) {
-        if (my_particles) flush_sim_stats(O, sim, my_steps, my_particles, my_nan, my_cap);
+        if (st.particles) flush_sim_stats(O, sim, st.steps, st.particles, st.nan, st.cap);
         if (lane == 0) atomicAdd((unsigned long long *)O.cycles, (unsigned long long)cycles);
     } else {
-        atomicAdd((unsigned long long *)&stat[ST_STEPS], (unsigned long long)my_steps);
-        atomicAdd((unsigned long long *)&stat[ST_PARTICLES], (unsigned long long)my_particles);
-        if (my_nan) atomicAdd((unsigned long long *)&stat[ST_NAN], (unsigned long long)my_nan);
-        if (my_cap) atomicAdd((unsigned long long *)&stat[ST_CAP], (unsigned long long)my_cap);
+        flush_lane_stats(stat, st);
         if (lane == 0) atomicAdd((unsigned long long *)&stat[ST_CYCLES], (unsigned long long)cycles);
-        if (my_max) atomicMax((unsigned long long *)&stat[ST_MAX_STEPS], (unsigned long long)my_max);
     }
 }
 
@@ -478,11 +513,7 @@ plain_kernel(const DevParams *__restrict__ Pp, const DevOut O) {
     __syncthreads();
     run_lanes<Model, false>(Pp, 1, nullptr, stat, &stage, bm, O);
     __syncthreads();
-    if (threadIdx.x < ST_COUNT_ && stat[threadIdx.x]) {
-        unsigned long long *g = (unsigned long long *)&O.g_stats[threadIdx.x];
-        if (threadIdx.x == ST_MAX_STEPS) atomicMax(g, (unsigned long long)stat[threadIdx.x]);
-        else atomicAdd(g, (unsigned long long)stat[threadIdx.x]);
-    }
+    flush_block_stats(stat, O);
 }
 
 // Batch of n_sims simulations of one model (n_sims <= kBatchMaxSims).
@@ -501,6 +532,171 @@ batch_kernel(const DevParams *__restrict__ sims, uint32_t n_sims, const uint64_t
     load_bm_tables(&bm);
     __syncthreads();
     run_lanes<Model, true>(sims, n_sims, off, nullptr, &stage, bm, O);
+}
+
+// ---------------------------------------------------------------- tails
+// The last particles of a run (and runs of few particles) are bound by the
+// latency of one particle's steps, not by throughput: 1e4 B-p particles need
+// 0.3 ms of the chip's issue slots, but the longest of them takes 8e4 steps one
+// after another.  A tail launch therefore spreads its particles over one wave
+// per SIMD, G lanes to a particle (G = 1 .. 64, as many as there is room for):
+//  - the G lanes form G Philox blocks of their particle at once, into LDS, and
+//    every step then reads its normals from there: the random numbers, half of
+//    a 1D step's instructions, cost 1/G of that;
+//  - all G lanes carry the particle's state and do the same steps (the first
+//    of them emits and counts), so no lane is masked off and no step branches:
+//    kTailCycles cycles run as fast steps, then one test.
+// G is fixed within a launch.  After `budget` cycles the live particles are
+// handed to the next launch, which spreads the fewer particles over the same
+// lanes; a launch that has 64 lanes per particle runs them to the end.
+// Statistics and results do not depend on any of this.
+template <class Model>
+struct TailShape {
+    static constexpr int kRingWords = kWave * Model::kNormals * 4;   // normals of one pass
+    // words between the particles' normals: their reads, one address per
+    // particle, go to different banks
+    __device__ static int stride(int g) { return g * Model::kNormals * 4 + 2; }
+    static constexpr int kPad = 2 * kWave;
+};
+
+template <class Model, bool kBatch>
+__global__ void __launch_bounds__(kTailThreads) tail_kernel(const DevParams *__restrict__ sims, uint32_t n_sims,
+                                                           const uint64_t *__restrict__ offsets, const DevOut O,
+                                                           const TailArgs A) {
+    constexpr int NPS = Model::kNormals, kWaves = kTailThreads / kWave;
+    using Shape = TailShape<Model>;
+    __shared__ uint64_t stat[ST_COUNT_];
+    __shared__ Stage<kWaves> stage;
+    __shared__ BmTables bm;
+    __shared__ alignas(16) double ring[kWaves][Shape::kRingWords + Shape::kPad];
+    const uint64_t n = A.in ? (*A.n_in < A.cap ? *A.n_in : A.cap) : A.fresh_n;
+    int g = 1;
+    while (g < kWave && n * (uint64_t)(2 * g) <= A.lanes) g *= 2;
+    const int wave = (int)(threadIdx.x / kWave), lane = (int)(threadIdx.x & (kWave - 1));
+    const uint64_t per_wave = (uint64_t)(kWave / g);
+    if ((uint64_t)blockIdx.x * kWaves * per_wave >= n) return;   // the whole workgroup
+    if (threadIdx.x < ST_COUNT_) stat[threadIdx.x] = 0;
+    if (threadIdx.x < kWaves) stage.count[threadIdx.x] = 0;
+    load_bm_tables(&bm);
+    __syncthreads();
+    const int sub = lane & (g - 1), group = lane / g;
+    const uint64_t idx = ((uint64_t)blockIdx.x * kWaves + wave) * per_wave + group;
+    double *rg = ring[wave];
+    const double *my = rg + group * Shape::stride(g);
+
+    const bool mine = idx < n;
+    bool active = mine;
+    const bool lead = mine && sub == 0;
+    uint64_t pid = 0;
+    uint32_t steps = 0, sim = 0;
+    Model m;
+    LaneStats st{0, 0, 0, 0, 0};
+    if (A.in) {
+        const SpillRec &rec = A.in[mine ? idx : 0];
+        m.load(rec.s);
+        pid = rec.pid;
+        steps = rec.steps;
+        if (kBatch) sim = rec.sim;
+    } else {
+        const uint64_t v = mine ? idx : 0;
+        if (kBatch) {
+            uint32_t lo = 0, hi = n_sims;   // largest s with offsets[s] <= v
+            while (hi - lo > 1) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (offsets[mid] <= v) lo = mid; else hi = mid;
+            }
+            sim = lo;
+        }
+        const DevParams &Q = sims[sim];
+        pid = Q.first_particle + (O.order ? (uint64_t)O.order[v] : v - (kBatch ? offsets[sim] : 0));
+    }
+    const DevParams &Q = sims[sim];
+    StepParams lp = static_cast<const StepParams &>(Q);
+    const uint32_t k0 = (uint32_t)Q.seed, k1 = (uint32_t)(Q.seed >> 32), cap = (uint32_t)Q.max_steps;
+    if (!A.in) {
+        const bool started = m.init(lp, injection_energy(Q, pid));
+        active = active && started;
+        if (lead) st.particles = 1;
+    }
+    auto emit = [&](double t_inj, double t_exit, double r, double theta, double sumac) {
+        if (lead) stage_event(&stage, O, pid, sim, t_inj, t_exit, r, theta, sumac);
+    };
+    const uint32_t budget = A.out && g < kWave ? A.budget : 0xffffffffu;
+    uint32_t cycles = 0;
+    uint32_t blk = steps / kCycleSteps * NPS;
+    while (__ballot(active) && cycles < budget) {
+        // ---- normals of the next g cycles: NPS blocks per lane
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+        for (int i = 0; i < NPS; ++i) {
+            double z[4];
+            const int b = i * g + sub;
+            normal_block(pid, blk + (uint32_t)b, k0, k1, bm, z);
+            double *d = rg + group * Shape::stride(g) + 4 * b;
+            d[0] = z[0]; d[1] = z[1]; d[2] = z[2]; d[3] = z[3];
+        }
+        __builtin_amdgcn_wave_barrier();
+        blk += (uint32_t)(NPS * g);
+        // ---- g cycles, kTailCycles at a time where g allows
+#pragma unroll 1
+        for (int c = 0; c < g; ++c) {
+            const double *zc = my + c * NPS * kCycleSteps;
+            const Model old = m;
+            typename Model::Watch watch = m.watch();
+#pragma unroll
+            for (int s = 0; s < kCycleSteps; ++s) {
+                double z[NPS];
+                for (int i = 0; i < NPS; ++i) z[i] = zc[NPS * s + i];
+                m.fast_step(lp, z, bm.trig, watch);
+            }
+            const bool again = active && !(m.fast_ok(watch, old) && cap - steps >= (uint32_t)kCycleSteps);
+            ++cycles;
+            if (__ballot(again)) {
+                if (again) {
+                    m = old;
+                    LaneStats one{0, 0, 0, 0, 0};
+                    active = slow_cycle(
+                        m, lp, [&](int s, double *z) { for (int i = 0; i < NPS; ++i) z[i] = zc[NPS * s + i]; }, bm.trig,
+                        cap, steps, one, emit);
+                    steps -= (uint32_t)kCycleSteps;
+                    if (lead) {
+                        st.steps += one.steps;
+                        st.nan += one.nan;
+                        st.cap += one.cap;
+                        st.max_steps = one.max_steps > st.max_steps ? one.max_steps : st.max_steps;
+                    }
+                }
+                stage_flush<kBatch>(&stage, O, kStageFlush);
+                if (__ballot(active) == 0) break;
+            }
+            steps += (uint32_t)kCycleSteps;
+        }
+    }
+    const uint64_t live = __ballot(active && sub == 0);
+    if (live) {   // the budget is spent: hand the live particles on
+        const uint64_t lane_lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+        unsigned long long base = 0;
+        if (lane == 0) base = atomicAdd((unsigned long long *)A.n_out, (unsigned long long)__popcll(live));
+        base = from_lane0(base);
+        const uint64_t slot = base + (uint64_t)__popcll(live & lane_lt);
+        if (active && sub == 0 && slot < A.cap) {   // (always: at most the particles taken from `in`)
+            SpillRec &rec = A.out[slot];
+            m.save(rec.s);
+            rec.pid = pid;
+            rec.steps = steps;
+            rec.sim = sim;
+        }
+    }
+    stage_flush<kBatch>(&stage, O, 1);
+    if constexpr (kBatch) {
+        if (lead) flush_sim_stats(O, sim, st.steps, st.particles, st.nan, st.cap);
+        if (lane == 0) atomicAdd((unsigned long long *)O.cycles, (unsigned long long)cycles);
+    } else {
+        flush_lane_stats(stat, st);
+        if (lane == 0) atomicAdd((unsigned long long *)&stat[ST_CYCLES], (unsigned long long)cycles);
+        __syncthreads();
+        flush_block_stats(stat, O);
+    }
 }
 
 // Histogram pass: workgroup (x, s) folds a strided share of simulation s's
@@ -871,6 +1067,32 @@ hipError_t gs_launch_traj(int model, bool batch, const DevParams *sims, uint32_t
     default: ok = false; break;
     }
     if (!ok) return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+template <class Model>
+static void launch_tail_t(bool batch, const DevParams *sims, uint32_t n_sims, const uint64_t *offsets,
+                          const DevOut &O, const TailArgs &A, unsigned grid, hipStream_t s) {
+    if (batch)
+        hipLaunchKernelGGL((tail_kernel<Model, true>), dim3(grid), dim3(kTailThreads), 0, s, sims, n_sims, offsets, O, A);
+    else
+        hipLaunchKernelGGL((tail_kernel<Model, false>), dim3(grid), dim3(kTailThreads), 0, s, sims, n_sims, offsets, O, A);
+}
+
+hipError_t gs_launch_tail(int model, bool batch, const DevParams *sims, uint32_t n_sims, const uint64_t *offsets,
+                          const DevOut &O, const TailArgs &A, unsigned grid, hipStream_t s) {
+    if (n_sims == 0 || grid == 0) return hipSuccess;
+    const uint64_t lanes = (uint64_t)grid * kTailThreads;
+    if ((!batch && n_sims != 1) || (batch && (n_sims > (uint32_t)kBatchMaxSims || !offsets)) ||
+        (A.in ? !A.n_in || A.cap > lanes : A.fresh_n > lanes) || (A.out && A.cap < (A.in ? A.cap : A.fresh_n)) || (A.out && !A.n_out) || A.budget == 0)
+        return hipErrorInvalidValue;
+    switch (model) {
+    case GS_MODEL_1D_FP: launch_tail_t<Fp>(batch, sims, n_sims, offsets, O, A, grid, s); break;
+    case GS_MODEL_1D_BP: launch_tail_t<Bp>(batch, sims, n_sims, offsets, O, A, grid, s); break;
+    case GS_MODEL_2D_SOLARPROP: launch_tail_t<Sp>(batch, sims, n_sims, offsets, O, A, grid, s); break;
+    case GS_MODEL_2D_GELIOSPHERE: launch_tail_t<Ge>(batch, sims, n_sims, offsets, O, A, grid, s); break;
+    default: return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }
 
