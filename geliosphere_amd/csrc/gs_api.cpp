@@ -52,7 +52,7 @@ struct gs_ctx {
     // batched runs: side streams for concurrent model groups, fork/join
     // events, and the graph of the last batch layout
     hipStream_t side[3] = {nullptr, nullptr, nullptr};
-    hipEvent_t fork = nullptr, join[3] = {nullptr, nullptr, nullptr};
+    hipEvent_t fork = nullptr, join[3] = {nullptr, nullptr, nullptr}, traj[4] = {nullptr, nullptr, nullptr, nullptr};
     std::vector<uint64_t> graph_key;
     hipGraphExec_t graph_exec = nullptr;
     uint64_t batch_event_budget = 1ull << 29;
@@ -379,8 +379,8 @@ const uint64_t kOrderMinParticles = 4096;   // smaller runs keep id order
 // about every time their number has halved.  Every launch is queued beforehand
 // and takes its particle count from the one before on the device; one that
 // finds none ends at once (about 3 us).
-constexpr int kTailRounds = 11;
-constexpr uint32_t kTailBudget = 128;
+constexpr int kTailRounds = 21;
+constexpr uint32_t tail_budget(int r) { return (r & 1 ? 181u : 128u) << (r >> 1); }
 
 uint64_t tail_lanes(const gs_ctx *ctx) { return (uint64_t)ctx->n_cu * 4 * gs::kWave; }
 
@@ -394,14 +394,20 @@ uint64_t tail_cap(const gs_ctx *ctx, uint64_t n, uint64_t traj_lanes) {
 // particles themselves (no throughput launch ran); otherwise those that the
 // throughput launch handed on to `half0` (counted in counts[0]).  counts: one
 // word per launch, zeroed.
-hipError_t queue_tail(const gs_ctx *ctx, int model, bool batch, const DevParams *sims, uint32_t n_sims,
+// all_lanes: one wave per SIMD of the device.  part of parts: the share of the
+// device that a batch's model group takes once its particles fit there.
+hipError_t queue_tail(uint64_t all_lanes, int part, int parts, int model, bool batch, const DevParams *sims, uint32_t n_sims,
                       const uint64_t *offsets, const DevOut &O, uint64_t fresh_n, gs::SpillRec *half0,
                       gs::SpillRec *half1, uint64_t cap, uint64_t *counts, hipStream_t s) {
-    const uint64_t lanes = tail_lanes(ctx);
     const uint64_t most = fresh_n ? fresh_n : cap;
-    // workgroups for up to 64 lanes per particle on `lanes`, or one lane each
-    const uint64_t threads = std::min<uint64_t>(most * gs::kWave, std::max(most, lanes));
-    const unsigned grid = (unsigned)((threads + gs::kTailThreads - 1) / gs::kTailThreads);
+    const uint32_t xcds = gs::kXcds / (uint32_t)parts;
+    const uint64_t lanes = all_lanes * xcds / gs::kXcds;
+    // workgroups for up to 64 lanes per particle on the share's lanes (kXcds /
+    // xcds workgroups for each one used), or one lane each on all
+    const uint64_t spread = std::min<uint64_t>(most * gs::kWave, lanes);
+    const uint64_t groups = (spread + gs::kTailThreads - 1) / gs::kTailThreads;
+    const uint64_t dense = (most + gs::kTailThreads - 1) / gs::kTailThreads;
+    const unsigned grid = (unsigned)std::max<uint64_t>(dense, (groups + xcds - 1) / xcds * gs::kXcds);
     const int rounds = most * gs::kWave <= lanes ? 1 : kTailRounds;   // 64 lanes each at once: no budget
     for (int r = 0; r < rounds; ++r) {
         gs::TailArgs A;
@@ -411,8 +417,10 @@ hipError_t queue_tail(const gs_ctx *ctx, int model, bool batch, const DevParams 
         A.out = r + 1 < rounds ? ((r & 1) ? half0 : half1) : nullptr;
         A.n_out = counts + r + 1;
         A.cap = cap;
-        A.budget = kTailBudget << r;
+        A.budget = tail_budget(r);
         A.lanes = (uint32_t)lanes;
+        A.xcd_lo = (uint32_t)part * xcds;
+        A.xcd_n = xcds;
         const hipError_t e = gs_launch_tail(model, batch, sims, n_sims, offsets, O, A, grid, s);
         if (e != hipSuccess) return e;
     }
@@ -438,7 +446,7 @@ bool record_less(const gs_exit_record &a, const gs_exit_record &b) {
 // affects the order of work, never the results).  Diffusive time across
 // the heliosphere ~ L^2 / (K0 dt), times the per-step cost of the model.
 double est_cost(const gs_params &p) {
-    static const double step_cost[4] = {1.0, 1.0, 4.0, 6.5};
+    static const double step_cost[4] = {0.004, 1.0, 4.0, 6.5};
     const double L = std::max(100.0 - std::min(p.r_inj, 100.0), 1.0);
     const double K = std::max(p.K0, 1e-12);
     return step_cost[p.model] * L * L / (K * p.dt);
@@ -488,7 +496,7 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
     for (uint32_t i : order) gcost[sims[i].model] += est_cost(sims[i]) * (double)sims[i].n_particles;
     std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) {
         const int ma = sims[a].model, mb = sims[b].model;
-        if (ma != mb) return gcost[ma] != gcost[mb] ? gcost[ma] > gcost[mb] : ma < mb;
+        if (ma != mb) return gcost[ma] != gcost[mb] ? gcost[ma] < gcost[mb] : ma < mb;
         return est_cost(sims[a]) > est_cost(sims[b]);
     });
     // ---- launches: (model, first sim, count)
@@ -600,6 +608,13 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
         hipError_t e = gs_launch_zero(ctx->d_words, m * words_per_sim(), s0);
         if (e == hipSuccess) e = gs_launch_zero(ctx->d_meta + 2 * m, m, s0);          // n_events
         if (e == hipSuccess) e = gs_launch_zero(ctx->d_meta + q_base, meta_words - q_base, s0);   // queues, cycles, hand-on
+        // Every group's order before any group's persistent waves: queued on the
+        // group's own stream behind another group's launch, the order kernels
+        // waited 25 ms for a free wave slot (64 simulations, 1.7e6 particles).
+        for (size_t l = 0; l < nl && ordered && e == hipSuccess; ++l)
+            e = gs_launch_batch_order(ctx->d_params + launches[l].base, launches[l].count, ctx->d_meta + launches[l].off_pos,
+                                      nv[l], ctx->d_bcounts + 2 * (size_t)gs::kOrderSimBuckets * launches[l].base,
+                                      ctx->d_border + perm_at[l], s0);
         if (e == hipSuccess) e = hipEventRecord(ctx->fork, s0);
         // model groups on up to four streams
         std::vector<int> group_of(nl);
@@ -608,6 +623,8 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
             if (l == 0 || launches[l].model != launches[l - 1].model) ++n_groups;
             group_of[l] = n_groups - 1;
         }
+        const int parts = n_groups >= 3 ? 4 : n_groups;   // of the device, for tails side by side
+        int after = 0;   // 1 + the stream of the throughput launch before
         bool used[3] = {false, false, false};
         for (size_t l = 0; l < nl && e == hipSuccess; ++l) {
             const int g = group_of[l] % 4;
@@ -626,13 +643,7 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
             uint64_t *counts = ctx->d_meta + t_base + l * (kTailRounds + 1);
             O.spill = half0; O.spill_count = counts; O.spill_cap = spill_cap[l];
             O.chunk = L.chunk;
-            if (ordered) {
-                e = gs_launch_batch_order(ctx->d_params + L.base, L.count, ctx->d_meta + L.off_pos, nv[l],
-                                          ctx->d_bcounts + 2 * (size_t)gs::kOrderSimBuckets * L.base,
-                                          ctx->d_border + perm_at[l], sg);
-                if (e != hipSuccess) break;
-                O.order = ctx->d_border + perm_at[l];
-            }
+            if (ordered) O.order = ctx->d_border + perm_at[l];
             O.g_count = W.count + (size_t)L.base * GS_MAX_BINS;
             O.g_digits = W.digits + (size_t)L.base * gs::kDigitsPerSim;
             O.g_stats = W.stats + (size_t)L.base * gs::ST_COUNT_;
@@ -641,11 +652,19 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
             O.ev_cap = ctx->d_meta + m + L.base;
             O.n_events = ctx->d_meta + 2 * m + L.base;
             const bool fresh = nv[l] > 0 && nv[l] <= tail_lanes(ctx);
-            if (!fresh)
-                e = gs_launch_traj(L.model, true, ctx->d_params + L.base, L.count, ctx->d_meta + L.off_pos, O,
-                                   L.grid, L.block, sg);
+            if (!fresh) {
+                // One throughput launch after another (each fills the device; the
+                // tail of one overlaps the next): with all at once the group with
+                // the longest tail got its share of the slots last.
+                if (after) e = hipStreamWaitEvent(sg, ctx->traj[after - 1], 0);
+                if (e == hipSuccess)
+                    e = gs_launch_traj(L.model, true, ctx->d_params + L.base, L.count, ctx->d_meta + L.off_pos, O,
+                                       L.grid, L.block, sg);
+                if (e == hipSuccess) e = hipEventRecord(ctx->traj[g], sg);
+                after = g + 1;
+            }
             if (e == hipSuccess && nv[l] > 0)
-                e = queue_tail(ctx, L.model, true, ctx->d_params + L.base, L.count, ctx->d_meta + L.off_pos, O,
+                e = queue_tail(tail_lanes(ctx), g, parts, L.model, true, ctx->d_params + L.base, L.count, ctx->d_meta + L.off_pos, O,
                                fresh ? nv[l] : 0, half0, half1, spill_cap[l], counts, sg);
         }
         for (int g = 0; g < 3 && e == hipSuccess; ++g) {
@@ -724,7 +743,7 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
 // order permutation, hand-on records).  own = false: fixed buffers (events,
 // order_counts and order of cap_events entries); no exit records, no
 // hand-on, and chunks are cut to fit the fixed event region.
-constexpr int kMetaSaved = 32;
+constexpr int kMetaSaved = 40;
 static_assert(4 + kTailRounds + 1 <= kMetaSaved && kMetaSaved + gs::ST_COUNT_ <= 64, "plain run's meta words");
 struct PlainBufs {
     uint64_t *words;
@@ -823,7 +842,7 @@ gs_status run_plain_core(gs_ctx *ctx, const gs_params &pp, gs_spectrum *out, gs_
         HIP_TRY(ctx, hipEventRecord(ctx->ev0, ctx->stream));
         if (!fresh) HIP_TRY(ctx, gs_launch_traj(q.model, false, B.params, 1, nullptr, O, grid, RS.block, ctx->stream));
         if (B.own && q.n_particles > 0)
-            HIP_TRY(ctx, queue_tail(ctx, q.model, false, B.params, 1, nullptr, O, fresh ? q.n_particles : 0, ctx->d_spill,
+            HIP_TRY(ctx, queue_tail(tail_lanes(ctx), 0, 1, q.model, false, B.params, 1, nullptr, O, fresh ? q.n_particles : 0, ctx->d_spill,
                                     ctx->d_spill + ctx->cap_spill, cap_tail, B.meta + 4, ctx->stream));
         HIP_TRY(ctx, hipEventRecord(ctx->ev1, ctx->stream));
         uint64_t nev = 0;
@@ -918,6 +937,7 @@ gs_status gs_create(gs_ctx **out, int device) {
         if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->join[i], hipEventDisableTiming);
     }
     if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->fork, hipEventDisableTiming);
+    for (int i = 0; i < 4 && e == hipSuccess; ++i) e = hipEventCreateWithFlags(&ctx->traj[i], hipEventDisableTiming);
     // the device's scratch array, with the device current (looked up once per device)
     if (e == hipSuccess) e = gs_scratch_address(device, &ctx->scratch, &ctx->scratch_bytes);
     if (e != hipSuccess) {
@@ -950,6 +970,8 @@ void gs_destroy(gs_ctx *ctx) {
         if (ctx->join[i]) (void)hipEventDestroy(ctx->join[i]);
     }
     if (ctx->fork) (void)hipEventDestroy(ctx->fork);
+    for (hipEvent_t ev : ctx->traj)
+        if (ev) (void)hipEventDestroy(ev);
     if (ctx->d_params) (void)hipFree(ctx->d_params);
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
     if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);

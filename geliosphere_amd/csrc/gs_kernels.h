@@ -161,8 +161,14 @@ struct TailArgs {
     uint64_t *n_out;
     uint64_t cap;            // records in `in` and `out`
     uint32_t budget;
-    uint32_t lanes;          // lanes to spread the particles over (one wave per SIMD)
+    // Lanes to spread the particles over (one wave per SIMD), on the dies
+    // xcd_lo .. xcd_lo + xcd_n - 1: workgroup i runs on die i mod 8, so groups of
+    // a batch with dies of their own do not meet on the same SIMDs while the
+    // others idle.  More particles than lanes go to all dies.
+    uint32_t lanes;
+    uint32_t xcd_lo, xcd_n;
 };
+constexpr uint32_t kXcds = 8;
 constexpr int kTailThreads = 256;
 
 // LDS layout per workgroup: count[n_bins] | digits[n_weights][2][n_bins][16] | stat[ST_COUNT_]

@@ -545,10 +545,10 @@ batch_kernel(const DevParams *__restrict__ sims, uint32_t n_sims, const uint64_t
 //    a 1D step's instructions, cost 1/G of that;
 //  - all G lanes carry the particle's state and do the same steps (the first
 //    of them emits and counts), so no lane is masked off and no step branches:
-//    kTailCycles cycles run as fast steps, then one test.
+//    every cycle runs as fast steps, then one test.
 // G is fixed within a launch.  After `budget` cycles the live particles are
 // handed to the next launch, which spreads the fewer particles over the same
-// lanes; a launch that has 64 lanes per particle runs them to the end.
+// lanes (in a batch: its model group's share of the dies); a launch that has 64 lanes per particle runs them to the end.
 // Statistics and results do not depend on any of this.
 template <class Model>
 struct TailShape {
@@ -574,13 +574,22 @@ __global__ void __launch_bounds__(kTailThreads) tail_kernel(const DevParams *__r
     while (g < kWave && n * (uint64_t)(2 * g) <= A.lanes) g *= 2;
     const int wave = (int)(threadIdx.x / kWave), lane = (int)(threadIdx.x & (kWave - 1));
     const uint64_t per_wave = (uint64_t)(kWave / g);
-    if ((uint64_t)blockIdx.x * kWaves * per_wave >= n) return;   // the whole workgroup
+    uint64_t block = blockIdx.x;
+    if (n <= A.lanes && A.xcd_n < kXcds) {
+        const uint32_t x = blockIdx.x % kXcds - A.xcd_lo;   // (below xcd_lo: wraps to a large number)
+        if (x >= A.xcd_n) return;
+        block = (uint64_t)(blockIdx.x / kXcds) * A.xcd_n + x;
+    }
+    if (block * kWaves * per_wave >= n) return;   // the whole workgroup
     if (threadIdx.x < ST_COUNT_) stat[threadIdx.x] = 0;
     if (threadIdx.x < kWaves) stage.count[threadIdx.x] = 0;
     load_bm_tables(&bm);
     __syncthreads();
+    // A tail runs beside other launches' throughput waves in a batch: its
+    // waves, on the critical path and at most one per SIMD, issue first.
+    __builtin_amdgcn_s_setprio(3);
     const int sub = lane & (g - 1), group = lane / g;
-    const uint64_t idx = ((uint64_t)blockIdx.x * kWaves + wave) * per_wave + group;
+    const uint64_t idx = (block * kWaves + wave) * per_wave + group;
     double *rg = ring[wave];
     const double *my = rg + group * Shape::stride(g);
 
@@ -637,7 +646,7 @@ __global__ void __launch_bounds__(kTailThreads) tail_kernel(const DevParams *__r
         }
         __builtin_amdgcn_wave_barrier();
         blk += (uint32_t)(NPS * g);
-        // ---- g cycles, kTailCycles at a time where g allows
+        // ---- g cycles
 #pragma unroll 1
         for (int c = 0; c < g; ++c) {
             const double *zc = my + c * NPS * kCycleSteps;
@@ -1084,7 +1093,7 @@ hipError_t gs_launch_tail(int model, bool batch, const DevParams *sims, uint32_t
     if (n_sims == 0 || grid == 0) return hipSuccess;
     const uint64_t lanes = (uint64_t)grid * kTailThreads;
     if ((!batch && n_sims != 1) || (batch && (n_sims > (uint32_t)kBatchMaxSims || !offsets)) ||
-        (A.in ? !A.n_in || A.cap > lanes : A.fresh_n > lanes) || (A.out && A.cap < (A.in ? A.cap : A.fresh_n)) || (A.out && !A.n_out) || A.budget == 0)
+        A.xcd_n == 0 || A.xcd_lo + A.xcd_n > kXcds || (A.in ? !A.n_in || A.cap > lanes : A.fresh_n > lanes) || (A.out && A.cap < (A.in ? A.cap : A.fresh_n)) || (A.out && !A.n_out) || A.budget == 0)
         return hipErrorInvalidValue;
     switch (model) {
     case GS_MODEL_1D_FP: launch_tail_t<Fp>(batch, sims, n_sims, offsets, O, A, grid, s); break;
