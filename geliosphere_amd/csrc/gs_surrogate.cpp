@@ -35,7 +35,8 @@ struct gs_surrogate {
     std::vector<size_t> woff, boff;    // per-member offsets (floats)
     size_t Pm = 0;                     // floats per member
     float *P = nullptr, *G = nullptr, *Mo = nullptr, *Ve = nullptr;
-    __bf16 *Pb = nullptr;
+    __bf16 *Pb = nullptr;              // row-major; fragment order for the fused kernels' shapes
+    __bf16 *PbT = nullptr;             // those shapes: every weight transposed, fragment order
     uint64_t step = 0;
     bool normalized = false;
     float mu[GS_SG_MAX_INPUTS], sd[GS_SG_MAX_INPUTS], lo[GS_SG_MAX_INPUTS], hi[GS_SG_MAX_INPUTS];
@@ -80,6 +81,7 @@ enum Buf {
     B_WSUM, B_LOSS,
     B_MEAN, B_SD,
     B_FLAGS,      // predict: fallback flags uint8 [n]
+    B_DZF, B_DZT, // fused training: hidden gradients [L-1][E][H][B], fp32 and bf16
     B_COUNT_
 };
 
@@ -144,6 +146,34 @@ gs_status forward(gs_surrogate *s, const __bf16 *X, size_t xstride, int rows, fl
 // otherwise the layer-by-layer GEMMs through the activation buffer.
 bool fused_shape(const gs_surrogate *s) {
     return s->cfg.hidden == 256 && s->L >= 2 && s->L <= kMlpMaxLayers && s->dims[0] == 32 && s->dims[s->L] == 32;
+}
+
+// The parameters as the fused kernels take them.
+TrainArgs param_args(const gs_surrogate *s) {
+    TrainArgs g{};
+    g.L = s->L;
+    g.P = s->P; g.Mo = s->Mo; g.Ve = s->Ve; g.G = s->G;
+    g.Pb = s->Pb; g.PbT = s->PbT;
+    g.Pm = s->Pm;
+    for (int l = 0; l < s->L; ++l) {
+        g.woff[l] = s->woff[l];
+        g.boff[l] = s->boff[l];
+    }
+    return g;
+}
+
+// The buffers and parameters of the fused training step for `rows` rows.
+gs_status train_args(gs_surrogate *s, int rows, TrainArgs &g) {
+    const size_t E = (size_t)s->E, B = (size_t)rows, hidden = (size_t)(s->L - 1) * E * 256;
+    g = param_args(s);
+    g.rows = rows;
+    SG_NEED(s, B_BX, E * kPad * B, g.XT);
+    SG_NEED(s, B_ACT, hidden * B, g.ActT);
+    SG_NEED(s, B_DZT, hidden * B, g.dZT);
+    SG_NEED(s, B_DZF, hidden * B, g.dZf);
+    SG_NEED(s, B_DYB, E * kPad * B, g.dYT);
+    SG_NEED(s, B_DYF, E * kPad * B, g.dYf);
+    return GS_OK;
 }
 
 gs_status forward_infer(gs_surrogate *s, const __bf16 *X, int rows, float *Out) {
@@ -324,6 +354,7 @@ gs_status gs_surrogate_create(int device, const gs_surrogate_config *cfg, gs_sur
     if (e == hipSuccess) e = hipMalloc((void **)&s->Mo, np * sizeof(float));
     if (e == hipSuccess) e = hipMalloc((void **)&s->Ve, np * sizeof(float));
     if (e == hipSuccess) e = hipMalloc((void **)&s->Pb, np * sizeof(__bf16));
+    if (e == hipSuccess && fused_shape(s)) e = hipMalloc((void **)&s->PbT, np * sizeof(__bf16));
     if (e != hipSuccess) {
         gs_surrogate_destroy(s);
         return e == hipErrorOutOfMemory ? GS_ERR_OUT_OF_MEMORY : GS_ERR_HIP;
@@ -358,7 +389,7 @@ void gs_surrogate_destroy(gs_surrogate *s) {
     if (s->stream) (void)hipStreamSynchronize(s->stream);
     for (DevBuf &b : s->bufs)
         if (b.p) (void)hipFree(b.p);
-    for (void *p : {(void *)s->P, (void *)s->G, (void *)s->Mo, (void *)s->Ve, (void *)s->Pb})
+    for (void *p : {(void *)s->P, (void *)s->G, (void *)s->Mo, (void *)s->Ve, (void *)s->Pb, (void *)s->PbT})
         if (p) (void)hipFree(p);
     if (s->stream) (void)hipStreamDestroy(s->stream);
     delete s;
@@ -395,7 +426,8 @@ gs_status gs_surrogate_set_params(gs_surrogate *s, const float *p, uint64_t coun
     SG_TRY(s, hipMemcpyAsync(s->P, p, count * sizeof(float), hipMemcpyHostToDevice, s->stream));
     SG_TRY(s, hipMemsetAsync(s->Mo, 0, count * sizeof(float), s->stream));
     SG_TRY(s, hipMemsetAsync(s->Ve, 0, count * sizeof(float), s->stream));
-    SG_TRY(s, sg_launch_to_bf16(s->P, s->Pb, count, s->stream));
+    if (fused_shape(s)) SG_TRY(s, sg_launch_pack(param_args(s), s->E, s->stream));
+    else SG_TRY(s, sg_launch_to_bf16(s->P, s->Pb, count, s->stream));
     SG_TRY(s, hipStreamSynchronize(s->stream));
     s->step = 0;
     return GS_OK;
@@ -468,21 +500,31 @@ gs_status gs_surrogate_train(gs_surrogate *s, const float *x, const float *y, co
     SG_TRY(s, hipMemcpyAsync(Y, yh.data(), yh.size() * sizeof(float), hipMemcpyHostToDevice, s->stream));
     SG_TRY(s, hipMemcpyAsync(W, wh.data(), wh.size() * sizeof(float), hipMemcpyHostToDevice, s->stream));
     const int E = s->E, H = (int)s->cfg.hidden;
+    const bool fused = fused_shape(s);
     uint32_t *idx;
-    __bf16 *bx, *act, *dyb;
-    float *by, *bw, *Z, *out, *dyf, *wsum, *loss;
+    __bf16 *bx = nullptr, *act = nullptr, *dyb = nullptr;
+    float *by = nullptr, *bw = nullptr, *Z = nullptr, *out = nullptr, *dyf = nullptr, *wsum, *loss;
     const int steps = (int)(n / (uint32_t)B);
-    const int parts = 8;
+    const int parts = fused ? B / 16 : 8;
+    TrainArgs ta;
     SG_NEED(s, B_IDX, (size_t)E * B * steps, idx);
-    SG_NEED(s, B_BX, (size_t)E * B * kPad, bx);
-    SG_NEED(s, B_BY, (size_t)E * B * kPad, by);
-    SG_NEED(s, B_BW, (size_t)E * B * kPad, bw);
-    SG_NEED(s, B_Z, (size_t)(s->L - 1) * E * B * H, Z);
-    SG_NEED(s, B_ACT, (size_t)(s->L - 1) * E * B * H, act);
-    SG_NEED(s, B_OUT, (size_t)E * B * kPad, out);
-    SG_NEED(s, B_DYF, (size_t)E * B * kPad, dyf);
-    SG_NEED(s, B_DYB, (size_t)E * B * kPad, dyb);
-    SG_NEED(s, B_WSUM, (size_t)E, wsum);
+    if (fused) {
+        st = train_args(s, B, ta);
+        if (st != GS_OK) return st;
+        ta.X = X;
+        ta.Y = Y;
+        ta.W = W;
+    } else {
+        SG_NEED(s, B_BX, (size_t)E * B * kPad, bx);
+        SG_NEED(s, B_BY, (size_t)E * B * kPad, by);
+        SG_NEED(s, B_BW, (size_t)E * B * kPad, bw);
+        SG_NEED(s, B_Z, (size_t)(s->L - 1) * E * B * H, Z);
+        SG_NEED(s, B_ACT, (size_t)(s->L - 1) * E * B * H, act);
+        SG_NEED(s, B_OUT, (size_t)E * B * kPad, out);
+        SG_NEED(s, B_DYF, (size_t)E * B * kPad, dyf);
+        SG_NEED(s, B_DYB, (size_t)E * B * kPad, dyb);
+    }
+    SG_NEED(s, B_WSUM, fused ? (size_t)E * steps : (size_t)E, wsum);
     SG_NEED(s, B_LOSS, (size_t)E * parts * steps, loss);
     std::vector<uint32_t> order(n), hidx((size_t)E * B * steps);
     std::vector<float> hl((size_t)E * parts * steps);
@@ -498,7 +540,19 @@ gs_status gs_surrogate_train(gs_surrogate *s, const float *x, const float *y, co
                           hidx.begin() + ((size_t)k * E + m) * B);
         }
         SG_TRY(s, hipMemcpyAsync(idx, hidx.data(), hidx.size() * sizeof(uint32_t), hipMemcpyHostToDevice, s->stream));
+        if (fused) SG_TRY(s, sg_launch_wsum(W, idx, B, steps, E, wsum, s->stream));
         for (int k = 0; k < steps; ++k) {
+            if (fused) {
+                ta.idx = idx + (size_t)k * E * B;
+                ta.wsum = wsum + (size_t)k * E;
+                ta.loss_part = loss + (size_t)k * E * parts;
+                SG_TRY(s, sg_launch_train_tile(ta, E, s->stream));
+                ++s->step;
+                const AdamArgs aa{c.lr, c.beta1, c.beta2, c.eps, c.weight_decay, 1.0f - std::pow(c.beta1, (float)s->step),
+                                  1.0f - std::pow(c.beta2, (float)s->step)};
+                SG_TRY(s, sg_launch_train_weights(ta, &aa, E, s->stream));
+                continue;
+            }
             SG_TRY(s, sg_launch_gather(X, Y, W, idx + (size_t)k * E * B, B, kPad, kPad, bx, by, bw, E, s->stream));
             st = forward(s, bx, (size_t)B * kPad, B, Z, act, out);
             if (st != GS_OK) return st;
@@ -540,33 +594,53 @@ gs_status gs_surrogate_gradients(gs_surrogate *s, const float *x, const float *y
     if (st != GS_OK) return st;
     const int E = s->E, H = (int)s->cfg.hidden;
     std::vector<float> yh = pad_rows(yp.data(), rows, s->cfg.n_outputs), wh = pad_rows(wp.data(), rows, s->cfg.n_outputs);
-    // the same rows for every member
-    std::vector<float> ye, we;
-    for (int m = 0; m < E; ++m) {
-        ye.insert(ye.end(), yh.begin(), yh.end());
-        we.insert(we.end(), wh.begin(), wh.end());
-    }
-    float *by, *bw, *Z, *out, *dyf, *wsum, *loss;
-    __bf16 *act, *dyb;
-    const int parts = 8;
-    SG_NEED(s, B_BY, ye.size(), by);
-    SG_NEED(s, B_BW, we.size(), bw);
-    SG_NEED(s, B_Z, (size_t)(s->L - 1) * E * rows * H, Z);
-    SG_NEED(s, B_ACT, (size_t)(s->L - 1) * E * rows * H, act);
-    SG_NEED(s, B_OUT, (size_t)E * rows * kPad, out);
-    SG_NEED(s, B_DYF, (size_t)E * rows * kPad, dyf);
-    SG_NEED(s, B_DYB, (size_t)E * rows * kPad, dyb);
+    const bool fused = fused_shape(s);
+    const int parts = fused ? (int)rows / 16 : 8;
+    float *by, *bw, *wsum, *loss;
     SG_NEED(s, B_WSUM, (size_t)E, wsum);
     SG_NEED(s, B_LOSS, (size_t)E * parts, loss);
-    SG_TRY(s, hipMemcpyAsync(by, ye.data(), ye.size() * sizeof(float), hipMemcpyHostToDevice, s->stream));
-    SG_TRY(s, hipMemcpyAsync(bw, we.data(), we.size() * sizeof(float), hipMemcpyHostToDevice, s->stream));
-    st = forward(s, X, 0, (int)rows, Z, act, out);
-    if (st != GS_OK) return st;
-    SG_TRY(s, sg_launch_loss(out, by, bw, (int)rows * kPad, (size_t)rows * kPad, (size_t)rows * kPad, wsum, dyf, dyb,
-                             loss, parts, E, s->stream));
-    // The first layer reads the shared inputs (member stride 0).
-    st = backward(s, X, 0, (int)rows, Z, act, dyf, dyb);
-    if (st != GS_OK) return st;
+    std::vector<float> ye, we;   // must outlive the copies
+    if (fused) {   // every member reads the same rows
+        SG_NEED(s, B_BY, yh.size(), by);
+        SG_NEED(s, B_BW, wh.size(), bw);
+        SG_TRY(s, hipMemcpyAsync(by, yh.data(), yh.size() * sizeof(float), hipMemcpyHostToDevice, s->stream));
+        SG_TRY(s, hipMemcpyAsync(bw, wh.data(), wh.size() * sizeof(float), hipMemcpyHostToDevice, s->stream));
+        TrainArgs ta;
+        st = train_args(s, (int)rows, ta);
+        if (st != GS_OK) return st;
+        ta.X = X;
+        ta.Y = by;
+        ta.W = bw;
+        ta.wsum = wsum;
+        ta.loss_part = loss;
+        for (int m = 0; m < E; ++m) SG_TRY(s, sg_launch_wsum(bw, nullptr, (int)rows, 1, 1, wsum + m, s->stream));
+        SG_TRY(s, sg_launch_train_tile(ta, E, s->stream));
+        SG_TRY(s, sg_launch_train_weights(ta, nullptr, E, s->stream));
+    } else {
+        float *Z, *out, *dyf;
+        __bf16 *act, *dyb;
+        // the same rows for every member
+        for (int m = 0; m < E; ++m) {
+            ye.insert(ye.end(), yh.begin(), yh.end());
+            we.insert(we.end(), wh.begin(), wh.end());
+        }
+        SG_NEED(s, B_BY, ye.size(), by);
+        SG_NEED(s, B_BW, we.size(), bw);
+        SG_NEED(s, B_Z, (size_t)(s->L - 1) * E * rows * H, Z);
+        SG_NEED(s, B_ACT, (size_t)(s->L - 1) * E * rows * H, act);
+        SG_NEED(s, B_OUT, (size_t)E * rows * kPad, out);
+        SG_NEED(s, B_DYF, (size_t)E * rows * kPad, dyf);
+        SG_NEED(s, B_DYB, (size_t)E * rows * kPad, dyb);
+        SG_TRY(s, hipMemcpyAsync(by, ye.data(), ye.size() * sizeof(float), hipMemcpyHostToDevice, s->stream));
+        SG_TRY(s, hipMemcpyAsync(bw, we.data(), we.size() * sizeof(float), hipMemcpyHostToDevice, s->stream));
+        st = forward(s, X, 0, (int)rows, Z, act, out);
+        if (st != GS_OK) return st;
+        SG_TRY(s, sg_launch_loss(out, by, bw, (int)rows * kPad, (size_t)rows * kPad, (size_t)rows * kPad, wsum, dyf, dyb,
+                                 loss, parts, E, s->stream));
+        // The first layer reads the shared inputs (member stride 0).
+        st = backward(s, X, 0, (int)rows, Z, act, dyf, dyb);
+        if (st != GS_OK) return st;
+    }
     SG_TRY(s, hipMemcpyAsync(grads, s->G, (size_t)E * s->Pm * sizeof(float), hipMemcpyDeviceToHost, s->stream));
     std::vector<float> hl((size_t)E * parts);
     SG_TRY(s, hipMemcpyAsync(hl.data(), loss, hl.size() * sizeof(float), hipMemcpyDeviceToHost, s->stream));

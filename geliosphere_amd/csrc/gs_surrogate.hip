@@ -18,6 +18,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "gs_surrogate_kernels.h"
 
 namespace gs {
@@ -27,6 +29,20 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int TM = 64, TN = 64, TK = 32, LDS_ROW = TK + 8;
+
+// Fragment order of a matrix M[n][k], k a multiple of 32: blocks of 16 n x 32 k
+// as the 64 lanes of an MFMA hold them, lane l the 8 values M[16 nt + l % 16][32
+// ks + 8 (l / 16) ..], so that a wave's operand load is 1 KB of consecutive
+// bytes.  Read row by row (16 pieces of 64 bytes per load) the same operands
+// came at 8 to 16 bytes per cycle and CU.
+__host__ __device__ inline size_t frag_at(int n, int k, int K) {
+    return (((size_t)(n >> 4) * (size_t)(K >> 5) + (size_t)(k >> 5)) * 64 + (size_t)((k >> 3) & 3) * 16 + (size_t)(n & 15)) * 8 +
+           (size_t)(k & 7);
+}
+// Lane `lane`'s fragment of block (nt, ks).
+__device__ __forceinline__ bf16x8 frag(const __bf16 *M, int K, int nt, int ks, int lane) {
+    return *(const bf16x8 *)(M + (((size_t)nt * (size_t)(K >> 5) + (size_t)ks) * 64 + (size_t)lane) * 8);
+}
 
 __device__ __forceinline__ float silu(float z) { return z / (1.0f + __expf(-z)); }
 __device__ __forceinline__ float dsilu(float z) {
@@ -138,7 +154,7 @@ __device__ __forceinline__ void mlp_hidden_layer(__bf16 *buf, const __bf16 *W, c
     for (int k0 = 0; k0 < K; k0 += 32) {
         bf16x8 b[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) b[j] = *(const bf16x8 *)(W + (size_t)(n0 + 16 * j + fr) * K + k0 + fk);
+        for (int j = 0; j < 4; ++j) b[j] = frag(W, K, 4 * wave + j, k0 / 32, lane);
 #pragma unroll
         for (int i = 0; i < FRT; ++i) {
             const bf16x8 a = *(const bf16x8 *)(buf + (16 * i + fr) * FLD + k0 + fk);
@@ -193,7 +209,7 @@ __global__ void __launch_bounds__(256, 2) mlp_forward_kernel(MlpArgs g) {
     for (int k0 = 0; k0 < FH; k0 += 32) {
         bf16x8 b[2];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) b[j] = *(const bf16x8 *)(W + (size_t)(16 * j + fr) * FH + k0 + fk);
+        for (int j = 0; j < 2; ++j) b[j] = frag(W, FH, j, k0 / 32, lane);
 #pragma unroll
         for (int i = 0; i < ORT; ++i) {
             const bf16x8 a = *(const bf16x8 *)(act + (r0 + 16 * i + fr) * FLD + k0 + fk);
@@ -213,14 +229,23 @@ __global__ void __launch_bounds__(256, 2) mlp_forward_kernel(MlpArgs g) {
 }
 
 // Column sums of a [rows x cols] fp32 matrix per member (bias gradients).
-// One thread per column, rows walked in order: deterministic.
+// One thread per column, rows added in order: deterministic.  Networks without
+// the fused training kernels only; 16 rows are loaded ahead of their sums.
 __global__ void colsum_kernel(const float *X, int rows, int cols, size_t strideX, float *out, size_t strideOut) {
     const int e = blockIdx.y;
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= cols) return;
     const float *x = X + (size_t)e * strideX;
     float s = 0.f;
-    for (int r = 0; r < rows; ++r) s += x[(size_t)r * cols + c];
+    int r = 0;
+    for (; r + 16 <= rows; r += 16) {
+        float v[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = x[(size_t)(r + i) * cols + c];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s += v[i];
+    }
+    for (; r < rows; ++r) s += x[(size_t)r * cols + c];
     out[(size_t)e * strideOut + c] = s;
 }
 
@@ -279,20 +304,362 @@ __global__ void gather_kernel(const __bf16 *X, const float *Y, const float *W, c
     }
 }
 
-// Adam (decoupled weight decay) over the flat parameter vector of every
-// member; refreshes the bf16 copy the GEMMs read.
+// Adam (decoupled weight decay) of one parameter, the fused multiply-adds
+// written out so that every kernel rounds alike.
+__device__ __forceinline__ float adam_update(float p, float g, float &mo, float &ve, float lr, float b1, float b2,
+                                             float eps, float wd, float c1, float c2) {
+    const float m = fmaf(1.0f - b1, g, b1 * mo);
+    const float v = fmaf(g, (1.0f - b2) * g, b2 * ve);
+    mo = m;
+    ve = v;
+    return fmaf(-lr, fmaf(wd, p, (m / c1) / (sqrtf(v / c2) + eps)), p);
+}
+
+// Adam over the flat parameter vector of every member; refreshes the bf16
+// copy the GEMMs read.
 __global__ void adam_kernel(float *P, const float *G, float *Mo, float *Ve, __bf16 *Pb, size_t n, float lr,
                             float b1, float b2, float eps, float wd, float c1, float c2) {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const float g = G[i];
-        const float m = b1 * Mo[i] + (1.0f - b1) * g;
-        const float v = b2 * Ve[i] + (1.0f - b2) * g * g;
+        float m = Mo[i], v = Ve[i];
+        const float p = adam_update(P[i], G[i], m, v, lr, b1, b2, eps, wd, c1, c2);
         Mo[i] = m;
         Ve[i] = v;
-        float p = P[i];
-        p -= lr * ((m / c1) / (sqrtf(v / c2) + eps) + wd * p);
         P[i] = p;
         Pb[i] = (__bf16)p;
+    }
+}
+
+// ---------------------------------------------------------------- fused training step
+// Layer by layer a training step was 29 launches, of which the column sums
+// (one thread per column, one row after another) took 590 of 870 us at
+// minibatches of 512 rows and 4 members.  Here a step is two launches:
+//  - train_tile_kernel takes a tile of 16 rows of one member through the
+//    forward pass, the loss and the data gradients.  A row's gradient chain
+//    touches no other row, so activations pass from layer to layer in LDS and
+//    pre-activations stay in the registers of the lanes that formed them
+//    (forward and backward give a lane the same elements).  What the weight
+//    gradients need goes out in their fragment order (frag_at, along the rows).
+//  - train_weights_kernel forms every layer's weight gradient (a wave takes
+//    32 x 32 elements over the whole minibatch, operands straight from L2)
+//    and bias gradient, and applies Adam to them where they are: the gradient
+//    never goes to memory.
+// 16 rows: at 512 rows x 4 members 128 workgroups.  16 waves (20.9 us at 8, 38 at
+// 4): a lone wave issues every 5 to 6 cycles and the SiLU of 16 elements each
+// was as long as a layer's product; a layer's 128 KB of weights are loaded into
+// registers while the layer before finishes.  Every sum is taken in the
+// layer-by-layer order (k ascending by 32 in the MFMAs, rows ascending in the
+// bias sums), so results are the same bits.
+// Measured per step, 512 rows x 4 members: 870 us of kernels before; 19 + 15 us.
+constexpr int BR = 16, BLD = 256 + 8;
+// Work item of workgroup b of n: items in order go to one die (workgroup b runs
+// on die b mod 8) in runs, so that a die reads the parameters of one member or
+// two instead of all.
+__device__ __forceinline__ int item_of(int b, int n) {
+    const int q = n / 8, r = n % 8, x = b % 8;
+    return x * q + (x < r ? x : r) + b / 8;
+}
+constexpr int TW = 16, TC = 256 / TW, TJ = TC / 16;   // waves per tile, columns and column tiles per wave
+
+struct WFrag {
+    bf16x8 f[8][TJ];   // [k step][column tile]
+};
+// The fragments of this wave's columns of a weight matrix with rows of K.
+template <int K>
+__device__ __forceinline__ void load_weights(WFrag &w, const __bf16 *W, int n0, int lane) {
+#pragma unroll
+    for (int k = 0; k < K / 32; ++k)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) w.f[k][j] = frag(W, K, n0 / 16 + j, k, lane);
+}
+template <int K>
+__device__ __forceinline__ void tile_product(f32x4 (&acc)[TJ], const __bf16 *buf, const WFrag &w, int fr, int fk) {
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < K / 32; ++k) {
+        const bf16x8 a = *(const bf16x8 *)(buf + fr * BLD + 32 * k + fk);
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w.f[k][j], acc[j], 0, 0, 0);
+    }
+}
+
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+
+// NH hidden layers of 256.
+template <int NH>
+__global__ void __launch_bounds__(TW * 64) train_tile_kernel(TrainArgs g) {
+    __shared__ __bf16 tile[2][BR * BLD];
+    __shared__ float red[2];
+    const int tiles = g.rows / BR, item = item_of((int)blockIdx.x, (int)gridDim.x);
+    const int e = item / tiles, tile_no = item % tiles, row0 = tile_no * BR;
+    const size_t E = gridDim.x / tiles;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int fr = lane & 15, quad = lane >> 4, fk = quad * 8, n0 = wave * TC;
+    const __bf16 *Pb = g.Pb + (size_t)e * g.Pm, *PbT = g.PbT + (size_t)e * g.Pm;
+    const float *P = g.P + (size_t)e * g.Pm;
+    const uint32_t *idx = g.idx ? g.idx + (size_t)e * g.rows : nullptr;
+    const size_t B = (size_t)g.rows;
+    // this lane's place in a column tile of the second launch's operands
+    // (fragments along the rows): 4 rows from row0 + 4 quad
+    const int b0 = row0 + 4 * quad;
+    auto operand = [&](__bf16 *M, size_t columns_before, int n) {
+        return (bf16x4 *)(M + columns_before * B + frag_at(n, b0, g.rows));
+    };
+    WFrag w;
+    load_weights<32>(w, Pb + g.woff[0], n0, lane);
+    if (t < BR * 4) {   // input tile
+        const int r = t >> 2, c = (t & 3) * 8;
+        const size_t row = idx ? (size_t)idx[row0 + r] : (size_t)(row0 + r);
+        const bf16x8 v = *(const bf16x8 *)(g.X + row * 32 + c);
+        *(bf16x8 *)(tile[0] + r * BLD + c) = v;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) g.XT[(size_t)e * 32 * B + frag_at(c + i, row0 + r, g.rows)] = v[i];
+    }
+    __syncthreads();
+    // ---- forward: layer l reads tile[l % 2] and writes the other
+    f32x4 z[NH][TJ];
+#pragma unroll
+    for (int l = 0; l < NH; ++l) {
+        f32x4 acc[TJ];
+        if (l == 0) tile_product<32>(acc, tile[0], w, fr, fk);
+        else tile_product<256>(acc, tile[l & 1], w, fr, fk);
+        if (l + 1 < NH) load_weights<256>(w, Pb + g.woff[l + 1], n0, lane);
+        __bf16 *out = tile[(l + 1) & 1];
+        const float *bias = P + g.boff[l];
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) {
+            const int n = n0 + 16 * j + fr;
+            const float bn = bias[n];
+            bf16x4 a;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                z[l][j][v] = acc[j][v] + bn;
+                a[v] = (__bf16)silu(z[l][j][v]);
+                out[(4 * quad + v) * BLD + n] = a[v];
+            }
+            *operand(g.ActT, ((size_t)l * E + e) * 256, n) = a;
+        }
+        __syncthreads();
+    }
+    // ---- output layer, loss and its gradient: waves 0 and 1, 16 columns each
+    const __bf16 *act = tile[NH & 1];
+    __bf16 *dout = tile[(NH + 1) & 1];
+    load_weights<32>(w, PbT + g.woff[NH], n0, lane);   // the first data gradient's
+    if (wave < 2) {
+        const int n = 16 * wave + fr;
+        const __bf16 *W = Pb + g.woff[NH];
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k0 = 0; k0 < 256; k0 += 32) {
+            const bf16x8 a = *(const bf16x8 *)(act + fr * BLD + k0 + fk);
+            const bf16x8 b = frag(W, 256, wave, k0 / 32, lane);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
+        }
+        const float bn = P[g.boff[NH] + n];
+        const float inv = 1.0f / fmaxf(g.wsum[e], 1e-30f);
+        float loss = 0.f;
+        bf16x4 gb;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int r = row0 + 4 * quad + v;
+            const size_t row = idx ? (size_t)idx[r] : (size_t)r;
+            const float y = acc[v] + bn, tt = g.Y[row * 32 + n], ww = g.W[row * 32 + n];
+            const float d = y - tt;
+            loss += ww * d * d * inv;
+            const float gr = 2.0f * ww * d * inv;
+            g.dYf[((size_t)e * B + r) * 32 + n] = gr;
+            gb[v] = (__bf16)gr;
+            dout[(4 * quad + v) * BLD + n] = gb[v];
+        }
+        *operand(g.dYT, (size_t)e * 32, n) = gb;
+#pragma unroll
+        for (int s = 32; s > 0; s >>= 1) loss += __shfl_xor(loss, s);
+        if (lane == 0) red[wave] = loss;
+    }
+    __syncthreads();
+    if (t == 0) g.loss_part[(size_t)e * tiles + tile_no] = red[0] + red[1];
+    // ---- data gradients: layer l's dZ from layer l + 1's
+#pragma unroll
+    for (int l = NH - 1; l >= 0; --l) {
+        const __bf16 *in = tile[(NH + 1 + NH - 1 - l) & 1];
+        __bf16 *out = tile[(NH + NH - 1 - l) & 1];
+        f32x4 acc[TJ];
+        if (l == NH - 1) tile_product<32>(acc, in, w, fr, fk);
+        else tile_product<256>(acc, in, w, fr, fk);
+        if (l > 0) load_weights<256>(w, PbT + g.woff[l], n0, lane);
+        const size_t at = ((size_t)l * E + e) * 256;
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) {
+            const int n = n0 + 16 * j + fr;
+            bf16x4 db;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const float d = acc[j][v] * dsilu(z[l][j][v]);
+                g.dZf[at * B + (size_t)(row0 + 4 * quad + v) * 256 + n] = d;
+                db[v] = (__bf16)d;
+                if (l > 0) out[(4 * quad + v) * BLD + n] = db[v];
+            }
+            *operand(g.dZT, at, n) = db;
+        }
+        if (l > 0) __syncthreads();
+    }
+}
+
+// Workgroup x of a member: 64 x 64 elements of one layer's weight gradient
+// (a wave 32 x 16), or, beyond those, 64 columns of a layer's bias gradient (one
+// wave: 512 dependent additions set its time, so the columns are spread).  The
+// output layer has 32 rows, the first layer 32 columns: the waves beyond have
+// nothing to do.
+constexpr int kBiasBlocks = 4;   // per layer; the output layer uses one
+template <bool kAdam>
+__global__ void __launch_bounds__(512) train_weights_kernel(TrainArgs g, AdamArgs a) {
+    const int L = g.L, blocks = 8 + 16 * (L - 2) + kBiasBlocks * (L - 1) + 1;   // of a member
+    const int item = item_of((int)blockIdx.x, (int)gridDim.x), e = item / blocks, bx = item % blocks;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const size_t B = (size_t)g.rows, E = gridDim.x / blocks;
+    const int n_tiles = 4 + 16 * (L - 2) + 4;
+    float *P = g.P + (size_t)e * g.Pm, *G = g.G + (size_t)e * g.Pm;
+    float *Mo = g.Mo + (size_t)e * g.Pm, *Ve = g.Ve + (size_t)e * g.Pm;
+    __bf16 *Pb = g.Pb + (size_t)e * g.Pm, *PbT = g.PbT + (size_t)e * g.Pm;
+    if (bx >= n_tiles) {   // bias of layer l: rows added in order
+        const int q = bx - n_tiles, l = q / kBiasBlocks, c = q % kBiasBlocks * 64 + t;
+        const int cols = l == L - 1 ? 32 : 256;
+        if (t >= 64 || c >= cols) return;
+        const float *x = l == L - 1 ? g.dYf + (size_t)e * B * 32 + c : g.dZf + ((size_t)l * E + e) * 256 * B + c;
+        const size_t o = g.boff[l] + c;
+        float m = 0.f, v = 0.f, p = 0.f;
+        if (kAdam) {
+            m = Mo[o];
+            v = Ve[o];
+            p = P[o];
+        }
+        float s = 0.f;
+        auto add_rows = [&](size_t r, auto rows) {
+            constexpr int R = decltype(rows)::value;
+            float d[R];
+#pragma unroll
+            for (int i = 0; i < R; ++i) d[i] = x[(r + i) * cols];
+#pragma unroll
+            for (int i = 0; i < R; ++i) s += d[i];
+        };
+        size_t r = 0;
+        for (; r + 128 <= B; r += 128) add_rows(r, std::integral_constant<int, 128>());
+        for (; r < B; r += 64) add_rows(r, std::integral_constant<int, 64>());
+        if (kAdam) {
+            p = adam_update(p, s, m, v, a.lr, a.b1, a.b2, a.eps, a.wd, a.c1, a.c2);
+            Mo[o] = m;
+            Ve[o] = v;
+            P[o] = p;
+        } else {
+            G[o] = s;
+        }
+        return;
+    }
+    int l, tm, tn;   // layer, tile row (outputs), tile column (inputs)
+    if (bx < 4) {
+        l = 0; tm = bx; tn = 0;
+    } else if (bx < n_tiles - 4) {
+        const int q = bx - 4;
+        l = 1 + q / 16; tm = (q % 16) / 4; tn = q % 4;
+    } else {
+        l = L - 1; tm = 0; tn = bx - (n_tiles - 4);
+    }
+    const int out_w = l == L - 1 ? 32 : 256, in_w = l == 0 ? 32 : 256;
+    const int m0 = tm * 64 + (wave >> 2) * 32, c0 = tn * 64 + (wave & 3) * 16;
+    if (m0 >= out_w || c0 >= in_w) return;
+    const __bf16 *A = l == L - 1 ? g.dYT + (size_t)e * 32 * B : g.dZT + ((size_t)l * E + e) * 256 * B;
+    const __bf16 *Bm = l == 0 ? g.XT + (size_t)e * 32 * B : g.ActT + ((size_t)(l - 1) * E + e) * 256 * B;
+    const int fr = lane & 15, quad = lane >> 4;
+    // Adam's operands, loaded before the product needs its own
+    const size_t o = g.woff[l] + (size_t)(m0 + 4 * quad) * in_w + c0 + fr;
+    float p[2][4], mo[2][4], ve[2][4];
+    if (kAdam) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const size_t ov = o + (size_t)(16 * i + v) * in_w;
+                p[i][v] = P[ov];
+                mo[i][v] = Mo[ov];
+                ve[i][v] = Ve[ov];
+            }
+    }
+    f32x4 acc[2];
+    acc[0] = acc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // 256 rows of loads in flight at once
+    auto rows_from = [&](int k0, auto steps) {
+        constexpr int S = decltype(steps)::value;
+        bf16x8 fa[S][2], fb[S];
+#pragma unroll
+        for (int k = 0; k < S; ++k) {
+            fb[k] = frag(Bm, g.rows, c0 / 16, k0 / 32 + k, lane);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) fa[k][i] = frag(A, g.rows, m0 / 16 + i, k0 / 32 + k, lane);
+        }
+#pragma unroll
+        for (int k = 0; k < S; ++k)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[k][i], fb[k], acc[i], 0, 0, 0);
+    };
+    int k0 = 0;
+    for (; k0 + 256 <= g.rows; k0 += 256) rows_from(k0, std::integral_constant<int, 8>());
+    for (; k0 < g.rows; k0 += 64) rows_from(k0, std::integral_constant<int, 2>());
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        if (kAdam) {
+            bf16x4 pt;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const size_t ov = o + (size_t)(16 * i + v) * in_w;
+                const float pn = adam_update(p[i][v], acc[i][v], mo[i][v], ve[i][v], a.lr, a.b1, a.b2, a.eps, a.wd, a.c1, a.c2);
+                Mo[ov] = mo[i][v];
+                Ve[ov] = ve[i][v];
+                P[ov] = pn;
+                pt[v] = (__bf16)pn;
+                Pb[g.woff[l] + frag_at(m0 + 16 * i + 4 * quad + v, c0 + fr, in_w)] = pt[v];
+            }
+            *(bf16x4 *)(PbT + g.woff[l] + frag_at(c0 + fr, m0 + 16 * i + 4 * quad, out_w)) = pt;
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v) G[o + (size_t)(16 * i + v) * in_w] = acc[i][v];
+        }
+    }
+}
+
+// wsum[step][e] in the order of wsum_kernel over the gathered minibatch.
+__global__ void __launch_bounds__(256) wsum_steps_kernel(const float *W, const uint32_t *idx, int rows, float *wsum) {
+    __shared__ float red[256];
+    const uint32_t *ix = idx ? idx + (size_t)blockIdx.x * rows : nullptr;
+    const int c = threadIdx.x & 31;
+    float s = 0.f;
+    for (int r = threadIdx.x >> 5; r < rows; r += 64) {   // rows: a multiple of 64
+        float w[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w[i] = W[(ix ? (size_t)ix[r + 8 * i] : (size_t)(r + 8 * i)) * 32 + c];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s += w[i];
+    }
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (int k = 128; k > 0; k >>= 1) {
+        if ((int)threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) wsum[blockIdx.x] = red[0];
+}
+
+// The weights of every layer in bf16 and fragment order: W [out][in] into Pb,
+// its transpose into PbT (when parameters are set; afterwards
+// train_weights_kernel keeps both).
+__global__ void __launch_bounds__(256) pack_kernel(TrainArgs g) {
+    const int e = blockIdx.y, l = blockIdx.z;
+    const int out_w = l == g.L - 1 ? 32 : 256, in_w = l == 0 ? 32 : 256;
+    const size_t at = (size_t)e * g.Pm + g.woff[l];
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < out_w * in_w; i += gridDim.x * 256) {
+        const int o = i / in_w, c = i % in_w;
+        const __bf16 v = (__bf16)g.P[at + i];
+        g.Pb[at + frag_at(o, c, in_w)] = v;
+        g.PbT[at + frag_at(c, o, out_w)] = v;
     }
 }
 
@@ -391,6 +758,42 @@ hipError_t sg_launch_gemm(bool a_col, bool b_col, int epi, const GemmArgs &g, in
 hipError_t sg_launch_mlp_forward(const MlpArgs &g, int members, hipStream_t s) {
     if (g.rows <= 0 || members <= 0 || g.L < 2 || g.L > kMlpMaxLayers) return hipErrorInvalidValue;
     hipLaunchKernelGGL(mlp_forward_kernel, dim3((unsigned)((g.rows + FR - 1) / FR), members), dim3(256), 0, s, g);
+    return hipGetLastError();
+}
+
+hipError_t sg_launch_wsum(const float *W, const uint32_t *idx, int rows, int steps, int members, float *wsum,
+                          hipStream_t s) {
+    if (rows <= 0 || rows % 64 || steps <= 0 || members <= 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(wsum_steps_kernel, dim3((unsigned)steps * (unsigned)members), dim3(256), 0, s, W, idx, rows, wsum);
+    return hipGetLastError();
+}
+
+hipError_t sg_launch_train_tile(const TrainArgs &g, int members, hipStream_t s) {
+    if (g.rows <= 0 || g.rows % 64 || members <= 0 || g.L < 2 || g.L > kMlpMaxLayers) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)(g.rows / BR) * (unsigned)members), block(TW * 64);
+    switch (g.L - 1) {
+    case 1: hipLaunchKernelGGL(train_tile_kernel<1>, grid, block, 0, s, g); break;
+    case 2: hipLaunchKernelGGL(train_tile_kernel<2>, grid, block, 0, s, g); break;
+    case 3: hipLaunchKernelGGL(train_tile_kernel<3>, grid, block, 0, s, g); break;
+    case 4: hipLaunchKernelGGL(train_tile_kernel<4>, grid, block, 0, s, g); break;
+    case 5: hipLaunchKernelGGL(train_tile_kernel<5>, grid, block, 0, s, g); break;
+    case 6: hipLaunchKernelGGL(train_tile_kernel<6>, grid, block, 0, s, g); break;
+    default: hipLaunchKernelGGL(train_tile_kernel<7>, grid, block, 0, s, g); break;
+    }
+    return hipGetLastError();
+}
+
+hipError_t sg_launch_train_weights(const TrainArgs &g, const AdamArgs *adam, int members, hipStream_t s) {
+    if (g.rows <= 0 || g.rows % 64 || members <= 0 || g.L < 2 || g.L > kMlpMaxLayers) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)(8 + 16 * (g.L - 2) + kBiasBlocks * (g.L - 1) + 1) * (unsigned)members), block(512);
+    if (adam) hipLaunchKernelGGL(train_weights_kernel<true>, grid, block, 0, s, g, *adam);
+    else hipLaunchKernelGGL(train_weights_kernel<false>, grid, block, 0, s, g, AdamArgs{});
+    return hipGetLastError();
+}
+
+hipError_t sg_launch_pack(const TrainArgs &g, int members, hipStream_t s) {
+    if (members <= 0 || g.L < 2 || g.L > kMlpMaxLayers) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(pack_kernel, dim3(32, (unsigned)members, (unsigned)g.L), dim3(256), 0, s, g);
     return hipGetLastError();
 }
 

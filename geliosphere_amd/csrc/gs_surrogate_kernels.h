@@ -32,12 +32,47 @@ constexpr int kMlpMaxLayers = 8;
 struct MlpArgs {
     const __bf16 *X;                    // [rows][32] standardised inputs
     int rows, L;                        // L weight layers
-    const __bf16 *Pb;                   // bf16 parameters, member stride Pm
+    const __bf16 *Pb;                   // bf16 weights in fragment order, member stride Pm
     const float *P;                     // fp32 parameters (biases)
     size_t Pm;
     size_t woff[kMlpMaxLayers], boff[kMlpMaxLayers];
     float *Out;                         // [members][rows][32]
 };
+
+// Fused training step of the same network shape: one launch for the forward
+// pass, the loss and the data gradients of every row tile, one for the weight
+// and bias gradients and Adam.  rows: a multiple of 64.
+struct TrainArgs {
+    const __bf16 *X;                    // standardised inputs [n][32]
+    const float *Y, *W;                 // targets and loss weights [n][32]
+    const uint32_t *idx;                // [members][rows] rows of the minibatch; nullptr: rows 0 .. rows-1
+    int rows, L;
+    float *P, *Mo, *Ve, *G;             // parameters, Adam moments, gradients (member stride Pm)
+    __bf16 *Pb, *PbT;                   // bf16 weights in fragment order, and with every weight transposed ([in][out])
+    size_t Pm;
+    size_t woff[kMlpMaxLayers], boff[kMlpMaxLayers];
+    const float *wsum;                  // [members] sums of the loss weights
+    // Written by the first launch for the second: bf16 operands of the products
+    // over the rows in fragment order ([columns][rows]), row-major fp32 for the
+    // bias sums.
+    __bf16 *XT;                         // [member][32][rows] inputs
+    __bf16 *ActT, *dZT;                 // [L-1][member][256][rows] activations, pre-activation gradients
+    float *dZf;                         // [L-1][member][rows][256]
+    __bf16 *dYT;                        // [member][32][rows] output gradients
+    float *dYf;                         // [member][rows][32]
+    float *loss_part;                   // [members][rows / 16]
+};
+struct AdamArgs {
+    float lr, b1, b2, eps, wd, c1, c2;
+};
+// Sums of the loss weights of `steps` consecutive minibatches: wsum[step][member].
+hipError_t sg_launch_wsum(const float *W, const uint32_t *idx, int rows, int steps, int members, float *wsum,
+                          hipStream_t s);
+hipError_t sg_launch_train_tile(const TrainArgs &g, int members, hipStream_t s);
+// adam == nullptr: gradients into G; otherwise the parameters are updated.
+hipError_t sg_launch_train_weights(const TrainArgs &g, const AdamArgs *adam, int members, hipStream_t s);
+// Pb and PbT from P.
+hipError_t sg_launch_pack(const TrainArgs &g, int members, hipStream_t s);
 
 hipError_t sg_launch_gemm(bool a_col, bool b_col, int epi, const GemmArgs &g, int members, hipStream_t s);
 hipError_t sg_launch_mlp_forward(const MlpArgs &g, int members, hipStream_t s);
