@@ -176,10 +176,16 @@ gs_status train_args(gs_surrogate *s, int rows, TrainArgs &g) {
     return GS_OK;
 }
 
-gs_status forward_infer(gs_surrogate *s, const __bf16 *X, int rows, float *Out) {
+// The members' outputs [E][rows][kPad] of raw inputs x [rows][n_inputs] in
+// device memory, or for fused shapes pinned host memory.
+gs_status forward_infer(gs_surrogate *s, const float *x, int rows, float *Out) {
+    const uint32_t ni = s->cfg.n_inputs;
     if (fused_shape(s)) {
         MlpArgs g{};
-        g.X = X;
+        g.x = x;
+        g.ni = (int)ni;
+        std::copy(s->mu, s->mu + ni, g.mu);
+        std::copy(s->sd, s->sd + ni, g.sd);
         g.rows = rows;
         g.L = s->L;
         g.Pb = s->Pb;
@@ -193,8 +199,10 @@ gs_status forward_infer(gs_surrogate *s, const __bf16 *X, int rows, float *Out) 
         SG_TRY(s, sg_launch_mlp_forward(g, s->E, s->stream));
         return GS_OK;
     }
-    __bf16 *act;
+    __bf16 *act, *X;
     SG_NEED(s, B_ACT, (size_t)(s->L - 1) * s->E * rows * s->cfg.hidden, act);
+    SG_NEED(s, B_X, (size_t)rows * kPad, X);
+    SG_TRY(s, sg_launch_standardise(x, rows, (int)ni, kPad, s->mu, s->sd, X, s->stream));
     return forward(s, X, 0, rows, nullptr, act, Out);
 }
 
@@ -257,16 +265,15 @@ gs_status backward(gs_surrogate *s, const __bf16 *X, size_t xstride, int rows, c
     return GS_OK;
 }
 
-// fp32 rows [n][n_inputs] (host memory, or device memory if x_on_device) ->
-// standardised, padded bf16 rows [n][kPad] on the device.
-gs_status upload_inputs(gs_surrogate *s, const float *x, uint32_t n, __bf16 **out, bool x_on_device = false) {
+// fp32 rows [n][n_inputs] in host memory -> standardised, padded bf16 rows
+// [n][kPad] on the device.
+gs_status upload_inputs(gs_surrogate *s, const float *x, uint32_t n, __bf16 **out) {
     const uint32_t ni = s->cfg.n_inputs;
     float *xf;
     __bf16 *xb;
     SG_NEED(s, B_XF, (size_t)n * ni, xf);
     SG_NEED(s, B_X, (size_t)n * kPad, xb);
-    SG_TRY(s, hipMemcpyAsync(xf, x, (size_t)n * ni * sizeof(float),
-                             x_on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s->stream));
+    SG_TRY(s, hipMemcpyAsync(xf, x, (size_t)n * ni * sizeof(float), hipMemcpyHostToDevice, s->stream));
     SG_TRY(s, sg_launch_standardise(xf, (int)n, (int)ni, kPad, s->mu, s->sd, xb, s->stream));
     SG_TRY(s, hipStreamSynchronize(s->stream));
     *out = xb;
@@ -654,9 +661,25 @@ gs_status gs_surrogate_gradients(gs_surrogate *s, const float *x, const float *y
     return GS_OK;
 }
 
+// Whether kernels of this surrogate may read x in place: memory of its device,
+// apart from the outputs (the statistics read the inputs again after other
+// queries' results are written).
+static bool reads_in_place(const gs_surrogate *s, const float *x, size_t n, const float *mean, const float *sd,
+                           const uint8_t *fallback) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, x) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (a.type != hipMemoryTypeDevice || a.device != s->device) return false;
+    const uintptr_t b = (uintptr_t)x, e = b + n * s->cfg.n_inputs * sizeof(float);
+    auto apart = [&](const void *p, size_t bytes) { return !p || (uintptr_t)p >= e || (uintptr_t)p + bytes <= b; };
+    const size_t out = n * s->cfg.n_outputs * sizeof(float);
+    return apart(mean, out) && apart(sd, out) && apart(fallback, n);
+}
+
 // Both predict entry points: host buffers (copied through the surrogate's
-// stream) or device buffers (the statistics and flags kernels write into the
-// caller's rows directly).
+// stream) or device buffers (read and written in place).
 static gs_status predict_rows(gs_surrogate *s, const float *x, uint32_t n, float *mean, float *sd,
                               uint8_t *fallback, bool on_device) {
     if (!s) return GS_ERR_INVALID_ARG;
@@ -666,39 +689,38 @@ static gs_status predict_rows(gs_surrogate *s, const float *x, uint32_t n, float
     const uint32_t no = s->cfg.n_outputs, ni = s->cfg.n_inputs;
     const int E = s->E;
     const uint32_t chunk = 65536;
+    const bool in_place = on_device && reads_in_place(s, x, n, mean, sd, fallback);
     for (uint32_t r0 = 0; r0 < n; r0 += chunk) {
         const uint32_t rows = std::min(chunk, n - r0);
-        __bf16 *X;
-        float *out, *dm, *ds;
-        gs_status st = upload_inputs(s, x + (size_t)r0 * ni, rows, &X, on_device);
-        if (st != GS_OK) return st;
-        SG_NEED(s, B_OUT, (size_t)E * rows * kPad, out);
-        if (on_device && mean) dm = mean + (size_t)r0 * no;
-        else SG_NEED(s, B_MEAN, (size_t)rows * no, dm);
-        if (on_device && sd) ds = sd + (size_t)r0 * no;
-        else SG_NEED(s, B_SD, (size_t)rows * no, ds);
-        st = forward_infer(s, X, (int)rows, out);
-        if (st != GS_OK) return st;
-        SG_TRY(s, sg_launch_stats(out, E, (int)rows, kPad, (int)no, (size_t)rows * kPad, dm, ds, s->stream));
-        // Flags on the device (from the raw inputs still in B_XF).
-        const size_t bytes = (size_t)rows * no * sizeof(float);
-        if (fallback) {
-            const float *xraw;
-            uint8_t *fl;
-            SG_NEED(s, B_XF, (size_t)rows * ni, xraw);
-            if (on_device) fl = fallback + r0;
-            else SG_NEED(s, B_FLAGS, (size_t)rows, fl);
-            SG_TRY(s, sg_launch_flags(ds, xraw, (int)rows, (int)no, (int)ni, s->cfg.std_outputs, s->cfg.std_limit,
-                                      s->lo, s->hi, fl, s->stream));
-            if (!on_device) SG_TRY(s, hipMemcpyAsync(fallback + r0, fl, rows, hipMemcpyDeviceToHost, s->stream));
+        const float *xr = x + (size_t)r0 * ni;
+        float *out, *dm = mean ? mean + (size_t)r0 * no : nullptr, *ds = sd ? sd + (size_t)r0 * no : nullptr;
+        uint8_t *fl = fallback ? fallback + r0 : nullptr;
+        if (!in_place) {
+            float *xf;
+            SG_NEED(s, B_XF, (size_t)rows * ni, xf);
+            SG_TRY(s, hipMemcpyAsync(xf, xr, (size_t)rows * ni * sizeof(float),
+                                     on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s->stream));
+            xr = xf;
         }
         if (!on_device) {
+            if (mean) SG_NEED(s, B_MEAN, (size_t)rows * no, dm);
+            if (sd) SG_NEED(s, B_SD, (size_t)rows * no, ds);
+            if (fallback) SG_NEED(s, B_FLAGS, (size_t)rows, fl);
+        }
+        SG_NEED(s, B_OUT, (size_t)E * rows * kPad, out);
+        gs_status st = forward_infer(s, xr, (int)rows, out);
+        if (st != GS_OK) return st;
+        SG_TRY(s, sg_launch_query_stats(out, E, (int)rows, (int)no, xr, (int)ni, s->cfg.std_outputs, s->cfg.std_limit,
+                                        s->lo, s->hi, dm, ds, fl, s->stream));
+        if (!on_device) {
+            const size_t bytes = (size_t)rows * no * sizeof(float);
+            if (fallback) SG_TRY(s, hipMemcpyAsync(fallback + r0, fl, rows, hipMemcpyDeviceToHost, s->stream));
             if (mean) SG_TRY(s, hipMemcpyAsync(mean + (size_t)r0 * no, dm, bytes, hipMemcpyDeviceToHost, s->stream));
             if (sd) SG_TRY(s, hipMemcpyAsync(sd + (size_t)r0 * no, ds, bytes, hipMemcpyDeviceToHost, s->stream));
         }
-        // B_XF and the scratch outputs are reused by the next chunk
-        SG_TRY(s, hipStreamSynchronize(s->stream));
     }
+    // the buffers are the next call's, and the outputs the caller's
+    SG_TRY(s, hipStreamSynchronize(s->stream));
     return GS_OK;
 }
 

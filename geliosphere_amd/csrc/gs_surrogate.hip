@@ -25,6 +25,7 @@
 namespace gs {
 namespace sg {
 
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -44,7 +45,14 @@ __device__ __forceinline__ bf16x8 frag(const __bf16 *M, int K, int nt, int ks, i
     return *(const bf16x8 *)(M + (((size_t)nt * (size_t)(K >> 5) + (size_t)ks) * 64 + (size_t)lane) * 8);
 }
 
-__device__ __forceinline__ float silu(float z) { return z / (1.0f + __expf(-z)); }
+// bf16(silu(z)), z / (1 + e^-z) with one Newton step in place of the IEEE division (div_fixup
+// keeps its zeros, infinities and NaN): over all 2^32 floats the same bf16 value
+// but for z in (-88.73, -87.33), results under 1e-36.  The division was half of
+// the activation's instructions.
+__device__ __forceinline__ __bf16 silu_act(float z) {
+    const float d = 1.0f + __expf(-z), y = __builtin_amdgcn_rcpf(d), q = z * y;
+    return (__bf16)__builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, z), y, q), d, z);
+}
 __device__ __forceinline__ float dsilu(float z) {
     const float s = 1.0f / (1.0f + __expf(-z));
     return s * (1.0f + z * (1.0f - s));
@@ -118,7 +126,7 @@ __global__ void __launch_bounds__(256) gemm_kernel(GemmArgs g) {
                 if (EPI == EPI_HIDDEN) {
                     const float z = x + g.bias[(size_t)e * g.strideBias + n];
                     if (g.Zf) g.Zf[o] = z;   // kept for the backward pass only
-                    g.Cb[o] = (__bf16)silu(z);
+                    g.Cb[o] = silu_act(z);
                 } else if (EPI == EPI_OUT) {
                     g.Cf[o] = x + g.bias[(size_t)e * g.strideBias + n];
                 } else if (EPI == EPI_DSILU) {
@@ -131,101 +139,131 @@ __global__ void __launch_bounds__(256) gemm_kernel(GemmArgs g) {
             }
 }
 
-// Fused inference of one member over a tile of FR rows: every layer runs in
-// one workgroup, with the bf16 activations held in LDS between layers instead
-// of making a round trip through HBM.  Hidden width 256, padded input and
-// output widths 32.  Each output element sees the same MFMA sequence as in
-// gemm_kernel (one 16x16x32 step per 32 values of k, k ascending) and the
-// same epilogue, so the outputs equal the layer-by-layer forward pass.
-constexpr int FR = 128, FH = 256, FLD = FH + 8, FRT = FR / 16;
+// Fused inference of one member over a tile of rows: standardisation of the
+// raw inputs, every layer in one workgroup with the bf16 activations in LDS,
+// no activation in memory.  Hidden width 256, padded input and output widths 32.
+// Each output element sees the MFMA sequence of gemm_kernel (16x16x32 steps, k
+// ascending) and the same epilogue, so the outputs equal the layer-by-layer
+// forward pass bit for bit.
+//  - The weights are the MFMA's first operand: a lane's four results are then
+//    neighbouring outputs of one row, which go to LDS as 8 bytes and to memory
+//    as 16.
+//  - Weight fragments stream from L2 (fragment order) kAheadK k steps ahead of
+//    their use, across layers, so that the epilogue of a layer hides the first
+//    loads of the next.
+//  - The SiLU is most of the vector work (two transcendentals and seven other
+//    operations per element): see silu_act.
+// RT row tiles of 16 by NW waves, chosen by sg_launch_mlp_forward.  Four waves per SIMD: two
+// (four waves of 64 columns each) gave 195 us instead of 160 for 65,536 rows of
+// four members.  There the products alone take 114 us, near the rate of a large
+// matrix product, and the activations 48 us beside them; before, with IEEE
+// divisions, 2-byte LDS writes and two k steps of loads, 190 us.  Ping-pong tiles
+// with the activations of one row tile scheduled into the products of the next
+// (twice the LDS, half the rows) gave 174 us, wave priorities nothing.
+template <int RT, int NW>
+struct MlpShape {
+    static constexpr int kRows = 16 * RT, kCols = 256 / NW, kColTiles = kCols / 16;
+    static constexpr int kAheadK = RT >= 4 ? 2 : RT == 2 ? 4 : 8;   // registers allow no more
+};
+constexpr int FH = 256, FLD = FH + 8;
 
-// One hidden layer in place: every wave reads the whole tile, then (after a
-// barrier) overwrites its own 64 columns with the activations.
-template <int K>
-__device__ __forceinline__ void mlp_hidden_layer(__bf16 *buf, const __bf16 *W, const float *bias, int lane,
-                                                 int wave) {
-    const int fr = lane & 15, fk = (lane >> 4) * 8, n0 = wave * 64;
-    f32x4 acc[FRT][4];
-#pragma unroll
-    for (int i = 0; i < FRT; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-    for (int k0 = 0; k0 < K; k0 += 32) {
-        bf16x8 b[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) b[j] = frag(W, K, 4 * wave + j, k0 / 32, lane);
-#pragma unroll
-        for (int i = 0; i < FRT; ++i) {
-            const bf16x8 a = *(const bf16x8 *)(buf + (16 * i + fr) * FLD + k0 + fk);
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[j], acc[i][j], 0, 0, 0);
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int n = n0 + 16 * j + fr;
-        const float bn = bias[n];
-#pragma unroll
-        for (int i = 0; i < FRT; ++i)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int m = 16 * i + 4 * (lane >> 4) + v;
-                buf[m * FLD + n] = (__bf16)silu(acc[i][j][v] + bn);
-            }
-    }
-}
-
-__global__ void __launch_bounds__(256, 2) mlp_forward_kernel(MlpArgs g) {
-    __shared__ __bf16 act[FR * FLD];
-    const int e = blockIdx.y, row0 = blockIdx.x * FR;
+template <int RT, int NW>
+__global__ void __launch_bounds__(NW * 64, 4) mlp_forward_kernel(MlpArgs g) {
+    using S = MlpShape<RT, NW>;
+    constexpr int CJ = S::kColTiles, AK = S::kAheadK;
+    __shared__ __bf16 act[S::kRows * FLD];
+    const int e = blockIdx.y, row0 = blockIdx.x * S::kRows;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int fr = lane & 15, quad = lane >> 4, ct0 = wave * CJ;   // first column tile
     const __bf16 *Pb = g.Pb + (size_t)e * g.Pm;
     const float *P = g.P + (size_t)e * g.Pm;
-    for (int q = t; q < FR * 4; q += 256) {   // input tile: FR rows x 32 bf16, zero beyond the last row
-        const int r = q >> 2, c = (q & 3) * 8;
-        bf16x8 v = {};
-        if (row0 + r < g.rows) v = *(const bf16x8 *)(g.X + (size_t)(row0 + r) * 32 + c);
-        *(bf16x8 *)(act + r * FLD + c) = v;
+    bf16x8 w[AK][CJ];
+    f32x4 acc[RT][CJ];
+    // the first layer's weights and the second's first steps
+    bf16x8 w0[CJ];
+#pragma unroll
+    for (int j = 0; j < CJ; ++j) w0[j] = frag(Pb + g.woff[0], 32, ct0 + j, 0, lane);
+    if (g.L > 2) {
+#pragma unroll
+        for (int k = 0; k < AK; ++k)
+#pragma unroll
+            for (int j = 0; j < CJ; ++j) w[k][j] = frag(Pb + g.woff[1], FH, ct0 + j, k, lane);
+    }
+    // standardised inputs, zero beyond the last row and column
+    const int sh = g.ni <= 8 ? 3 : g.ni <= 16 ? 4 : 5;
+    for (int q = t; q < S::kRows << sh; q += NW * 64) {
+        const int r = q >> sh, c = q & ((1 << sh) - 1);
+        float v = 0.0f;
+        if (c < g.ni && row0 + r < g.rows) v = (g.x[(size_t)(row0 + r) * g.ni + c] - g.mu[c]) / g.sd[c];
+        act[r * FLD + c] = (__bf16)v;
+    }
+    if (sh < 5)
+        for (int q = t; q < S::kRows * 3; q += NW * 64) {
+            const int r = q / 3, c = 8 * (q % 3 + 1);
+            if (c >= 1 << sh) *(bf16x8 *)(act + r * FLD + c) = bf16x8{};
+        }
+    __syncthreads();
+    auto epilogue = [&](const float *bias) {   // all waves have read the tile
+#pragma unroll
+        for (int j = 0; j < CJ; ++j) {
+            const int n = 16 * (ct0 + j) + 4 * quad;
+            const f32x4 b = *(const f32x4 *)(bias + n);
+#pragma unroll
+            for (int i = 0; i < RT; ++i) {
+                bf16x4 a;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) a[v] = silu_act(acc[i][j][v] + b[v]);
+                *(bf16x4 *)(act + (16 * i + fr) * FLD + n) = a;
+            }
+        }
+    };
+    auto row_frag = [&](int i, int k) { return *(const bf16x8 *)(act + (16 * i + fr) * FLD + 32 * k + 8 * quad); };
+    // ---- first layer, K = 32
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+        const bf16x8 a = row_frag(i, 0);
+#pragma unroll
+        for (int j = 0; j < CJ; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0[j], a, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
     }
     __syncthreads();
-    mlp_hidden_layer<32>(act, Pb + g.woff[0], P + g.boff[0], lane, wave);
+    epilogue(P + g.boff[0]);
     __syncthreads();
+    // ---- hidden layers, K = 256
+#pragma unroll 1
     for (int l = 1; l < g.L - 1; ++l) {
-        mlp_hidden_layer<FH>(act, Pb + g.woff[l], P + g.boff[l], lane, wave);
+        const __bf16 *W = Pb + g.woff[l], *Wn = Pb + g.woff[l + 1 < g.L - 1 ? l + 1 : l];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+#pragma unroll
+            for (int i = 0; i < RT; ++i) {
+                const bf16x8 a = row_frag(i, k);
+#pragma unroll
+                for (int j = 0; j < CJ; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[k % AK][j], a, k ? acc[i][j] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            }
+#pragma unroll
+            for (int j = 0; j < CJ; ++j)   // (after the last layer: its own first steps again, unused)
+                w[k % AK][j] = k + AK < 8 ? frag(W, FH, ct0 + j, k + AK, lane) : frag(Wn, FH, ct0 + j, k + AK - 8, lane);
+        }
+        __syncthreads();
+        epilogue(P + g.boff[l]);
         __syncthreads();
     }
-    // output layer, 32 padded columns: wave w owns rows FR/4 * w .. FR/4 * (w + 1) - 1
-    constexpr int ORT = FRT / 4;
-    const int l = g.L - 1, fr = lane & 15, fk = (lane >> 4) * 8, r0 = wave * (FR / 4);
-    const __bf16 *W = Pb + g.woff[l];
-    const float *bias = P + g.boff[l];
-    f32x4 acc[ORT][2];
+    // ---- output layer, 32 padded columns: 2 RT tiles over the waves
+    const __bf16 *W = Pb + g.woff[g.L - 1];
+    const float *bias = P + g.boff[g.L - 1];
 #pragma unroll
-    for (int i = 0; i < ORT; ++i) acc[i][0] = acc[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int task = 0; task < 2 * RT; task += NW) {
+        const int q = task + wave, i = q >> 1, j = q & 1;
+        if (q >= 2 * RT) break;
+        f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int k0 = 0; k0 < FH; k0 += 32) {
-        bf16x8 b[2];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) b[j] = frag(W, FH, j, k0 / 32, lane);
-#pragma unroll
-        for (int i = 0; i < ORT; ++i) {
-            const bf16x8 a = *(const bf16x8 *)(act + (r0 + 16 * i + fr) * FLD + k0 + fk);
-#pragma unroll
-            for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[j], acc[i][j], 0, 0, 0);
-        }
+        for (int k = 0; k < 8; ++k) o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(W, FH, j, k, lane), row_frag(i, k), o, 0, 0, 0);
+        const int n = 16 * j + 4 * quad, row = row0 + 16 * i + fr;
+        const f32x4 b = *(const f32x4 *)(bias + n);
+        if (row < g.rows) *(f32x4 *)(g.Out + ((size_t)e * g.rows + row) * 32 + n) = f32x4{o[0] + b[0], o[1] + b[1], o[2] + b[2], o[3] + b[3]};
     }
-#pragma unroll
-    for (int i = 0; i < ORT; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int m = r0 + 16 * i + 4 * (lane >> 4) + v, n = 16 * j + fr;
-                if (row0 + m < g.rows) g.Out[((size_t)e * g.rows + row0 + m) * 32 + n] = acc[i][j][v] + bias[n];
-            }
 }
 
 // Column sums of a [rows x cols] fp32 matrix per member (bias gradients).
@@ -383,7 +421,6 @@ __device__ __forceinline__ void tile_product(f32x4 (&acc)[TJ], const __bf16 *buf
     }
 }
 
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
 // NH hidden layers of 256.
 template <int NH>
@@ -434,7 +471,7 @@ __global__ void __launch_bounds__(TW * 64) train_tile_kernel(TrainArgs g) {
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 z[l][j][v] = acc[j][v] + bn;
-                a[v] = (__bf16)silu(z[l][j][v]);
+                a[v] = silu_act(z[l][j][v]);
                 out[(4 * quad + v) * BLD + n] = a[v];
             }
             *operand(g.ActT, ((size_t)l * E + e) * 256, n) = a;
@@ -690,39 +727,41 @@ struct FlagArgs {
     float lo[32], hi[32];
 };
 
-// Fallback flags, one thread per query: bit 0x1 when an output selected by
-// `mask` has a spread that is not <= `limit` (NaN included), bit 0x2 when an
-// input lies outside [lo, hi] (NaN included).
-__global__ void fallback_flags_kernel(const float *sd, const float *x, int n, int no, int ni, uint32_t mask,
-                                      float limit, FlagArgs b, uint8_t *flags) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n) return;
-    uint32_t f = 0;
-    for (int c = 0; c < no; ++c)
-        if (((mask >> c) & 1u) && !(sd[(size_t)r * no + c] <= limit)) f |= 0x1u;
-    for (int c = 0; c < ni; ++c) {
-        const float v = x[(size_t)r * ni + c];
-        if (!(v >= b.lo[c] && v <= b.hi[c])) f |= 0x2u;
+// Per query, half a wave: mean and (population) standard deviation over the
+// members of the outputs [E][n][32], first `no` columns, and the fallback flags:
+// bit 0x1 when an output selected by `mask` has a spread that is not <= `limit`
+// (NaN included), bit 0x2 when one of its ni inputs lies outside [lo, hi] (NaN
+// included).  mean, sd and flags may be null.  Reads 128 bytes per query and
+// member and is bound by that: as three launches (statistics, flags from the
+// spread in memory) it took 17 us for 65,536 queries.
+__global__ void __launch_bounds__(256) query_stats_kernel(const float *Y, int E, int n, int no, const float *x, int ni,
+                                                         uint32_t mask, float limit, FlagArgs b, float *mean, float *sd,
+                                                         uint8_t *flags) {
+    const int c = threadIdx.x & 31, lane = threadIdx.x & 63;
+    for (size_t r = (size_t)blockIdx.x * 8 + (threadIdx.x >> 5); r < (size_t)n; r += (size_t)gridDim.x * 8) {
+        float s = 0.f, s2 = 0.f;
+        for (int e = 0; e < E; ++e) {
+            const float y = Y[((size_t)e * n + r) * 32 + c];
+            s += y;
+            s2 = fmaf(y, y, s2);
+        }
+        const float mu = s / E;
+        const float sp = sqrtf(fmaxf(fmaf(-mu, mu, s2 / E), 0.f));
+        if (c < no) {
+            if (mean) mean[r * no + c] = mu;
+            if (sd) sd[r * no + c] = sp;
+        }
+        if (flags) {
+            bool out = false;
+            if (c < ni) {
+                const float v = x[r * ni + c];
+                out = !(v >= b.lo[c] && v <= b.hi[c]);
+            }
+            const uint64_t wide = __ballot(c < no && ((mask >> c) & 1u) && !(sp <= limit)), outside = __ballot(out);
+            const int half = lane & 32;
+            if (c == 0) flags[r] = (uint8_t)(((uint32_t)(wide >> half) ? 0x1u : 0u) | ((uint32_t)(outside >> half) ? 0x2u : 0u));
+        }
     }
-    flags[r] = (uint8_t)f;
-}
-
-// Mean and (population) standard deviation over the members of [E][n][ldy]
-// outputs, first `cols` columns.
-__global__ void ensemble_stats_kernel(const float *Y, int E, int n, int ldy, int cols, size_t strideY, float *mean,
-                                      float *sd) {
-    const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    if (i >= (size_t)n * cols) return;
-    const size_t r = i / cols, c = i % cols;
-    float s = 0.f, s2 = 0.f;
-    for (int e = 0; e < E; ++e) {
-        const float y = Y[(size_t)e * strideY + r * ldy + c];
-        s += y;
-        s2 += y * y;
-    }
-    const float mu = s / E;
-    mean[i] = mu;
-    sd[i] = sqrtf(fmaxf(s2 / E - mu * mu, 0.f));
 }
 
 }  // namespace sg
@@ -755,10 +794,26 @@ hipError_t sg_launch_gemm(bool a_col, bool b_col, int epi, const GemmArgs &g, in
     return hipErrorInvalidValue;
 }
 
-hipError_t sg_launch_mlp_forward(const MlpArgs &g, int members, hipStream_t s) {
-    if (g.rows <= 0 || members <= 0 || g.L < 2 || g.L > kMlpMaxLayers) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(mlp_forward_kernel, dim3((unsigned)((g.rows + FR - 1) / FR), members), dim3(256), 0, s, g);
+template <int RT, int NW>
+static hipError_t launch_mlp(const MlpArgs &g, int members, hipStream_t s) {
+    const int tile = MlpShape<RT, NW>::kRows;
+    hipLaunchKernelGGL((mlp_forward_kernel<RT, NW>), dim3((unsigned)((g.rows + tile - 1) / tile), (unsigned)members),
+                       dim3(NW * 64), 0, s, g);
     return hipGetLastError();
+}
+
+hipError_t sg_launch_mlp_forward(const MlpArgs &g, int members, hipStream_t s) {
+    if (g.rows <= 0 || members <= 0 || g.L < 2 || g.L > kMlpMaxLayers || g.ni < 1 || g.ni > 32) return hipErrorInvalidValue;
+    // The smallest tiles that fill the CUs: latency, and no long last wave of
+    // workgroups.  One call, four members, in us (tiles of 16 / 32 / 64 / 128 rows):
+    // 1 row 23 / 25 / 28 / 38; 2,048 rows 34 / 28 / 30 / 41; 8,192 rows 77 / 48 / 42 / 45;
+    // 20,011 rows 159 / 93 / 73 / 80; 40,000 rows 297 / 165 / 126 / 123; 65,536 rows
+    // 471 / 258 / 198 / 183.  256 CUs, two workgroups of 64 or 128 rows each.
+    const size_t rows = (size_t)g.rows * (size_t)members;
+    if (rows <= 16 * 256) return launch_mlp<1, 16>(g, members, s);
+    if (rows <= 32 * 256) return launch_mlp<2, 8>(g, members, s);
+    if (rows <= 64 * 2048) return launch_mlp<4, 8>(g, members, s);
+    return launch_mlp<8, 8>(g, members, s);
 }
 
 hipError_t sg_launch_wsum(const float *W, const uint32_t *idx, int rows, int steps, int members, float *wsum,
@@ -843,23 +898,16 @@ hipError_t sg_launch_standardise(const float *x, int n, int ni, int ldo, const f
     return hipGetLastError();
 }
 
-hipError_t sg_launch_flags(const float *sd, const float *x, int n, int no, int ni, uint32_t mask, float limit,
-                           const float *lo, const float *hi, uint8_t *flags, hipStream_t s) {
-    if (n <= 0 || no < 0 || no > 32 || ni < 1 || ni > 32) return hipErrorInvalidValue;
+hipError_t sg_launch_query_stats(const float *Y, int E, int n, int no, const float *x, int ni, uint32_t mask, float limit,
+                                 const float *lo, const float *hi, float *mean, float *sd, uint8_t *flags,
+                                 hipStream_t s) {
+    if (E <= 0 || n <= 0 || no < 0 || no > 32 || ni < 1 || ni > 32) return hipErrorInvalidValue;
     FlagArgs b{};
     for (int c = 0; c < ni; ++c) {
         b.lo[c] = lo[c];
         b.hi[c] = hi[c];
     }
-    hipLaunchKernelGGL(fallback_flags_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, sd, x, n, no, ni,
-                       mask, limit, b, flags);
-    return hipGetLastError();
-}
-
-hipError_t sg_launch_stats(const float *Y, int E, int n, int ldy, int cols, size_t strideY, float *mean, float *sd,
-                           hipStream_t s) {
-    const size_t total = (size_t)n * cols;
-    hipLaunchKernelGGL(ensemble_stats_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, Y, E, n, ldy,
-                       cols, strideY, mean, sd);
+    hipLaunchKernelGGL(query_stats_kernel, dim3((unsigned)((n + 7) / 8)), dim3(256), 0, s, Y, E, n, no, x, ni, mask, limit, b,
+                       mean, sd, flags);
     return hipGetLastError();
 }

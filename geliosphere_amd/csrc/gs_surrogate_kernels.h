@@ -26,11 +26,13 @@ struct GemmArgs {
     __bf16 *Cb;
 };
 
-// Fused inference (all layers of a member per 128-row tile, activations in LDS):
+// Fused inference (all layers of a member per row tile, activations in LDS):
 // hidden width 256, input and output padded to 32, 2..kMlpMaxLayers weight layers.
 constexpr int kMlpMaxLayers = 8;
 struct MlpArgs {
-    const __bf16 *X;                    // [rows][32] standardised inputs
+    const float *x;                     // [rows][ni] raw inputs, standardised as (x - mu) / sd
+    int ni;
+    float mu[32], sd[32];
     int rows, L;                        // L weight layers
     const __bf16 *Pb;                   // bf16 weights in fragment order, member stride Pm
     const float *P;                     // fp32 parameters (biases)
@@ -90,10 +92,10 @@ hipError_t sg_launch_to_bf16(const float *x, __bf16 *y, size_t n, hipStream_t s)
 // y = bf16((x - mu) / sd), with ni <= 32.
 hipError_t sg_launch_standardise(const float *x, int n, int ni, int ldo, const float *mu, const float *sd, __bf16 *y,
                                  hipStream_t s);
-// Fallback flags per query from the ensemble spread sd [n][no] and the raw
-// inputs x [n][ni]: 0x1 spread above limit on an output of mask, 0x2 input
-// outside [lo, hi]; no, ni <= 32.
-hipError_t sg_launch_flags(const float *sd, const float *x, int n, int no, int ni, uint32_t mask, float limit,
-                           const float *lo, const float *hi, uint8_t *flags, hipStream_t s);
-hipError_t sg_launch_stats(const float *Y, int E, int n, int ldy, int cols, size_t strideY, float *mean, float *sd,
-                           hipStream_t s);
+// Ensemble mean and spread of the outputs Y [E][n][32], first no columns, and
+// the fallback flags of the raw inputs x [n][ni]: 0x1 spread above limit on an
+// output of mask, 0x2 input outside [lo, hi]; no, ni <= 32.  mean, sd and flags
+// may be null.
+hipError_t sg_launch_query_stats(const float *Y, int E, int n, int no, const float *x, int ni, uint32_t mask, float limit,
+                                 const float *lo, const float *hi, float *mean, float *sd, uint8_t *flags,
+                                 hipStream_t s);
