@@ -70,6 +70,10 @@ struct gs_ctx {
     uint64_t cap_bcounts = 0;
     gs::SpillRec *d_spill = nullptr;     // hand-on records: two halves of cap_spill each
     uint64_t cap_spill = 0;
+    gs_exit_record *d_recs = nullptr;    // ordered exit records
+    uint64_t cap_recs = 0;
+    uint32_t *d_rec_at = nullptr;        // their counters (gs_records_scratch)
+    uint64_t cap_rec_at = 0;
     // launch shape per [plain, batch][model]; zero fields take the defaults
     // (256 threads, the occupancy's blocks per CU, kChunk ids per grab)
     gs_launch_shape shape[2][4] = {};
@@ -199,7 +203,15 @@ gs_status ensure_meta(gs_ctx *ctx, size_t words) {
 gs_status ensure_events(gs_ctx *ctx, uint64_t n) {
     if (ctx->cap_events >= n) return GS_OK;
     if (ctx->d_events) { (void)hipFree(ctx->d_events); ctx->d_events = nullptr; ctx->cap_events = 0; }
-    HIP_TRY(ctx, hipMalloc((void **)&ctx->d_events, n * sizeof(gs::DevEvent)));
+    hipError_t e = hipMalloc((void **)&ctx->d_events, n * sizeof(gs::DevEvent));
+    if (e == hipErrorOutOfMemory && ctx->d_recs) {   // events before the ordered copy of an earlier run's records
+        (void)hipGetLastError();
+        (void)hipFree(ctx->d_recs);
+        ctx->d_recs = nullptr;
+        ctx->cap_recs = 0;
+        e = hipMalloc((void **)&ctx->d_events, n * sizeof(gs::DevEvent));
+    }
+    HIP_TRY(ctx, e);
     ctx->cap_events = n;
     return GS_OK;
 }
@@ -440,6 +452,48 @@ gs_exit_record to_record(const gs::DevEvent &e) {
 
 bool record_less(const gs_exit_record &a, const gs_exit_record &b) {
     return a.id != b.id ? a.id < b.id : a.sumac < b.sumac;
+}
+
+// Room for n elements in a buffer that grows; false where the device has none.
+template <class T>
+bool grow(T *&p, uint64_t &cap, uint64_t n) {
+    if (cap >= n) return true;
+    if (p) (void)hipFree(p);
+    p = nullptr;
+    cap = 0;
+    if (hipMalloc((void **)&p, n * sizeof(T)) != hipSuccess) {
+        (void)hipGetLastError();
+        p = nullptr;
+        return false;
+    }
+    cap = n;
+    return true;
+}
+
+// The first `room` records of the nev > 0 events of a simulation, ordered, into
+// out.  Ordered on the device and copied as they are; few records (where the
+// seven launches, 40 us, cost more than the sort) and a device without room for
+// the ordered copy take the host's way.
+constexpr uint64_t kHostRecords = 512;
+gs_status ordered_records(gs_ctx *ctx, const gs_params &q, const gs::DevEvent *events, uint64_t nev, gs_exit_record *out,
+                          uint64_t room) {
+    const uint64_t kept = std::min(nev, room);
+    if (nev > kHostRecords && nev <= 0xFFFFFFFFull && grow(ctx->d_recs, ctx->cap_recs, nev) &&
+        grow(ctx->d_rec_at, ctx->cap_rec_at, gs_records_scratch(q.n_particles))) {
+        HIP_TRY(ctx, gs_launch_records(events, nev, q.first_particle, q.n_particles, q.model == GS_MODEL_1D_FP,
+                                       ctx->d_rec_at, ctx->d_recs, ctx->stream));
+        HIP_TRY(ctx, hipMemcpyAsync(out, ctx->d_recs, kept * sizeof(gs_exit_record), hipMemcpyDeviceToHost, ctx->stream));
+        HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+        return GS_OK;
+    }
+    std::vector<gs::DevEvent> h(nev);
+    HIP_TRY(ctx, hipMemcpyAsync(h.data(), events, nev * sizeof(gs::DevEvent), hipMemcpyDeviceToHost, ctx->stream));
+    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    std::vector<gs_exit_record> rs(nev);
+    for (uint64_t i = 0; i < nev; ++i) rs[i] = to_record(h[i]);
+    std::sort(rs.begin(), rs.end(), record_less);
+    std::copy(rs.begin(), rs.begin() + (ptrdiff_t)kept, out);
+    return GS_OK;
 }
 
 // Relative work per particle used to order a batch (heuristic only: it
@@ -717,14 +771,8 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
         if (R.n_recs) R.n_recs[i] = nev;
         if (R.want(i) && nev > 0) {
             // the simulation's event region, in gs_run_plain's record order
-            std::vector<gs::DevEvent> h(nev);
-            HIP_TRY(ctx, hipMemcpyAsync(h.data(), ctx->d_events + hmeta[j], nev * sizeof(gs::DevEvent),
-                                        hipMemcpyDeviceToHost, ctx->stream));
-            HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-            std::vector<gs_exit_record> rs(nev);
-            for (uint64_t e = 0; e < nev; ++e) rs[e] = to_record(h[e]);
-            std::sort(rs.begin(), rs.end(), record_less);
-            std::copy(rs.begin(), rs.begin() + (ptrdiff_t)std::min<uint64_t>(nev, R.caps[i]), R.recs[i]);
+            const gs_status rst = ordered_records(ctx, sims[i], ctx->d_events + hmeta[j], nev, R.recs[i], R.caps[i]);
+            if (rst != GS_OK) return rst;
         }
         acc.active_cycles += stats[gs::ST_STEPS];
     }
@@ -770,7 +818,7 @@ gs_status run_plain_core(gs_ctx *ctx, const gs_params &pp, gs_spectrum *out, gs_
     HIP_TRY(ctx, gs_launch_zero(B.words, kWordsPerSim, ctx->stream));
     const Resolved RS = resolve_shape(ctx, p->model, false);
     const unsigned grid = RS.grid;
-    std::vector<gs_exit_record> kept;   // records only (never with fixed buffers)
+    uint64_t kept = 0;   // records stored
     uint64_t total_events = 0;
     double kernel_ms = 0.0;
     const uint64_t N = p->n_particles;
@@ -874,15 +922,10 @@ gs_status run_plain_core(gs_ctx *ctx, const gs_params &pp, gs_spectrum *out, gs_
         HIP_TRY(ctx, gs_launch_fold(B.params, 1, O, fold_lds_bytes(q.n_bins, q.n_weights), fold_blocks(nev),
                                     ctx->stream));
         total_events += nev;
-        if (want_recs && nev > 0 && kept.size() < rec_cap) {
-            std::vector<gs::DevEvent> h(nev);
-            HIP_TRY(ctx, hipMemcpyAsync(h.data(), events, nev * sizeof(gs::DevEvent), hipMemcpyDeviceToHost,
-                                        ctx->stream));
-            HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-            std::vector<gs_exit_record> rs(nev);
-            for (uint64_t i = 0; i < nev; ++i) rs[i] = to_record(h[i]);
-            std::sort(rs.begin(), rs.end(), record_less);
-            for (uint64_t i = 0; i < nev && kept.size() < rec_cap; ++i) kept.push_back(rs[i]);
+        if (want_recs && nev > 0 && kept < rec_cap) {
+            st = ordered_records(ctx, q, events, nev, recs + kept, rec_cap - kept);
+            if (st != GS_OK) return st;
+            kept += std::min(nev, rec_cap - kept);
         }
         c0 += size;
         size = std::min(chunk_max, N - c0);
@@ -894,7 +937,6 @@ gs_status run_plain_core(gs_ctx *ctx, const gs_params &pp, gs_spectrum *out, gs_
     Layout H = layout(host, 1);
     H.stats[gs::ST_EVENTS] = total_events;
     fill_spectrum(*p, H.count, H.digits, H.stats, out);
-    if (want_recs) std::copy(kept.begin(), kept.end(), recs);
     if (n_recs) *n_recs = total_events;
     ctx->stats.kernel_ms = kernel_ms;
     ctx->stats.total_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_start).count();
@@ -963,6 +1005,8 @@ void gs_destroy(gs_ctx *ctx) {
     if (ctx->d_order_counts) (void)hipFree(ctx->d_order_counts);
     if (ctx->d_border) (void)hipFree(ctx->d_border);
     if (ctx->d_spill) (void)hipFree(ctx->d_spill);
+    if (ctx->d_recs) (void)hipFree(ctx->d_recs);
+    if (ctx->d_rec_at) (void)hipFree(ctx->d_rec_at);
     if (ctx->d_bcounts) (void)hipFree(ctx->d_bcounts);
     if (ctx->graph_exec) (void)hipGraphExecDestroy(ctx->graph_exec);
     for (int i = 0; i < 3; ++i) {

@@ -227,6 +227,12 @@ hipError_t gs_launch_order(const gs::DevParams *sims, uint64_t n, const gs::Orde
 // order where nb = 0).  counts: 2 * n_sims * kOrderSimBuckets words.
 hipError_t gs_launch_batch_order(const gs::DevParams *sims, uint32_t n_sims, const uint64_t *offsets, uint64_t n,
                                  uint32_t *counts, uint32_t *perm, hipStream_t s);
+// Records of one simulation's events (any order) by particle id, then by sumac
+// (several: a particle may have more than one); ids first .. first + n - 1,
+// n > 0, n_events < 2^32.  at: gs_records_scratch(n) words, 8-byte aligned.
+hipError_t gs_launch_records(const gs::DevEvent *events, uint64_t n_events, uint64_t first, uint64_t n, bool several,
+                             uint32_t *at, gs_exit_record *out, hipStream_t s);
+uint64_t gs_records_scratch(uint64_t n);
 // Histograms of n_sims simulations from their event regions; lds_bytes fits
 // the largest (n_bins, n_weights) among them.
 hipError_t gs_launch_fold(const gs::DevParams *sims, uint32_t n_sims, const gs::DevOut &O,
