@@ -388,8 +388,9 @@ struct Bp {
         W.hmin = min(W.hmin, h);
     }
     __device__ __forceinline__ bool fast_ok(const Watch &W, const Bp &old) const {
-        return W.hmax < kRHi && W.hmin > kRLo && hi_of(old.P) - (kPLo + 1) < kInf - (kPLo + 1) &&
-               hi_of(P) - (kPLo + 1) < kInf - (kPLo + 1);
+        // (int: no short circuits, each of which is a branch)
+        return (int)(W.hmax < kRHi) & (int)(W.hmin > kRLo) & (int)(hi_of(old.P) - (kPLo + 1) < kInf - (kPLo + 1)) &
+               (int)(hi_of(P) - (kPLo + 1) < kInf - (kPLo + 1));
     }
 };
 
@@ -482,7 +483,7 @@ struct Fp {
         W.hmin = min(W.hmin, h);
     }
     __device__ __forceinline__ bool fast_ok(const Watch &W, const Fp &old) const {
-        return W.hmax < kRHi && W.hmin > kRLo && beta >= 0.01 && old.beta >= 0.01;
+        return (int)(W.hmax < kRHi) & (int)(W.hmin > kRLo) & (int)(beta >= 0.01) & (int)(old.beta >= 0.01);
     }
 };
 

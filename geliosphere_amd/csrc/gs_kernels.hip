@@ -13,6 +13,7 @@
 // another lane's particle except at the very end of the run.
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "gs_device.hpp"
 #include "gs_kernels.h"
@@ -196,14 +197,14 @@ __device__ __forceinline__ void flush_block_stats(const uint64_t *stat, const De
 }
 
 // The cycle of a lane to which something happens (or the step cap comes
-// near): up to kCycleSteps full steps.  Returns whether the particle goes on;
+// near): up to kSteps full steps.  Returns whether the particle goes on;
 // `steps` counts the steps taken.
-template <class Model, class Prm, class Normals, class Emit>
+template <int kSteps, class Model, class Prm, class Normals, class Emit>
 __device__ __forceinline__ bool slow_cycle(Model &m, const Prm &P, const Normals &normals, const double *trig,
                                            uint32_t cap, uint32_t &steps, LaneStats &st, const Emit &emit) {
     bool active = true;
 #pragma unroll 1
-    for (int s = 0; s < kCycleSteps; ++s) {
+    for (int s = 0; s < kSteps; ++s) {
         double z[Model::kNormals];
         normals(s, z);
         if (active) {
@@ -432,12 +433,12 @@ __device__ void run_lanes(const DevParams *__restrict__ sims, uint32_t n_sims, c
                 m.fast_step(params(), z, bm.trig, watch);
             }
         }
-        const bool again = active && !(m.fast_ok(watch, old) && cap - steps >= (uint32_t)kCycleSteps);
+        const bool again = active & !((int)m.fast_ok(watch, old) & (int)(cap - steps >= (uint32_t)kCycleSteps));
         if (__ballot(again)) {
             if (again) {
                 m = old;
                 double q0 = z1[0], q1 = z1[1], q2 = z1[2], q3 = z1[3];
-                active = slow_cycle(
+                active = slow_cycle<kCycleSteps>(
                     m, params(),
                     [&](int s, double *z) {
                         if constexpr (NPS == 1) {
@@ -545,10 +546,18 @@ batch_kernel(const DevParams *__restrict__ sims, uint32_t n_sims, const uint64_t
 //    a 1D step's instructions, cost 1/G of that;
 //  - all G lanes carry the particle's state and do the same steps (the first
 //    of them emits and counts), so no lane is masked off and no step branches:
-//    every cycle runs as fast steps, then one test.
+//    kAtOnce cycles run as fast steps, then one test whether any has to be
+//    repeated in full steps.  A lone wave pays about 130 cycles for a test (the
+//    compare, the branch, the first normals' LDS latency), so where a wave holds
+//    few particles, whose events are then rare, it looks less often: per step
+//    93 -> 66 ns in 1D at 64 lanes (8 cycles to a test; 4: 66 to 73), 606 -> 566 ns
+//    SolarProp, 760 -> 711 ns Geliosphere (4 cycles; 2: 580 and 740; 4 of its
+//    cycles are 50 KB of code, and more would leave the instruction cache).
+//    (About 1 in 5000 lane-cycles of a 1D B-p run has an event.)
 // G is fixed within a launch.  After `budget` cycles the live particles are
 // handed to the next launch, which spreads the fewer particles over the same
-// lanes (in a batch: its model group's share of the dies); a launch that has 64 lanes per particle runs them to the end.
+// lanes (in a batch: its model group's share of the dies); a launch that has 64
+// lanes per particle runs them to the end.
 // Statistics and results do not depend on any of this.
 template <class Model>
 struct TailShape {
@@ -646,40 +655,47 @@ __global__ void __launch_bounds__(kTailThreads) tail_kernel(const DevParams *__r
         }
         __builtin_amdgcn_wave_barrier();
         blk += (uint32_t)(NPS * g);
-        // ---- g cycles
+        // ---- g cycles, kAtOnce to a test (both powers of two, kAtOnce <= g)
+        auto run_cycles = [&](auto at_once) {
+            constexpr int kAtOnce = decltype(at_once)::value, kSteps = kAtOnce * kCycleSteps;
 #pragma unroll 1
-        for (int c = 0; c < g; ++c) {
-            const double *zc = my + c * NPS * kCycleSteps;
-            const Model old = m;
-            typename Model::Watch watch = m.watch();
+            for (int c = 0; c < g; c += kAtOnce) {
+                const double *zc = my + c * NPS * kCycleSteps;
+                const Model old = m;
+                typename Model::Watch watch = m.watch();
 #pragma unroll
-            for (int s = 0; s < kCycleSteps; ++s) {
-                double z[NPS];
-                for (int i = 0; i < NPS; ++i) z[i] = zc[NPS * s + i];
-                m.fast_step(lp, z, bm.trig, watch);
-            }
-            const bool again = active && !(m.fast_ok(watch, old) && cap - steps >= (uint32_t)kCycleSteps);
-            ++cycles;
-            if (__ballot(again)) {
-                if (again) {
-                    m = old;
-                    LaneStats one{0, 0, 0, 0, 0};
-                    active = slow_cycle(
-                        m, lp, [&](int s, double *z) { for (int i = 0; i < NPS; ++i) z[i] = zc[NPS * s + i]; }, bm.trig,
-                        cap, steps, one, emit);
-                    steps -= (uint32_t)kCycleSteps;
-                    if (lead) {
-                        st.steps += one.steps;
-                        st.nan += one.nan;
-                        st.cap += one.cap;
-                        st.max_steps = one.max_steps > st.max_steps ? one.max_steps : st.max_steps;
-                    }
+                for (int s = 0; s < kSteps; ++s) {
+                    double z[NPS];
+                    for (int i = 0; i < NPS; ++i) z[i] = zc[NPS * s + i];
+                    m.fast_step(lp, z, bm.trig, watch);
                 }
-                stage_flush<kBatch>(&stage, O, kStageFlush);
-                if (__ballot(active) == 0) break;
+                const bool again = active & !((int)m.fast_ok(watch, old) & (int)(cap - steps >= (uint32_t)kSteps));
+                cycles += kAtOnce;
+                if (__ballot(again)) {
+                    if (again) {
+                        m = old;
+                        LaneStats one{0, 0, 0, 0, 0};
+                        active = slow_cycle<kSteps>(
+                            m, lp, [&](int s, double *z) { for (int i = 0; i < NPS; ++i) z[i] = zc[NPS * s + i]; },
+                            bm.trig, cap, steps, one, emit);
+                        steps -= (uint32_t)kSteps;
+                        if (lead) {
+                            st.steps += one.steps;
+                            st.nan += one.nan;
+                            st.cap += one.cap;
+                            st.max_steps = one.max_steps > st.max_steps ? one.max_steps : st.max_steps;
+                        }
+                    }
+                    stage_flush<kBatch>(&stage, O, kStageFlush);
+                    if (__ballot(active) == 0) break;
+                }
+                steps += (uint32_t)kSteps;
             }
-            steps += (uint32_t)kCycleSteps;
-        }
+        };
+        if (NPS == 1 && g == kWave) run_cycles(std::integral_constant<int, 8>());
+        else if (g >= 16) run_cycles(std::integral_constant<int, 4>());
+        else if (g >= 8) run_cycles(std::integral_constant<int, 2>());
+        else run_cycles(std::integral_constant<int, 1>());
     }
     const uint64_t live = __ballot(active && sub == 0);
     if (live) {   // the budget is spent: hand the live particles on

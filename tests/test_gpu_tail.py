@@ -43,6 +43,17 @@ def test_step_cap_inside_a_cycle(engine, model, max_steps):
     assert got.n_step_cap > 0 and got.total_steps <= 3000 * max_steps
 
 
+@pytest.mark.parametrize("model", MODELS)
+@pytest.mark.parametrize("n", (500, 3000, 6000, 20_000))   # 64, 16, 8 and 2 lanes to a particle
+@pytest.mark.parametrize("max_steps", (15, 33, 64, 1031))
+def test_step_cap_between_two_tests(engine, model, n, max_steps):
+    """Caps inside and at the ends of the cycles that are tested together."""
+    p = params(model, n, r_inj=1.0, T_min=0.01, max_steps=max_steps)
+    got, _, _ = engine.run_plain(p)
+    assert bytes(got) == bytes(engine.run_plain_noalloc(p))
+    assert got.n_step_cap > 0 and got.total_steps <= n * max_steps
+
+
 @pytest.mark.parametrize("model", MODELS[1:])
 def test_particles_that_end_at_once(engine, model):
     p = params(model, 500, r_inj=150.0)
