@@ -77,6 +77,7 @@ struct gs_ctx {
     // launch shape per [plain, batch][model]; zero fields take the defaults
     // (256 threads, the occupancy's blocks per CU, kChunk ids per grab)
     gs_launch_shape shape[2][4] = {};
+    bool tuning = false;            // the autotuner measures shapes as they are
     double tuned_rate[2][4] = {};   // particle-steps/s of the tuned shapes (0: not tuned)
     std::string arch;               // gcnArchName of the device
     // the device's fixed scratch array (gs_run_plain_noalloc), looked up once
@@ -400,6 +401,23 @@ uint64_t tail_lanes(const gs_ctx *ctx) { return (uint64_t)ctx->n_cu * 4 * gs::kW
 // throughput launch, or one per particle.
 uint64_t tail_cap(const gs_ctx *ctx, uint64_t n, uint64_t traj_lanes) {
     return std::max<uint64_t>(1, std::min<uint64_t>(n, std::max(traj_lanes, tail_lanes(ctx))));
+}
+
+// Workgroups of the throughput launch for n particles: as the shape says, but no
+// more than two waves per SIMD, or one for every kLaneParticles particles per lane.
+// With few particles per lane the launch's end is the run's: a lane of five waves
+// a SIMD takes a B-p step in 626 ns, one of two in 297, and what is left when the
+// ids run out is as long in steps either way.  B-p, five waves / two, in ms:
+// 500,000 particles 32 / 23, 1,000,000 44.5 / 37.5, 2,000,000 72 / 69; from there on
+// more waves (3,000,000: 98.5, 100.6, three 96.9).  Geliosphere, three / two:
+// 300,000 239 / 224, 1,000,000 83 / 79.  1D F-p ends on a few lone particles with
+// any number of waves.  (Plain runs only: a batch's groups fill each other's gaps;
+// there it cost a fifth.)
+constexpr uint64_t kLaneParticles = 16;
+unsigned throughput_grid(const gs_ctx *ctx, int model, const Resolved &R, uint64_t n) {
+    if (model == GS_MODEL_1D_FP || ctx->tuning) return R.grid;
+    const uint64_t waves = std::max<uint64_t>(2, n / (kLaneParticles * tail_lanes(ctx)));
+    return (unsigned)std::min<uint64_t>(R.grid, waves * tail_lanes(ctx) / R.block);
 }
 
 // Queues the tail launches of one run on stream s.  fresh_n > 0: the run's
@@ -817,7 +835,7 @@ gs_status run_plain_core(gs_ctx *ctx, const gs_params &pp, gs_spectrum *out, gs_
     Layout L = layout(B.words, 1);
     HIP_TRY(ctx, gs_launch_zero(B.words, kWordsPerSim, ctx->stream));
     const Resolved RS = resolve_shape(ctx, p->model, false);
-    const unsigned grid = RS.grid;
+    unsigned grid = RS.grid;
     uint64_t kept = 0;   // records stored
     uint64_t total_events = 0;
     double kernel_ms = 0.0;
@@ -830,7 +848,6 @@ gs_status run_plain_core(gs_ctx *ctx, const gs_params &pp, gs_spectrum *out, gs_
     O.order = nullptr;
     O.spill = nullptr; O.spill_count = nullptr; O.spill_cap = 0;
     O.chunk = RS.chunk;
-    const uint64_t lanes = (uint64_t)grid * RS.block;
     // largest chunk: 2^27 particles, or what the fixed event region holds
     // (B-p and 2D models emit at most one event per particle)
     const uint64_t chunk_max = B.own ? ctx->plain_chunk
@@ -878,7 +895,8 @@ gs_status run_plain_core(gs_ctx *ctx, const gs_params &pp, gs_spectrum *out, gs_
         HIP_TRY(ctx, gs_launch_zero(B.meta + 2, 2 + kTailRounds + 1, ctx->stream));   // events, cycles, hand-on counts
         O.events = events;
         // the tail needs the context's record buffer
-        const uint64_t cap_tail = tail_cap(ctx, q.n_particles, lanes);
+        if (B.own) grid = throughput_grid(ctx, q.model, RS, q.n_particles);
+        const uint64_t cap_tail = tail_cap(ctx, q.n_particles, (uint64_t)grid * RS.block);
         const bool fresh = B.own && q.n_particles > 0 && q.n_particles <= tail_lanes(ctx);
         if (B.own) {
             st = ensure_spill(ctx, cap_tail);
@@ -1123,8 +1141,10 @@ gs_status gs_autotune_shape(gs_ctx *ctx, const gs_params *pilots, uint32_t n_pil
         ctx->shape[kernel][model] = sh;
         double best = 0.0;
         for (uint32_t r = 0; r < repeats; ++r) {
+            ctx->tuning = true;
             const gs_status st = batch ? gs_run_batch(ctx, pilots, n_pilots, outs.data())
                                        : gs_run_plain(ctx, pilots, outs.data(), nullptr, 0, nullptr);
+            ctx->tuning = false;
             if (st != GS_OK) return st;
             uint64_t steps = 0;
             for (const gs_spectrum &o : outs) steps += o.total_steps;

@@ -246,8 +246,9 @@ gs_status gs_set_plain_limits(gs_ctx *ctx, uint64_t max_chunk, uint64_t max_even
 /* Launch shape of a trajectory kernel.  block_threads: workgroup size (128,
  * 256 or 512); blocks_per_cu: persistent blocks per CU, so that each lane
  * integrates about N / (blocks_per_cu x CUs x block_threads) particles one
- * after another (capped at the kernel's occupancy); chunk: particle ids a
- * wave takes from the work queue per grab.  0 in a field: the default (256,
+ * after another (capped at the kernel's occupancy; a plain run of fewer than
+ * 16 particles per lane launches fewer blocks); chunk: particle ids a wave
+ * takes from the work queue per grab.  0 in a field: the default (256,
  * the occupancy, 64).  Results never depend on the shape. */
 typedef struct gs_launch_shape {
     uint32_t block_threads;
