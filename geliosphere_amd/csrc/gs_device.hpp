@@ -298,107 +298,117 @@ __device__ void fold_one(const DevParams &P, uint64_t *lds, const DevEvent &e) {
 constexpr uint32_t hi_word(double x) { return (uint32_t)(__builtin_bit_cast(uint64_t, x) >> 32); }
 __device__ __forceinline__ uint32_t hi_of(double x) { return (uint32_t)(fm::double_to_bits(x) >> 32); }
 
-// The 1D models carry momenta in units of T0: P = pc / (q T0 1e9), so that
-// E^2 = P^2 + 1 takes the inline constant 1.0.  K = K0 beta P [GV] enters
-// only as sqrt(2 K dt) = sqrt(2 K0 dt T0) w with w = sqrt(beta P)
-// (Pm.sk2dt = sqrt(2 K0 dt T0)), and as 2 K dt / r = (sqrt(2 K dt))^2 / r.
-// With beta = P / E the common case has w = P E^(-1/2) = P q and beta =
-// P q^2, q = (P^2 + 1)^(-1/4) from one rsqrt4: one transcendental chain per
-// step instead of a 1/sqrt(E^2) and a sqrt(2 K dt).
+// The 1D models carry momenta in units of T0, P = pc / (q T0 1e9), so that E^2 =
+// P^2 + 1 and beta = P / E, and K = K0 beta P [GV] only as sK = sqrt(2 K dt) =
+// sqrt(2 K0 dt T0) sqrt(beta P), and as 2 K dt / r = sK^2 / r.  What they hold is S =
+// alpha P with alpha = 2 K0 dt T0 (Pm.al): then with E2 = S^2 + alpha^2 = alpha^2
+// E^2 and q = E2^(-1/4) from one rsqrt4,
+//   sK = S q    (alpha P / sqrt(alpha E)),    beta = S q^2    (alpha P / (alpha E)),
+// no factor left to multiply.  16 FP64 operations and 3 transcendental seeds per
+// B-p step (19 and 3 with P itself: 561 ms for 2e7 particles, now 538).  A
+// simulation whose alpha^2 is far from 1 (K0 dt beyond anything physical) has
+// alpha = 1 instead and sK = kappa S q (Pm.kap = sqrt(2 K0 dt T0); 1 otherwise)
+// and takes full steps only (Pm.s_lo).
 constexpr double kInvT0 = 1.0 / kT0;
+constexpr uint32_t kInfHi = 0x7ff00000u;
 
-// 1D B-p.  State: r [AU], P (units of T0), w = sqrt(beta P) with beta of
-// the last computed T, which a reflection does not restore
+// The kinetic energy T0 (E - 1) = T0 P^2 / (E + 1) at S.
+__device__ __forceinline__ double kinetic(const StepParams &Pm, double S) {
+    const double P = S * fm::rcp(Pm.al), P2 = P * P;
+    return kT0 * P2 * fm::rcp(fm::sqrt_nn(P2 + 1.0) + 1.0);
+}
+
+// 1D B-p.  State: r [AU], S, sK = sqrt(2 K dt) with the beta of the last
+// computed T, which a reflection does not restore
 // (OneDimensionBpCpuModel.cpp:108-140).  Pm.vdt = -V dt and Pm.cp =
 // -(2/3) V dt carry the backward sign of V (Constants.hpp:213-218).
-// T = T0 (E - 1) is formed only for an exit; the test T < 200 is
-// E^2 < ((200 + T0) / T0)^2.
+// T is formed only for an exit; the test T < 200 is E^2 < ((200 + T0) / T0)^2.
 struct Bp {
     static constexpr int kNormals = 1;
     static constexpr bool kLatencyBound = false;
     static constexpr bool kVecParams = false;
     __device__ static void to_vgprs(StepParams &) {}
     static constexpr double kE2Exit = ((200.0 + kT0) * kInvT0) * ((200.0 + kT0) * kInvT0);
-    double r, P, w, t_inj;
-    __device__ __forceinline__ void save(double *s) const { s[0] = r; s[1] = P; s[2] = w; s[3] = t_inj; }
-    __device__ __forceinline__ void load(const double *s) { r = s[0]; P = s[1]; w = s[2]; t_inj = s[3]; }
+    double r, S, sK, t_inj;
+    __device__ __forceinline__ void save(double *s) const { s[0] = r; s[1] = S; s[2] = sK; s[3] = t_inj; }
+    __device__ __forceinline__ void load(const double *s) { r = s[0]; S = s[1]; sK = s[2]; t_inj = s[3]; }
     __device__ __forceinline__ bool init(const StepParams &Pm, double T) {
         t_inj = T;
         const double t = T * kInvT0;
-        P = fm::sqrt_nn(t * (t + 2.0));
-        w = P * fm::rsqrt(t + 1.0);   // E = t + 1
+        const double P = fm::sqrt_nn(t * (t + 2.0));
+        S = Pm.al * P;
+        sK = Pm.sk2dt * (P * fm::rsqrt(t + 1.0));   // E = t + 1
         r = Pm.r_inj;
         return r < 100.0002;
     }
     template <class Emit>
     __device__ __forceinline__ bool step(const StepParams &Pm, const double *z, const double *trig, const Emit &emit) {
         const double inv_r = fm::rcp(r);
-        const double sK = Pm.sk2dt * w;                                // sqrt(2 K dt)
-        const double Pn = fma(-(Pm.cp * P), inv_r, P);               // p - 2 V p dt / (3 r)
-        const double dr = sK * fma(sK, inv_r, z[0]) + Pm.vdt;       // (V + 2K/r) dt + z sqrt(2 K dt)
+        const double Sn = fma(-(Pm.cp * S), inv_r, S);               // p - 2 V p dt / (3 r)
+        const double t = fma(sK, inv_r, z[0]);                       // dr = (V + 2K/r) dt + z sqrt(2 K dt)
+        const double dr = fma(sK, t, Pm.vdt);
         const double rn = r + dr;
-        const double E2 = fma(Pn, Pn, 1.0);
+        const double E2 = fma(Sn, Sn, Pm.al2);
         const double q = fm::rsqrt4(E2);
-        const double invE = q * q;
-        const double bn = Pn * invE;
-        const double wn = Pn * q;
+        const double u = Sn * q;
+        const double sKn = u * Pm.kap;
+        const double bn = u * q;
         // Goes on while beta >= 0.01 (false for a NaN state, which ends it as
         // r < 100.0002 does in the reference loop).
         const bool alive = bn >= kBetaMinBp;
         if (rn > 100.0) {
             // at the outer boundary (no reflection possible): exit or end
-            const bool out = bn > kBetaMinBp && E2 < kE2Exit && rn - dr < 100.0;
-            if (out) emit(t_inj, kT0 * fma(E2, invE, -1.0), rn, 0.0, 0.0);
+            const bool out = bn > kBetaMinBp && E2 < kE2Exit * Pm.al2 && rn - dr < 100.0;
+            if (out) emit(t_inj, kinetic(Pm, Sn), rn, 0.0, 0.0);
             r = rn;
-            P = Pn;
-            w = wn;
+            S = Sn;
+            sK = sKn;
             return alive && !out && rn < 100.0002;
         }
         // r stays below 100.0002: rn <= 100.  A reflection restores the
         // previous r as r - dr and keeps P, while beta stays that of Pn; it
         // is rare, and a branch that a wave without one skips costs no
         // selects.
-        const double P0 = P;
+        const double S0 = S;
         r = rn;
-        P = Pn;
-        w = wn;
+        S = Sn;
+        sK = sKn;
         if (rn < kReflectBp) {
             asm volatile("");   // emits nothing; keeps the branch from becoming selects
             r = rn - dr;
-            P = P0;
-            w = fm::sqrt_nn(bn * P0);
+            S = S0;
+            sK = Pm.kap * fm::sqrt_nn(bn * S0);
         }
         return alive;
     }
     // Nothing happens while 0.31 < r < 99.99 after each step and beta stays
     // above 0.01: P grows from step to step (V > 0, r > 0), so it is enough that
-    // the first P of the cycle lies above 0.0101 (beta = 0.0100995), and the
-    // last is neither below that nor NaN.
+    // the first S of the cycle lies above 0.0101 alpha (beta = 0.0100995; Pm.s_lo
+    // holds its high word and one), and the last is neither below that nor NaN.
     struct Watch { uint32_t hmax, hmin; };
-    static constexpr uint32_t kRLo = hi_word(0.31), kRHi = hi_word(99.99), kPLo = hi_word(0.0101), kInf = 0x7ff00000u;
+    static constexpr uint32_t kRLo = hi_word(0.31), kRHi = hi_word(99.99);
     __device__ __forceinline__ Watch watch() const { return {0u, 0xffffffffu}; }
     __device__ __forceinline__ void fast_step(const StepParams &Pm, const double *z, const double *trig, Watch &W) {
         const double inv_r = fm::rcp(r);
-        const double sK = Pm.sk2dt * w;
-        P = fma(-(Pm.cp * P), inv_r, P);
-        r = r + (sK * fma(sK, inv_r, z[0]) + Pm.vdt);
-        w = P * fm::rsqrt4(fma(P, P, 1.0));
+        S = fma(-(Pm.cp * S), inv_r, S);
+        r = r + fma(sK, fma(sK, inv_r, z[0]), Pm.vdt);   // (not r + V dt first: it rounds the same way in every step)
+        sK = S * fm::rsqrt4(fma(S, S, Pm.al2));
         const uint32_t h = hi_of(r);
         W.hmax = max(W.hmax, h);
         W.hmin = min(W.hmin, h);
     }
-    __device__ __forceinline__ bool fast_ok(const Watch &W, const Bp &old) const {
+    __device__ __forceinline__ bool fast_ok(const StepParams &Pm, const Watch &W, const Bp &old) const {
         // (int: no short circuits, each of which is a branch)
-        return (int)(W.hmax < kRHi) & (int)(W.hmin > kRLo) & (int)(hi_of(old.P) - (kPLo + 1) < kInf - (kPLo + 1)) &
-               (int)(hi_of(P) - (kPLo + 1) < kInf - (kPLo + 1));
+        return (int)(W.hmax < kRHi) & (int)(W.hmin > kRLo) & (int)(hi_of(old.S) - Pm.s_lo < kInfHi - Pm.s_lo) &
+               (int)(hi_of(S) - Pm.s_lo < kInfHi - Pm.s_lo);
     }
 };
 
-// 1D F-p.  State: r, P (units of T0), beta of the last computed T, w =
-// sqrt(beta R) with R = that T's momentum (a reflection keeps P but not
-// beta or R), sumac.  OneDimensionFpCpuModel.cpp:84-152.  Pm.vdt = V dt,
-// Pm.cp = (2/3) V dt, Pm.csum = (4/3) V dt.  T is formed only for a
-// crossing; the test T < 100 is E^2 < ((100 + T0) / T0)^2.
+// 1D F-p.  State: r, S, beta of the last computed T, sK = sqrt(2 K dt) with
+// that T's beta and momentum (a reflection keeps S but not beta or sK), sumac.
+// OneDimensionFpCpuModel.cpp:84-152.  Pm.vdt = V dt, Pm.cp = (2/3) V dt,
+// Pm.csum = (4/3) V dt.  T is formed only for a crossing; the test T < 100 is
+// E^2 < ((100 + T0) / T0)^2.
 struct Fp {
     static constexpr int kNormals = 1;
     // A run lasts as long as its longest trajectory (a lone wave at the end),
@@ -409,23 +419,23 @@ struct Fp {
     static constexpr bool kLatencyBound = true;
     static constexpr bool kVecParams = true;
     __device__ static void to_vgprs(StepParams &p) {
-        asm volatile("" : "+v"(p.cp), "+v"(p.csum), "+v"(p.sk2dt), "+v"(p.vdt));
+        asm volatile("" : "+v"(p.cp), "+v"(p.csum), "+v"(p.al2), "+v"(p.vdt));
     }
     static constexpr double kE2Cross = ((100.0 + kT0) * kInvT0) * ((100.0 + kT0) * kInvT0);
-    double r, P, beta, w, sumac, t_inj;
+    double r, S, beta, sK, sumac, t_inj;
     __device__ __forceinline__ void save(double *s) const {
-        s[0] = r; s[1] = P; s[2] = beta; s[3] = w; s[4] = sumac; s[5] = t_inj;
+        s[0] = r; s[1] = S; s[2] = beta; s[3] = sK; s[4] = sumac; s[5] = t_inj;
     }
     __device__ __forceinline__ void load(const double *s) {
-        r = s[0]; P = s[1]; beta = s[2]; w = s[3]; sumac = s[4]; t_inj = s[5];
+        r = s[0]; S = s[1]; beta = s[2]; sK = s[3]; sumac = s[4]; t_inj = s[5];
     }
     __device__ __forceinline__ bool init(const StepParams &Pm, double T) {
         t_inj = T;
         const double t = T * kInvT0;
-        P = fm::sqrt_nn(t * (t + 2.0));
-        const double q2 = fm::rcp(t + 1.0);   // 1/E
-        beta = P * q2;
-        w = P * fm::rsqrt(t + 1.0);
+        const double P = fm::sqrt_nn(t * (t + 2.0));
+        S = Pm.al * P;
+        beta = P * fm::rcp(t + 1.0);   // E = t + 1
+        sK = Pm.sk2dt * (P * fm::rsqrt(t + 1.0));
         sumac = 0.0;
         r = 100.0001;
         return true;
@@ -433,31 +443,32 @@ struct Fp {
     template <class Emit>
     __device__ __forceinline__ bool step(const StepParams &Pm, const double *z, const double *trig, const Emit &emit) {
         const double inv_r = fm::rcp(r);
-        const double sK = Pm.sk2dt * w;
-        const double dr = sK * fma(sK, inv_r, z[0]) + Pm.vdt;
-        const double Pn = fma(-(Pm.cp * P), inv_r, P);
-        sumac = fma(Pm.csum, inv_r, sumac);
+        const double t = fma(sK, inv_r, z[0]);
+        const double dr = fma(sK, t, Pm.vdt);
         const double rn = r + dr;
-        const double E2 = fma(Pn, Pn, 1.0);
+        const double Sn = fma(-(Pm.cp * S), inv_r, S);
+        sumac = fma(Pm.csum, inv_r, sumac);
+        const double E2 = fma(Sn, Sn, Pm.al2);
         const double q = fm::rsqrt4(E2);
         const double rb = rn - dr;
         if (fmin(rn, rb) < 1.0) {
             // a crossing of 1 AU needs one of rn, r - dr below 1:
             // (rn - 1) / ((rn - dr) - 1) < 0, without the division
             const double a = rn - 1.0, b = rb - 1.0;
-            if (beta > 0.01 && E2 < kE2Cross && ((a < 0.0 && b >= 0.0) || (a > 0.0 && b < 0.0)))
-                emit(t_inj, kT0 * fma(E2, q * q, -1.0), rn, 0.0, sumac);
+            if (beta > 0.01 && E2 < kE2Cross * Pm.al2 && ((a < 0.0 && b >= 0.0) || (a > 0.0 && b < 0.0)))
+                emit(t_inj, kinetic(Pm, Sn), rn, 0.0, sumac);
         }
         const bool stop = beta < 0.01;
-        w = Pn * q;
-        beta = w * q;
+        const double u = Sn * q;
+        sK = u * Pm.kap;
+        beta = u * q;
         // a reflected step (rn < 0.1) keeps r and P; rn < 100.0002 holds
         // then as well, so the loop test reads the unreflected rn.  Selects,
         // not a branch: a run's time is its longest trajectory, where a
         // branch's latency counts and the selects' issue slots do not.
         const bool refl = rn < 0.1;
         r = refl ? r : rn;
-        P = refl ? P : Pn;
+        S = refl ? S : Sn;
         return !stop && rn < 100.0002;
     }
     // Nothing happens while r stays between 1.01 and 100.00018 (the start of
@@ -471,19 +482,19 @@ struct Fp {
     __device__ __forceinline__ Watch watch() const { return {hi_of(r), hi_of(r)}; }
     __device__ __forceinline__ void fast_step(const StepParams &Pm, const double *z, const double *trig, Watch &W) {
         const double inv_r = fm::rcp(r);
-        const double sK = Pm.sk2dt * w;
-        P = fma(-(Pm.cp * P), inv_r, P);
+        S = fma(-(Pm.cp * S), inv_r, S);
         sumac = fma(Pm.csum, inv_r, sumac);
-        r = r + (sK * fma(sK, inv_r, z[0]) + Pm.vdt);
-        const double q = fm::rsqrt4(fma(P, P, 1.0));
-        w = P * q;
-        beta = w * q;
+        r = r + fma(sK, fma(sK, inv_r, z[0]), Pm.vdt);
+        const double q = fm::rsqrt4(fma(S, S, Pm.al2));
+        sK = S * q;
+        beta = sK * q;
         const uint32_t h = hi_of(r);
         W.hmax = max(W.hmax, h);
         W.hmin = min(W.hmin, h);
     }
-    __device__ __forceinline__ bool fast_ok(const Watch &W, const Fp &old) const {
-        return (int)(W.hmax < kRHi) & (int)(W.hmin > kRLo) & (int)(beta >= 0.01) & (int)(old.beta >= 0.01);
+    __device__ __forceinline__ bool fast_ok(const StepParams &Pm, const Watch &W, const Fp &old) const {
+        return (int)(W.hmax < kRHi) & (int)(W.hmin > kRLo) & (int)(beta >= 0.01) & (int)(old.beta >= 0.01) &
+               (int)(hi_of(S) - Pm.s_lo < kInfHi - Pm.s_lo);
     }
 };
 
@@ -532,7 +543,7 @@ struct Sp {
         theta = fmin(fabs(theta), fabs(2.0 * kPi - fabs(theta)));
         W.hmax = max(W.hmax, hi_of(r));
     }
-    __device__ __forceinline__ bool fast_ok(const Watch &W, const Sp &old) const { return W.hmax < kRHi; }
+    __device__ __forceinline__ bool fast_ok(const StepParams &, const Watch &W, const Sp &old) const { return W.hmax < kRHi; }
 
     // One Euler step of r, theta and T before the reflections and the exit.
     // Every fused multiply-add is written out (contraction is off): the 2D
@@ -633,7 +644,7 @@ struct Ge {
         theta = fmin(fabs(theta), fabs(2.0 * kPi - fabs(theta)));
         W.hmax = max(W.hmax, hi_of(r));
     }
-    __device__ __forceinline__ bool fast_ok(const Watch &W, const Ge &old) const { return W.hmax < kRHi; }
+    __device__ __forceinline__ bool fast_ok(const StepParams &, const Watch &W, const Ge &old) const { return W.hmax < kRHi; }
 
     // One Euler step of r, theta and T before the reflections and the exit
     // (fused multiply-adds written out, as in Sp).

@@ -48,6 +48,7 @@ struct StepParams {
     double sqdt;          // sqrt(dt)
     double two_dt;        // 2 dt
     double sk2dt;         // sqrt(2 K0 dt T0) (the 1D models carry momenta in units of T0)
+    double al, al2, kap;  // 1D: scale alpha of the momenta, its square, and kappa (see gs_device.hpp)
     double vdt;           // signed V dt as the model uses it (1D B-p: -V dt)
     double cp;            // (2/3) V dt with the same sign (momentum / energy loss)
     double csum;          // (4/3) V dt (1D F-p loss integral)
@@ -67,6 +68,8 @@ struct StepParams {
     double polthdt;       // pol_theta dt (2D SolarProp theta drift)
     double sq2dt;         // sqrt(2 dt)
     double delta0_rh;     // delta0 / rh
+    uint32_t s_lo;        // 1D fast steps: the high word that alpha P has to reach (0x7ff00000: none)
+    uint32_t pad_;
 };
 
 // Scheduling order of a run's particles (gs_launch_order, batches): offsets

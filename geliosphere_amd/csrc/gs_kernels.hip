@@ -433,7 +433,7 @@ __device__ void run_lanes(const DevParams *__restrict__ sims, uint32_t n_sims, c
                 m.fast_step(params(), z, bm.trig, watch);
             }
         }
-        const bool again = active & !((int)m.fast_ok(watch, old) & (int)(cap - steps >= (uint32_t)kCycleSteps));
+        const bool again = active & !((int)m.fast_ok(params(), watch, old) & (int)(cap - steps >= (uint32_t)kCycleSteps));
         if (__ballot(again)) {
             if (again) {
                 m = old;
@@ -550,7 +550,7 @@ batch_kernel(const DevParams *__restrict__ sims, uint32_t n_sims, const uint64_t
 //    repeated in full steps.  A lone wave pays about 130 cycles for a test (the
 //    compare, the branch, the first normals' LDS latency), so where a wave holds
 //    few particles, whose events are then rare, it looks less often: per step
-//    93 -> 66 ns in 1D at 64 lanes (8 cycles to a test; 4: 66 to 73), 606 -> 566 ns
+//    93 -> 62 ns in 1D at 64 lanes (8 cycles to a test; 4: 69), 606 -> 566 ns
 //    SolarProp, 760 -> 711 ns Geliosphere (4 cycles; 2: 580 and 740; 4 of its
 //    cycles are 50 KB of code, and more would leave the instruction cache).
 //    (About 1 in 5000 lane-cycles of a 1D B-p run has an event.)
@@ -667,9 +667,12 @@ __global__ void __launch_bounds__(kTailThreads) tail_kernel(const DevParams *__r
                 for (int s = 0; s < kSteps; ++s) {
                     double z[NPS];
                     for (int i = 0; i < NPS; ++i) z[i] = zc[NPS * s + i];
+                    // 1D: the normals of one cycle at a time in registers (all 32 at the
+                    // start took 36 more, and 64.7 ns a step instead of 62.2)
+                    if (NPS == 1 && s % kCycleSteps == kCycleSteps - 1) __builtin_amdgcn_sched_barrier(0);
                     m.fast_step(lp, z, bm.trig, watch);
                 }
-                const bool again = active & !((int)m.fast_ok(watch, old) & (int)(cap - steps >= (uint32_t)kSteps));
+                const bool again = active & !((int)m.fast_ok(lp, watch, old) & (int)(cap - steps >= (uint32_t)kSteps));
                 cycles += kAtOnce;
                 if (__ballot(again)) {
                     if (again) {

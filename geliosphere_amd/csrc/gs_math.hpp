@@ -92,14 +92,13 @@ __device__ __forceinline__ double sqrt_nn(double x) {
 }
 
 // x^(-1/4) for normal x > 0: the seed sqrt(rsq(x)) from two hardware
-// seeds, then the series of (1 - e)^(-1/4) to third order, e = 1 - x q^4,
-// written in f = e/4 = 1/4 - (x/4) q^4: q (1 + f + 5/2 f^2).  (Each fused
-// multiply-add then has at most one non-inline constant.)
+// seeds, then the series of (1 - e)^(-1/4) to third order, e = 1 - x q^4:
+// q (1 + e/4 + 5/32 e^2).
 __device__ __forceinline__ double rsqrt4(double x) {
     const double q = __builtin_amdgcn_sqrt(__builtin_amdgcn_rsq(x));
     const double q2 = q * q;
-    const double f = fma(-0.25 * x, q2 * q2, 0.25);
-    return fma(q, f * fma(2.5, f, 1.0), q);
+    const double e = fma(-x, q2 * q2, 1.0);
+    return fma(q, e * fma(0.15625, e, 0.25), q);
 }
 
 // sqrt(x), 0 for x <= 0.
