@@ -42,6 +42,10 @@ struct gs_surrogate {
     float mu[GS_SG_MAX_INPUTS], sd[GS_SG_MAX_INPUTS], lo[GS_SG_MAX_INPUTS], hi[GS_SG_MAX_INPUTS];
     // work buffers, grown on demand
     std::vector<DevBuf> bufs;
+    // host predictions: two halves of pinned memory and their events (pin_half)
+    char *pin = nullptr;
+    size_t pin_half = 0;
+    hipEvent_t pin_done[2] = {nullptr, nullptr};
     std::string err;
 };
 
@@ -396,6 +400,9 @@ void gs_surrogate_destroy(gs_surrogate *s) {
     if (s->stream) (void)hipStreamSynchronize(s->stream);
     for (DevBuf &b : s->bufs)
         if (b.p) (void)hipFree(b.p);
+    for (hipEvent_t e : s->pin_done)
+        if (e) (void)hipEventDestroy(e);
+    if (s->pin) (void)hipHostFree(s->pin);
     for (void *p : {(void *)s->P, (void *)s->G, (void *)s->Mo, (void *)s->Ve, (void *)s->Pb, (void *)s->PbT})
         if (p) (void)hipFree(p);
     if (s->stream) (void)hipStreamDestroy(s->stream);
@@ -661,6 +668,15 @@ gs_status gs_surrogate_gradients(gs_surrogate *s, const float *x, const float *y
     return GS_OK;
 }
 
+// Whether the inputs share no memory with the outputs.
+static bool apart(const gs_surrogate *s, const float *x, size_t n, const float *mean, const float *sd,
+                  const uint8_t *fallback) {
+    const uintptr_t b = (uintptr_t)x, e = b + n * s->cfg.n_inputs * sizeof(float);
+    auto from_x = [&](const void *p, size_t bytes) { return !p || (uintptr_t)p >= e || (uintptr_t)p + bytes <= b; };
+    const size_t out = n * s->cfg.n_outputs * sizeof(float);
+    return from_x(mean, out) && from_x(sd, out) && from_x(fallback, n);
+}
+
 // Whether kernels of this surrogate may read x in place: memory of its device,
 // apart from the outputs (the statistics read the inputs again after other
 // queries' results are written).
@@ -671,15 +687,94 @@ static bool reads_in_place(const gs_surrogate *s, const float *x, size_t n, cons
         (void)hipGetLastError();
         return false;
     }
-    if (a.type != hipMemoryTypeDevice || a.device != s->device) return false;
-    const uintptr_t b = (uintptr_t)x, e = b + n * s->cfg.n_inputs * sizeof(float);
-    auto apart = [&](const void *p, size_t bytes) { return !p || (uintptr_t)p >= e || (uintptr_t)p + bytes <= b; };
-    const size_t out = n * s->cfg.n_outputs * sizeof(float);
-    return apart(mean, out) && apart(sd, out) && apart(fallback, n);
+    return a.type == hipMemoryTypeDevice && a.device == s->device && apart(s, x, n, mean, sd, fallback);
 }
 
-// Both predict entry points: host buffers (copied through the surrogate's
-// stream) or device buffers (read and written in place).
+// Pinned memory for host predictions of `bytes` per half, at most kHostChunk rows
+// each; false where there is none.
+static bool pin_halves(gs_surrogate *s, size_t bytes) {
+    for (hipEvent_t &e : s->pin_done)
+        if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+            (void)hipGetLastError();
+            e = nullptr;
+            return false;
+        }
+    if (s->pin_half >= bytes) return true;
+    if (s->pin) (void)hipHostFree(s->pin);
+    s->pin = nullptr;
+    s->pin_half = 0;
+    if (hipHostMalloc((void **)&s->pin, 2 * bytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        s->pin = nullptr;
+        return false;
+    }
+    s->pin_half = bytes;
+    return true;
+}
+
+// The statistics of one block of rows whose inputs x and outputs the kernels can
+// reach.
+static gs_status infer_rows(gs_surrogate *s, const float *x, uint32_t rows, float *mean, float *sd, uint8_t *fallback) {
+    const int E = s->E, no = (int)s->cfg.n_outputs, ni = (int)s->cfg.n_inputs;
+    float *out;
+    SG_NEED(s, B_OUT, (size_t)E * rows * kPad, out);
+    gs_status st = forward_infer(s, x, (int)rows, out);
+    if (st != GS_OK) return st;
+    SG_TRY(s, sg_launch_query_stats(out, E, (int)rows, no, x, ni, s->cfg.std_outputs, s->cfg.std_limit, s->lo, s->hi,
+                                    mean, sd, fallback, s->stream));
+    return GS_OK;
+}
+
+// Host buffers through pinned memory that the kernels write themselves, in
+// blocks of kHostChunk rows: while the device works on one block the host copies
+// the results of the one before.  Pageable copies, four to a call with one in and
+// three out, were two thirds of a small call and took turns with the kernels in a
+// large one.  In us, before / now: 1 row 52 / 29, 512 82 / 33, 4,096 87 / 63, 20,011
+// 281 / 193 (four members, means and flags).
+// The inputs of up to kDirectRows rows are read from pinned memory too (each by
+// every member); of more, copied first (4,096 rows: 63 read, 70 copied; 20,011: 281, 251).
+constexpr uint32_t kHostChunk = 8192, kDirectRows = 4096;
+static gs_status predict_pinned(gs_surrogate *s, const float *x, uint32_t n, float *mean, float *sd, uint8_t *fallback) {
+    const size_t no = s->cfg.n_outputs, ni = s->cfg.n_inputs;
+    const size_t most = std::min(n, kHostChunk);
+    // a half: inputs, means, spreads, flags
+    auto half = [&](uint32_t c) { return s->pin + (c & 1) * s->pin_half; };
+    auto take = [&](uint32_t c) -> gs_status {   // results of block c, when they are there
+        const size_t r0 = (size_t)c * kHostChunk, rows = std::min<size_t>(n - r0, kHostChunk);
+        SG_TRY(s, hipEventSynchronize(s->pin_done[c & 1]));
+        const float *m = (const float *)half(c) + most * ni, *d = m + most * no;
+        const uint8_t *f = (const uint8_t *)(d + most * no);
+        if (mean) std::memcpy(mean + r0 * no, m, rows * no * sizeof(float));
+        if (sd) std::memcpy(sd + r0 * no, d, rows * no * sizeof(float));
+        if (fallback) std::memcpy(fallback + r0, f, rows);
+        return GS_OK;
+    };
+    const uint32_t blocks = (n + kHostChunk - 1) / kHostChunk;
+    gs_status st = GS_OK;
+    for (uint32_t c = 0; c < blocks && st == GS_OK; ++c) {
+        if (c >= 2 && (st = take(c - 2)) != GS_OK) break;
+        const size_t r0 = (size_t)c * kHostChunk;
+        const uint32_t rows = (uint32_t)std::min<size_t>(n - r0, kHostChunk);
+        float *px = (float *)half(c), *m = px + most * ni, *d = m + most * no;
+        std::memcpy(px, x + r0 * ni, rows * ni * sizeof(float));
+        const float *in = px;
+        if (rows > kDirectRows) {
+            float *xf;
+            SG_NEED(s, B_XF, (size_t)rows * ni, xf);
+            SG_TRY(s, hipMemcpyAsync(xf, px, rows * ni * sizeof(float), hipMemcpyHostToDevice, s->stream));
+            in = xf;
+        }
+        st = infer_rows(s, in, rows, mean ? m : nullptr, sd ? d : nullptr, fallback ? (uint8_t *)(d + most * no) : nullptr);
+        if (st == GS_OK) SG_TRY(s, hipEventRecord(s->pin_done[c & 1], s->stream));
+    }
+    if (st == GS_OK && blocks > 1) st = take(blocks - 2);
+    if (st == GS_OK) st = take(blocks - 1);
+    return st;
+}
+
+// Both predict entry points: host buffers (through pinned memory, or where
+// there is none, or the inputs share memory with the outputs, copied through the
+// surrogate's stream) or device buffers (read and written in place).
 static gs_status predict_rows(gs_surrogate *s, const float *x, uint32_t n, float *mean, float *sd,
                               uint8_t *fallback, bool on_device) {
     if (!s) return GS_ERR_INVALID_ARG;
@@ -687,13 +782,16 @@ static gs_status predict_rows(gs_surrogate *s, const float *x, uint32_t n, float
     if (n == 0) return GS_OK;
     SG_TRY(s, hipSetDevice(s->device));
     const uint32_t no = s->cfg.n_outputs, ni = s->cfg.n_inputs;
-    const int E = s->E;
+    // (results go out block by block before later inputs are read)
+    if (!on_device && apart(s, x, n, mean, sd, fallback) &&
+        pin_halves(s, (size_t)std::min(n, kHostChunk) * ((ni + 2 * no) * sizeof(float) + 1) + 64))
+        return predict_pinned(s, x, n, mean, sd, fallback);
     const uint32_t chunk = 65536;
     const bool in_place = on_device && reads_in_place(s, x, n, mean, sd, fallback);
     for (uint32_t r0 = 0; r0 < n; r0 += chunk) {
         const uint32_t rows = std::min(chunk, n - r0);
         const float *xr = x + (size_t)r0 * ni;
-        float *out, *dm = mean ? mean + (size_t)r0 * no : nullptr, *ds = sd ? sd + (size_t)r0 * no : nullptr;
+        float *dm = mean ? mean + (size_t)r0 * no : nullptr, *ds = sd ? sd + (size_t)r0 * no : nullptr;
         uint8_t *fl = fallback ? fallback + r0 : nullptr;
         if (!in_place) {
             float *xf;
@@ -707,11 +805,8 @@ static gs_status predict_rows(gs_surrogate *s, const float *x, uint32_t n, float
             if (sd) SG_NEED(s, B_SD, (size_t)rows * no, ds);
             if (fallback) SG_NEED(s, B_FLAGS, (size_t)rows, fl);
         }
-        SG_NEED(s, B_OUT, (size_t)E * rows * kPad, out);
-        gs_status st = forward_infer(s, xr, (int)rows, out);
+        const gs_status st = infer_rows(s, xr, rows, dm, ds, fl);
         if (st != GS_OK) return st;
-        SG_TRY(s, sg_launch_query_stats(out, E, (int)rows, (int)no, xr, (int)ni, s->cfg.std_outputs, s->cfg.std_limit,
-                                        s->lo, s->hi, dm, ds, fl, s->stream));
         if (!on_device) {
             const size_t bytes = (size_t)rows * no * sizeof(float);
             if (fallback) SG_TRY(s, hipMemcpyAsync(fallback + r0, fl, rows, hipMemcpyDeviceToHost, s->stream));

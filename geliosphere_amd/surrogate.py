@@ -169,9 +169,9 @@ class Surrogate:
         which halves the bytes copied back."""
         x, px = _f32(x)
         n = x.shape[0]
-        mean = np.zeros((n, self.cfg.n_outputs), dtype=np.float32)
-        sd = np.zeros_like(mean) if want_sd else None
-        fb = np.zeros(n, dtype=np.uint8)
+        mean = np.empty((n, self.cfg.n_outputs), dtype=np.float32)   # (every element is written)
+        sd = np.empty_like(mean) if want_sd else None
+        fb = np.empty(n, dtype=np.uint8)
         psd = sd.ctypes.data_as(ctypes.POINTER(ctypes.c_float)) if want_sd else None
         self._check(lib().gs_surrogate_predict(self._h, px, n, mean.ctypes.data_as(ctypes.POINTER(ctypes.c_float)),
                                                psd, fb.ctypes.data_as(ctypes.POINTER(ctypes.c_uint8))), "predict")

@@ -59,3 +59,29 @@ def test_device_inputs_may_share_memory_with_the_outputs():
     sd_d = DeviceArray((300, 30), np.float32)
     m_d, _, fb_d = s.predict_device(view, b, sd_d)
     assert np.array_equal(m_d.to_host(), mean) and np.array_equal(sd_d.to_host(), sd) and np.array_equal(fb_d.to_host(), fb)
+
+
+@pytest.mark.parametrize("n", (1, 4096, 4097, 8192, 8193, 16_385, 24_577))
+def test_host_blocks_equal_device_call(n):
+    """Host calls go in blocks of 8,192 rows through two halves of pinned memory
+    (inputs read there up to 4,096 rows of a block, copied beyond); outputs that
+    share memory with the inputs take the copies."""
+    import ctypes
+
+    from geliosphere_amd.devmem import DeviceArray
+    from geliosphere_amd.surrogate import lib
+    s = make(4, 4, 8)
+    x = np.random.default_rng(n).normal(0, 1, (n, 8)).astype(np.float32)
+    sd_d = DeviceArray((n, 30), np.float32)
+    m_d, _, f_d = s.predict_device(DeviceArray.from_host(x), None, sd_d)
+    want = m_d.to_host(), sd_d.to_host(), f_d.to_host()
+    for a, b in zip(s.predict(x), want):
+        assert np.array_equal(a, b)
+    m, none, f = s.predict(x, want_sd=False)
+    assert none is None and np.array_equal(m, want[0]) and np.array_equal(f, want[2])
+    shared = np.zeros((n, 30), np.float32)
+    shared.reshape(-1)[-x.size:] = x.reshape(-1)
+    pf = ctypes.POINTER(ctypes.c_float)
+    px = ctypes.cast(shared.ctypes.data + 4 * (shared.size - x.size), pf)
+    assert lib().gs_surrogate_predict(s._h, px, n, shared.ctypes.data_as(pf), None, None) == 0
+    assert np.array_equal(shared, want[0])
