@@ -160,14 +160,14 @@ DevParams derive(const gs_params &p) {
     d.sqdt = std::sqrt(p.dt);
     d.two_dt = 2.0 * p.dt;
     d.sk2dt = std::sqrt(d.two_dt * p.K0 * gs::kT0);   // the 1D models' momenta are in units of T0
-    // the scale of the 1D momenta: 2 K0 dt T0, unless its square leaves the
-    // middle of the double range
-    const double al = d.two_dt * p.K0 * gs::kT0;
-    const bool scaled = al > 1e-60 && al < 1e60;
+    // the scale of the 1D momenta: 2 K0 dt T0, unless alpha^2 E^2 leaves 1e-28 ..
+    // 1e30 (SolarProp's bins end below 1,300 GeV)
+    const double al = d.two_dt * p.K0 * gs::kT0, Emax = std::max(std::max(p.T_min, p.T_max), 2e3) / gs::kT0 + 1.0;
+    const bool scaled = al > 1e-14 && al * Emax < 1e15;
     d.al = scaled ? al : 1.0;
     d.al2 = d.al * d.al;
     d.kap = scaled ? 1.0 : d.sk2dt;
-    d.s_lo = !scaled ? 0x7ff00000u : p.model == GS_MODEL_1D_BP ? hi_word(d.al * 0.0101) + 1 : 1u;
+    d.s_lo = !scaled ? hi_word(1e17) : p.model == GS_MODEL_1D_BP ? hi_word(d.al * 0.0101) + 1 : 1u;
     const double vs = p.model == GS_MODEL_1D_BP ? -p.V : p.V;
     d.vdt = vs * p.dt;
     d.cp = (2.0 / 3.0) * vs * p.dt;

@@ -305,13 +305,19 @@ __device__ __forceinline__ uint32_t hi_of(double x) { return (uint32_t)(fm::doub
 // E^2 and q = E2^(-1/4) from one rsqrt4,
 //   sK = S q    (alpha P / sqrt(alpha E)),    beta = S q^2    (alpha P / (alpha E)),
 // no factor left to multiply.  16 FP64 operations and 3 transcendental seeds per
-// B-p step (19 and 3 with P itself: 561 ms for 2e7 particles, now 538).  A
-// simulation whose alpha^2 is far from 1 (K0 dt beyond anything physical) has
-// alpha = 1 instead and sK = kappa S q (Pm.kap = sqrt(2 K0 dt T0); 1 otherwise)
+// B-p step (19 and 3 with P itself: 561 ms for 2e7 particles, then 538, with
+// single-precision seeds of q 524).  A simulation that may leave the middle of the
+// single-precision range (K0 dt or energies beyond anything physical) has alpha = 1
+// instead and sK = kappa S q (Pm.kap = sqrt(2 K0 dt T0); 1 otherwise)
 // and takes full steps only (Pm.s_lo).
 constexpr double kInvT0 = 1.0 / kT0;
-constexpr uint32_t kInfHi = 0x7ff00000u;
 
+// E2^(-1/4) in a full step; fast steps stand where S < 1e17 and alpha > 1e-14,
+// so that the single-precision seeds serve.
+constexpr uint32_t kSHi = hi_word(1e17);
+__device__ __forceinline__ double root4(double E2) {
+    return E2 > 1e-30 && E2 < 1e36 ? fm::rsqrt4_mid(E2) : fm::rsqrt4(E2);
+}
 // The kinetic energy T0 (E - 1) = T0 P^2 / (E + 1) at S.
 __device__ __forceinline__ double kinetic(const StepParams &Pm, double S) {
     const double P = S * fm::rcp(Pm.al), P2 = P * P;
@@ -349,7 +355,7 @@ struct Bp {
         const double dr = fma(sK, t, Pm.vdt);
         const double rn = r + dr;
         const double E2 = fma(Sn, Sn, Pm.al2);
-        const double q = fm::rsqrt4(E2);
+        const double q = root4(E2);
         const double u = Sn * q;
         const double sKn = u * Pm.kap;
         const double bn = u * q;
@@ -384,7 +390,7 @@ struct Bp {
     // Nothing happens while 0.31 < r < 99.99 after each step and beta stays
     // above 0.01: P grows from step to step (V > 0, r > 0), so it is enough that
     // the first S of the cycle lies above 0.0101 alpha (beta = 0.0100995; Pm.s_lo
-    // holds its high word and one), and the last is neither below that nor NaN.
+    // holds its high word and one), and the last is neither below that nor 1e17 nor NaN.
     struct Watch { uint32_t hmax, hmin; };
     static constexpr uint32_t kRLo = hi_word(0.31), kRHi = hi_word(99.99);
     __device__ __forceinline__ Watch watch() const { return {0u, 0xffffffffu}; }
@@ -392,15 +398,15 @@ struct Bp {
         const double inv_r = fm::rcp(r);
         S = fma(-(Pm.cp * S), inv_r, S);
         r = r + fma(sK, fma(sK, inv_r, z[0]), Pm.vdt);   // (not r + V dt first: it rounds the same way in every step)
-        sK = S * fm::rsqrt4(fma(S, S, Pm.al2));
+        sK = S * fm::rsqrt4_mid(fma(S, S, Pm.al2));
         const uint32_t h = hi_of(r);
         W.hmax = max(W.hmax, h);
         W.hmin = min(W.hmin, h);
     }
     __device__ __forceinline__ bool fast_ok(const StepParams &Pm, const Watch &W, const Bp &old) const {
         // (int: no short circuits, each of which is a branch)
-        return (int)(W.hmax < kRHi) & (int)(W.hmin > kRLo) & (int)(hi_of(old.S) - Pm.s_lo < kInfHi - Pm.s_lo) &
-               (int)(hi_of(S) - Pm.s_lo < kInfHi - Pm.s_lo);
+        return (int)(W.hmax < kRHi) & (int)(W.hmin > kRLo) & (int)(hi_of(old.S) - Pm.s_lo < kSHi - Pm.s_lo) &
+               (int)(hi_of(S) - Pm.s_lo < kSHi - Pm.s_lo);
     }
 };
 
@@ -449,7 +455,7 @@ struct Fp {
         const double Sn = fma(-(Pm.cp * S), inv_r, S);
         sumac = fma(Pm.csum, inv_r, sumac);
         const double E2 = fma(Sn, Sn, Pm.al2);
-        const double q = fm::rsqrt4(E2);
+        const double q = root4(E2);
         const double rb = rn - dr;
         if (fmin(rn, rb) < 1.0) {
             // a crossing of 1 AU needs one of rn, r - dr below 1:
@@ -485,7 +491,7 @@ struct Fp {
         S = fma(-(Pm.cp * S), inv_r, S);
         sumac = fma(Pm.csum, inv_r, sumac);
         r = r + fma(sK, fma(sK, inv_r, z[0]), Pm.vdt);
-        const double q = fm::rsqrt4(fma(S, S, Pm.al2));
+        const double q = fm::rsqrt4_mid(fma(S, S, Pm.al2));
         sK = S * q;
         beta = sK * q;
         const uint32_t h = hi_of(r);
@@ -494,7 +500,7 @@ struct Fp {
     }
     __device__ __forceinline__ bool fast_ok(const StepParams &Pm, const Watch &W, const Fp &old) const {
         return (int)(W.hmax < kRHi) & (int)(W.hmin > kRLo) & (int)(beta >= 0.01) & (int)(old.beta >= 0.01) &
-               (int)(hi_of(S) - Pm.s_lo < kInfHi - Pm.s_lo);
+               (int)(hi_of(S) - Pm.s_lo < kSHi - Pm.s_lo);
     }
 };
 

@@ -68,7 +68,7 @@ struct StepParams {
     double polthdt;       // pol_theta dt (2D SolarProp theta drift)
     double sq2dt;         // sqrt(2 dt)
     double delta0_rh;     // delta0 / rh
-    uint32_t s_lo;        // 1D fast steps: the high word that alpha P has to reach (0x7ff00000: none)
+    uint32_t s_lo;        // 1D fast steps: the high word that alpha P has to reach (that of 1e17: none)
     uint32_t pad_;
 };
 

@@ -9,8 +9,9 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("model", (abi.MODEL_1D_BP, abi.MODEL_1D_FP))
-# ordinary, and 2 K0 dt T0 beyond 1e-60 and 1e60
-@pytest.mark.parametrize("k0,steps", ((5e22, 0), (5e-60, 3000), (5e110, 3000)))
+# ordinary; 2 K0 dt T0 near 1e-13 and 1e10 (scaled, momenta growing out of the range
+# of the single-precision seeds in the first), and beyond both ends
+@pytest.mark.parametrize("k0,steps", ((5e22, 0), (5e10, 30_000), (5e32, 3000), (5e-60, 3000), (5e110, 3000)))
 def test_scales_against_the_oracle(engine, oracle, model, k0, steps):
     n = 1500 if model == abi.MODEL_1D_BP else 40_000
     p = abi.make_params(model, N=n, seed=19, K0_cm2s=k0, max_steps=steps, T_min=0.05, r_inj=70.0)
