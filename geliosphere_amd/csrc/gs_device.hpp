@@ -394,6 +394,7 @@ struct Bp {
     struct Watch { uint32_t hmax, hmin; };
     static constexpr uint32_t kRLo = hi_word(0.31), kRHi = hi_word(99.99);
     __device__ __forceinline__ Watch watch() const { return {0u, 0xffffffffu}; }
+    template <int kLanes = 1>
     __device__ __forceinline__ void fast_step(const StepParams &Pm, const double *z, const double *trig, Watch &W) {
         const double inv_r = fm::rcp(r);
         S = fma(-(Pm.cp * S), inv_r, S);
@@ -486,6 +487,7 @@ struct Fp {
     struct Watch { uint32_t hmax, hmin; };
     static constexpr uint32_t kRLo = hi_word(1.01), kRHi = hi_word(100.0002);
     __device__ __forceinline__ Watch watch() const { return {hi_of(r), hi_of(r)}; }
+    template <int kLanes = 1>
     __device__ __forceinline__ void fast_step(const StepParams &Pm, const double *z, const double *trig, Watch &W) {
         const double inv_r = fm::rcp(r);
         S = fma(-(Pm.cp * S), inv_r, S);
@@ -524,7 +526,7 @@ struct Sp {
     }
     template <class Emit>
     __device__ __forceinline__ bool step(const StepParams &Pm, const double *z, const double *trig, const Emit &emit) {
-        advance(Pm, z, trig);
+        advance<1>(Pm, z, trig);
         theta = fabs(theta);   // theta < 0 -> |theta| (also takes -0 to +0)
         if (theta > kPi) {
             asm volatile("");   // emits nothing; a pole crossing is rare: no selects on the common path
@@ -544,8 +546,9 @@ struct Sp {
     struct Watch { uint32_t hmax; };
     static constexpr uint32_t kRHi = hi_word(100.0);
     __device__ __forceinline__ Watch watch() const { return {0u}; }
+    template <int kLanes = 1>
     __device__ __forceinline__ void fast_step(const StepParams &Pm, const double *z, const double *trig, Watch &W) {
-        advance(Pm, z, trig);
+        advance<kLanes>(Pm, z, trig);
         theta = fmin(fabs(theta), fabs(2.0 * kPi - fabs(theta)));
         W.hmax = max(W.hmax, hi_of(r));
     }
@@ -555,20 +558,21 @@ struct Sp {
     // Every fused multiply-add is written out (contraction is off): the 2D
     // models amplify a last-bit difference into another trajectory, so the
     // rounding must not depend on what surrounds the inlined step.
+    template <int kLanes>
     __device__ __forceinline__ void advance(const StepParams &Pm, const double *z, const double *trig) {
         double s, c;
         fm::sincosd(theta, trig, s, c);
         const double Tp = T + 2.0 * kT0;
-        const double Rig = fm::sqrt_nn(T * Tp);
         const double r2 = r * r;
         const double gamma = r * Pm.omega_v * s;
         const double opg = fma(gamma, gamma, 1.0);   // 1 + gamma^2
         const double tpg = fma(gamma, gamma, 2.0);   // 2 + gamma^2
         const double tmg = 2.0 - gamma * gamma;      // 2 - gamma^2
+        double Rig, sq;
+        fm::DevOps::roots<kLanes>(T * Tp, opg, Rig, sq);
         double inv_E, inv_r, inv_opg, inv_s;
         fm::rcp4(T + kT0, r, opg, s, inv_E, inv_r, inv_opg, inv_s);
         const double beta = Rig * inv_E;
-        const double sq = fm::sqrt_nn(opg);
         const double inv_sq = sq * inv_opg;
         const double inv_opg15 = inv_opg * inv_sq;
         const double inv_opg25 = inv_opg * inv_opg15;
@@ -585,15 +589,15 @@ struct Sp {
         // since 5/(3 3.4) = (5/3.4)/3 = C.
         const double krc = kbc * Rig * r;
         const double dKrr = krc * fma(Pm.ratio * tpg, inv_opg15, (1.0 - Pm.ratio) * tmg * inv_opg25);
-        const double sKrr = fm::sqrt_nn(Pm.two_dt * Krr);
-        const double sKtt = fm::sqrt_nn(Pm.two_dt * Kper);
+        // drifts: sheet angle alphaM + 2 Larmor pi / (180 r), Larmor = (0.0225 / A) P r^2 / sq
+        const double sy = fm::sind(fma(Rig * r * inv_sq, (0.0225 / kA) * (kPi / 90.0), Pm.tilt), trig);
+        double sKrr, sKtt, Y;
+        fm::DevOps::roots<kLanes>(Pm.two_dt * Krr, Pm.two_dt * Kper, fm::sheet_arg(sy), sKrr, sKtt, Y);
         double dr = fma(fma(2.0 * Krr, inv_r, dKrr) - Pm.V, Pm.dt, z[0] * sKrr);
         const double cs = c * inv_s;
         double dth = fma(Kper * cs * inv_r * inv_r * inv_opg, Pm.dt, z[1] * sKtt * inv_r);
-        // drifts: sheet angle alphaM + 2 Larmor pi / (180 r), Larmor = (0.0225 / A) P r^2 / sq
-        const double sy = fm::sind(fma(Rig * r * inv_sq, (0.0225 / kA) * (kPi / 90.0), Pm.tilt), trig);
         double f, g;
-        fm::sheet_drift<fm::DevOps>(sy, fma(theta, -(2.0 / kPi), 1.0), trig + fm::kBmTrigWords, f, g);
+        fm::sheet_drift<fm::DevOps, kLanes>(sy, Y, fma(theta, -(2.0 / kPi), 1.0), trig + fm::kBmTrigWords, f, g);
         const double rbg = Rig * beta * r * gamma * inv_opg;
         const double dc = rbg * ((kKonvF * (2.0 / (3.0 * kA))) * f) * inv_opg;
         // (DriftR + DriftSheetR) dt, with fprime = -(2/pi) g
@@ -627,7 +631,7 @@ struct Ge {
     }
     template <class Emit>
     __device__ __forceinline__ bool step(const StepParams &Pm, const double *z, const double *trig, const Emit &emit) {
-        advance(Pm, z, trig);
+        advance<1>(Pm, z, trig);
         theta = fabs(theta);   // theta < 0 -> |theta| (also takes -0 to +0)
         if (theta > kPi) {
             asm volatile("");   // emits nothing; a pole crossing is rare: no selects on the common path
@@ -645,8 +649,9 @@ struct Ge {
     struct Watch { uint32_t hmax; };
     static constexpr uint32_t kRHi = hi_word(100.0);
     __device__ __forceinline__ Watch watch() const { return {0u}; }
+    template <int kLanes = 1>
     __device__ __forceinline__ void fast_step(const StepParams &Pm, const double *z, const double *trig, Watch &W) {
-        advance(Pm, z, trig);
+        advance<kLanes>(Pm, z, trig);
         theta = fmin(fabs(theta), fabs(2.0 * kPi - fabs(theta)));
         W.hmax = max(W.hmax, hi_of(r));
     }
@@ -654,6 +659,7 @@ struct Ge {
 
     // One Euler step of r, theta and T before the reflections and the exit
     // (fused multiply-adds written out, as in Sp).
+    template <int kLanes>
     __device__ __forceinline__ void advance(const StepParams &Pm, const double *z, const double *trig) {
         // The reference's factors are regrouped so that each per-simulation
         // product is formed once on the host (StepParams ge_*): with
@@ -666,7 +672,6 @@ struct Ge {
         double s, c;
         fm::sincosd(theta, trig, s, c);
         const double Tp = T + 2.0 * kT0;
-        const double Rig = fm::sqrt_nn(T * Tp);
         const double r2 = r * r;
         double inv_E, inv_r, inv_s, inv_E_r;
         {
@@ -678,7 +683,6 @@ struct Ge {
             inv_E = r * inv_E_r;
             inv_r = (T + kT0) * inv_E_r;
         }
-        const double beta = Rig * inv_E;
         const bool polar = (theta < Pm.th_lo) || (theta > Pm.th_hi);
         const bool band = (theta > Pm.th_lo) && (theta < Pm.th_hi);
         double deltarh = Pm.delta0_rh * inv_s;   // delta / rh
@@ -693,7 +697,9 @@ struct Ge {
         const double h = fma(r2, deltarh2, g2);       // Cb - 1
         const double Cb = 1.0 + h;
         const double inv_Cb = fm::rcp(Cb);
-        const double sqCb = fm::sqrt_nn(Cb);
+        double Rig, sqCb;
+        fm::DevOps::roots<kLanes>(T * Tp, Cb, Rig, sqCb);
+        const double beta = Rig * inv_E;
         const double inv_sqCb = sqCb * inv_Cb;
         const double inv_Cb15 = inv_Cb * inv_sqCb;
         const double inv_Cb25 = inv_Cb * inv_Cb15;
@@ -708,8 +714,11 @@ struct Ge {
         // 1/Ktt and sqrt(2 Ktt dt) from one rsqrt
         const double rK = fm::rsqrt(Ktt);
         const double inv_Ktt = rK * rK;
-        // times sqrt(dt); a rounding-negative argument counts as 0
-        const double B11 = fm::sqrt_nn(fmax(Pm.two_dt * fma(Krr, Ktt, -(Krt * Krt)) * inv_Ktt, 0.0));
+        // sheet angle alphaM + 2 Larmor pi / (180 r), Larmor = (0.0225 / A) P r^2 / sqrt(Cb)
+        const double sy = fm::sind(fma(Rig * r * inv_sqCb, (0.0225 / kA) * (kPi / 90.0), Pm.tilt), trig);
+        // B11 times sqrt(dt); a rounding-negative argument counts as 0
+        double B11, Y;
+        fm::DevOps::roots<kLanes>(fmax(Pm.two_dt * fma(Krr, Ktt, -(Krt * Krt)) * inv_Ktt, 0.0), fm::sheet_arg(sy), B11, Y);
         const double B12 = (Pm.sq2dt * Krt) * rK;
         const double B22 = (Pm.sq2dt * Ktt) * rK * inv_r;
         const double kbrc = kbc * Rig;                // C K0 beta P
@@ -741,11 +750,9 @@ struct Ge {
         }
         double dr = fma(fma(fma(Krt, csi, fma(2.0, Krr, dKrtt)), inv_r, dKrr) - Pm.V, Pm.dt, fma(z[0], B11, z[1] * B12));
         double dth = fma(fma(fma(fma(Ktt, csi, dKtt), inv_r, 2.0 * Krt), inv_r, dKrtr), Pm.dt, z[2] * B22);
-        // drifts (Kappl 2016 Eq. 26, 32-37 with Cb in place of 1 + gamma^2); sheet
-        // angle alphaM + 2 Larmor pi / (180 r), Larmor = (0.0225 / A) P r^2 / sqrt(Cb)
-        const double sy = fm::sind(fma(Rig * r * inv_sqCb, (0.0225 / kA) * (kPi / 90.0), Pm.tilt), trig);
+        // drifts (Kappl 2016 Eq. 26, 32-37 with Cb in place of 1 + gamma^2)
         double f, g;
-        fm::sheet_drift<fm::DevOps>(sy, fma(theta, -(2.0 / kPi), 1.0), trig + fm::kBmTrigWords, f, g);
+        fm::sheet_drift<fm::DevOps, kLanes>(sy, Y, fma(theta, -(2.0 / kPi), 1.0), trig + fm::kBmTrigWords, f, g);
         const double rbg = Rig * beta * r * gamma * inv_Cb;
         const double dc = rbg * ((kKonvF * (2.0 / (3.0 * kA))) * f) * inv_Cb;
         // (DriftR + DriftSheetR) dt, with fprime = -(2/pi) g

@@ -554,6 +554,12 @@ batch_kernel(const DevParams *__restrict__ sims, uint32_t n_sims, const uint64_t
 //    SolarProp, 760 -> 711 ns Geliosphere (4 cycles; 2: 580 and 740; 4 of its
 //    cycles are 50 KB of code, and more would leave the instruction cache).
 //    (About 1 in 5000 lane-cycles of a 1D B-p run has an event.)
+//  - a 2D step has parts that are the same instructions on other numbers: two
+//    arctangents, and roots two and three at a time.  Neighbouring lanes of a
+//    particle form one of them each and exchange the results by quad_perm moves
+//    (DevOps::lane_of: 11 cycles for a double, against 190 for an arctangent and
+//    52 for a root): the arctangents took SolarProp from 566 to 498 ns a step and
+//    Geliosphere from 719 to 652, the roots to 480 and 637.
 // G is fixed within a launch.  After `budget` cycles the live particles are
 // handed to the next launch, which spreads the fewer particles over the same
 // lanes (in a batch: its model group's share of the dies); a launch that has 64
@@ -656,8 +662,9 @@ __global__ void __launch_bounds__(kTailThreads) tail_kernel(const DevParams *__r
         __builtin_amdgcn_wave_barrier();
         blk += (uint32_t)(NPS * g);
         // ---- g cycles, kAtOnce to a test (both powers of two, kAtOnce <= g)
-        auto run_cycles = [&](auto at_once) {
+        auto run_cycles = [&](auto at_once, auto lanes) {
             constexpr int kAtOnce = decltype(at_once)::value, kSteps = kAtOnce * kCycleSteps;
+            constexpr int kLanes = decltype(lanes)::value;   // that many lanes share a particle's 2D steps
 #pragma unroll 1
             for (int c = 0; c < g; c += kAtOnce) {
                 const double *zc = my + c * NPS * kCycleSteps;
@@ -670,7 +677,7 @@ __global__ void __launch_bounds__(kTailThreads) tail_kernel(const DevParams *__r
                     // 1D: the normals of one cycle at a time in registers (all 32 at the
                     // start took 36 more, and 64.7 ns a step instead of 62.2)
                     if (NPS == 1 && s % kCycleSteps == kCycleSteps - 1) __builtin_amdgcn_sched_barrier(0);
-                    m.fast_step(lp, z, bm.trig, watch);
+                    m.template fast_step<kLanes>(lp, z, bm.trig, watch);
                 }
                 const bool again = active & !((int)m.fast_ok(lp, watch, old) & (int)(cap - steps >= (uint32_t)kSteps));
                 cycles += kAtOnce;
@@ -695,10 +702,17 @@ __global__ void __launch_bounds__(kTailThreads) tail_kernel(const DevParams *__r
                 steps += (uint32_t)kSteps;
             }
         };
-        if (NPS == 1 && g == kWave) run_cycles(std::integral_constant<int, 8>());
-        else if (g >= 16) run_cycles(std::integral_constant<int, 4>());
-        else if (g >= 8) run_cycles(std::integral_constant<int, 2>());
-        else run_cycles(std::integral_constant<int, 1>());
+        constexpr std::integral_constant<int, 8> k8;
+        constexpr std::integral_constant<int, 4> k4;
+        constexpr std::integral_constant<int, 2> k2;
+        constexpr std::integral_constant<int, 1> k1;
+        constexpr bool k2D = NPS != 1;
+        constexpr std::integral_constant<int, k2D ? 4 : 1> quad;
+        if (!k2D && g == kWave) run_cycles(k8, quad);
+        else if (g >= 16) run_cycles(k4, quad);
+        else if (g >= 8) run_cycles(k2, quad);
+        else if (k2D && g >= 2) run_cycles(k1, k2);
+        else run_cycles(k1, k1);
     }
     const uint64_t live = __ballot(active && sub == 0);
     if (live) {   // the budget is spent: hand the live particles on

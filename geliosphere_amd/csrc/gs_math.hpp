@@ -121,6 +121,40 @@ struct DevOps {
     __device__ static double fmac(double a, double b, double c) { return fma(a, b, c); }
     __device__ static double inv(double v) { return rcp(v); }
     __device__ static double root(double v) { return sqrt_nn(v); }
+    // Lane i's v of each kLanes (2 or 4) neighbouring lanes (quad_perm: all lanes
+    // take part).
+    template <int kLanes, int i>
+    __device__ static double lane_of(double v) {
+        constexpr int ctrl = kLanes == 2 ? 5 * i + 0xA0 + 0x50 * i : 0x55 * i;
+        const uint64_t b = double_to_bits(v);
+        return join(__builtin_amdgcn_mov_dpp((int)(uint32_t)b, ctrl, 0xf, 0xf, true),
+                    __builtin_amdgcn_mov_dpp((int)(uint32_t)(b >> 32), ctrl, 0xf, 0xf, true));
+    }
+    // Two and three roots, by one lane of kLanes each where lanes share arguments.
+    template <int kLanes>
+    __device__ static void roots(double x0, double x1, double &r0, double &r1) {
+        if constexpr (kLanes > 1) {
+            const double r = sqrt_nn((threadIdx.x & 1) != 0 ? x1 : x0);
+            r0 = lane_of<2, 0>(r);
+            r1 = lane_of<2, 1>(r);
+        } else {
+            r0 = sqrt_nn(x0);
+            r1 = sqrt_nn(x1);
+        }
+    }
+    template <int kLanes>
+    __device__ static void roots(double x0, double x1, double x2, double &r0, double &r1, double &r2) {
+        if constexpr (kLanes == 4) {
+            const double r = sqrt_nn((threadIdx.x & 2) != 0 ? x2 : (threadIdx.x & 1) != 0 ? x1 : x0);
+            r0 = lane_of<4, 0>(r);
+            r1 = lane_of<4, 1>(r);
+            r2 = lane_of<4, 2>(r);
+        } else {
+            roots<kLanes>(x0, x1, r0, r1);
+            r2 = sqrt_nn(x2);
+        }
+    }
+    __device__ static double join(int lo, int hi) { return bits_to_double((uint64_t)(uint32_t)hi << 32 | (uint32_t)lo); }
 };
 struct HostOps {
     static double fma3(double a, double b, double c) { return std::fma(a, b, c); }
@@ -269,21 +303,40 @@ __host__ __device__ inline double atan_frac(double n, double d, const double *re
 // quotients (x, tan, arg, 1/alphaH, 1/(1 + arg^2)) is formed on its own: two
 // atan_frac reciprocals and one of alphaH (X^2 + k^2 Y^2) for both results.
 // At sy = 0 this gives the limits f = +-(pi/2)/alphaH, g = 0.
-template <class Ops>
-__host__ __device__ inline void sheet_drift(double sy, double k, const double *red, double &f, double &g) {
+//
+// Y is the root of sheet_arg(sy).  kLanes > 1 (device): that many neighbouring
+// lanes hold the same arguments, and the two arctangents, the same instructions on
+// other numbers, are formed by one lane of a pair each.
+__host__ __device__ inline double sheet_arg(double sy) {
     constexpr double kPiD = 3.141592653589793;
+    return kPiD * (kPiD - 2.0 * sy);
+}
+template <class Ops, int kLanes = 1>
+__host__ __device__ inline void sheet_drift(double sy, double Y, double k, const double *red, double &f, double &g) {
     const double X = sy, ax = fabs(sy);
-    const double Y = Ops::root(kPiD * (kPiD - 2.0 * sy));
-    const double a0 = atan_frac<Ops>(ax, Y, red);
-    const double aH = kPi2Hi - (copysign(a0, X) - kPi2Lo);   // a0 >= 0 takes X's sign
     const double kY = fabs(k) * Y;
+    double a0, a1;
+    if constexpr (kLanes > 1) {
+        const bool odd = (threadIdx.x & 1) != 0;
+        const double a = atan_frac<Ops>(odd ? fmin(ax, kY) : ax, odd ? fmax(ax, kY) : Y, red);
+        a0 = Ops::template lane_of<2, 0>(a);
+        a1 = Ops::template lane_of<2, 1>(a);
+    } else {
+        a0 = atan_frac<Ops>(ax, Y, red);
+        a1 = atan_frac<Ops>(fmin(ax, kY), fmax(ax, kY), red);   // the smaller over the larger
+    }
+    const double aH = kPi2Hi - (copysign(a0, X) - kPi2Lo);   // a0 >= 0 takes X's sign
     const bool swap = kY > ax;
-    const double a1 = atan_frac<Ops>(fmin(ax, kY), fmax(ax, kY), red);   // the smaller over the larger
     const double at = swap ? kPi2Hi - (a1 - kPi2Lo) : a1;     // atan(|k| Y / |X|)
     const double D2 = Ops::fma3(X, X, kY * kY);
     const double R = Ops::inv(aH * D2);
     f = ((k < 0.0) != (X < 0.0) ? -at : at) * (D2 * R);      // atan(arg) / alphaH
     g = (X * Y) * R;                                          // (X Y / D2) / alphaH
+}
+
+template <class Ops>
+__host__ __device__ inline void sheet_drift(double sy, double k, const double *red, double &f, double &g) {
+    sheet_drift<Ops>(sy, Ops::root(sheet_arg(sy)), k, red, f, g);
 }
 
 // ------------------------------------------------------------ Box-Muller

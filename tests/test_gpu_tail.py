@@ -44,7 +44,7 @@ def test_step_cap_inside_a_cycle(engine, model, max_steps):
 
 
 @pytest.mark.parametrize("model", MODELS)
-@pytest.mark.parametrize("n", (500, 3000, 6000, 20_000))   # 64, 16, 8 and 2 lanes to a particle
+@pytest.mark.parametrize("n", (500, 3000, 6000, 10_000, 20_000))   # 64, 16, 8, 4 and 2 lanes to a particle
 @pytest.mark.parametrize("max_steps", (15, 33, 64, 1031))
 def test_step_cap_between_two_tests(engine, model, n, max_steps):
     """Caps inside and at the ends of the cycles that are tested together."""
