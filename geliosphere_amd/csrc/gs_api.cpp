@@ -191,10 +191,26 @@ DevParams derive(const gs_params &p) {
     return d;
 }
 
+// Room for n elements.  Where the device has none, the ordered copy of an earlier
+// run's records is given back first (a run can do without it: ordered_records).
+template <class T>
+hipError_t device_alloc(gs_ctx *ctx, T *&p, uint64_t n) {
+    hipError_t e = hipMalloc((void **)&p, n * sizeof(T));
+    if (e == hipErrorOutOfMemory && ctx->d_recs) {
+        (void)hipGetLastError();
+        (void)hipFree(ctx->d_recs);
+        ctx->d_recs = nullptr;
+        ctx->cap_recs = 0;
+        e = hipMalloc((void **)&p, n * sizeof(T));
+    }
+    if (e != hipSuccess) p = nullptr;
+    return e;
+}
+
 gs_status ensure_sims(gs_ctx *ctx, size_t sims) {
     if (ctx->cap_sims >= sims) return GS_OK;
     if (ctx->d_words) { (void)hipFree(ctx->d_words); ctx->d_words = nullptr; ctx->cap_sims = 0; }
-    HIP_TRY(ctx, hipMalloc((void **)&ctx->d_words, sims * words_per_sim() * sizeof(uint64_t)));
+    HIP_TRY(ctx, device_alloc(ctx, ctx->d_words, sims * words_per_sim()));
     ctx->cap_sims = sims;
     return GS_OK;
 }
@@ -202,7 +218,7 @@ gs_status ensure_sims(gs_ctx *ctx, size_t sims) {
 gs_status ensure_params(gs_ctx *ctx, size_t n) {
     if (ctx->cap_params >= n) return GS_OK;
     if (ctx->d_params) { (void)hipFree(ctx->d_params); ctx->d_params = nullptr; ctx->cap_params = 0; }
-    HIP_TRY(ctx, hipMalloc((void **)&ctx->d_params, n * sizeof(DevParams)));
+    HIP_TRY(ctx, device_alloc(ctx, ctx->d_params, n));
     ctx->cap_params = n;
     return GS_OK;
 }
@@ -210,7 +226,7 @@ gs_status ensure_params(gs_ctx *ctx, size_t n) {
 gs_status ensure_meta(gs_ctx *ctx, size_t words) {
     if (ctx->cap_meta >= words) return GS_OK;
     if (ctx->d_meta) { (void)hipFree(ctx->d_meta); ctx->d_meta = nullptr; ctx->cap_meta = 0; }
-    HIP_TRY(ctx, hipMalloc((void **)&ctx->d_meta, words * sizeof(uint64_t)));
+    HIP_TRY(ctx, device_alloc(ctx, ctx->d_meta, words));
     ctx->cap_meta = words;
     return GS_OK;
 }
@@ -218,25 +234,17 @@ gs_status ensure_meta(gs_ctx *ctx, size_t words) {
 gs_status ensure_events(gs_ctx *ctx, uint64_t n) {
     if (ctx->cap_events >= n) return GS_OK;
     if (ctx->d_events) { (void)hipFree(ctx->d_events); ctx->d_events = nullptr; ctx->cap_events = 0; }
-    hipError_t e = hipMalloc((void **)&ctx->d_events, n * sizeof(gs::DevEvent));
-    if (e == hipErrorOutOfMemory && ctx->d_recs) {   // events before the ordered copy of an earlier run's records
-        (void)hipGetLastError();
-        (void)hipFree(ctx->d_recs);
-        ctx->d_recs = nullptr;
-        ctx->cap_recs = 0;
-        e = hipMalloc((void **)&ctx->d_events, n * sizeof(gs::DevEvent));
-    }
-    HIP_TRY(ctx, e);
+    HIP_TRY(ctx, device_alloc(ctx, ctx->d_events, n));
     ctx->cap_events = n;
     return GS_OK;
 }
 
 gs_status ensure_order(gs_ctx *ctx, uint64_t n) {
     if (!ctx->d_order_counts)
-        HIP_TRY(ctx, hipMalloc((void **)&ctx->d_order_counts, 2 * gs::kOrderMaxBuckets * sizeof(uint32_t)));
+        HIP_TRY(ctx, device_alloc(ctx, ctx->d_order_counts, 2 * gs::kOrderMaxBuckets));
     if (ctx->cap_order >= n) return GS_OK;
     if (ctx->d_order) { (void)hipFree(ctx->d_order); ctx->d_order = nullptr; ctx->cap_order = 0; }
-    HIP_TRY(ctx, hipMalloc((void **)&ctx->d_order, n * sizeof(uint32_t)));
+    HIP_TRY(ctx, device_alloc(ctx, ctx->d_order, n));
     ctx->cap_order = n;
     return GS_OK;
 }
@@ -244,7 +252,7 @@ gs_status ensure_order(gs_ctx *ctx, uint64_t n) {
 gs_status ensure_spill(gs_ctx *ctx, uint64_t n) {
     if (ctx->cap_spill >= n) return GS_OK;
     if (ctx->d_spill) { (void)hipFree(ctx->d_spill); ctx->d_spill = nullptr; ctx->cap_spill = 0; }
-    HIP_TRY(ctx, hipMalloc((void **)&ctx->d_spill, 2 * n * sizeof(gs::SpillRec)));
+    HIP_TRY(ctx, device_alloc(ctx, ctx->d_spill, 2 * n));
     ctx->cap_spill = n;
     return GS_OK;
 }
@@ -252,12 +260,12 @@ gs_status ensure_spill(gs_ctx *ctx, uint64_t n) {
 gs_status ensure_batch_order(gs_ctx *ctx, uint64_t n, uint64_t count_words) {
     if (ctx->cap_border < n) {
         if (ctx->d_border) { (void)hipFree(ctx->d_border); ctx->d_border = nullptr; ctx->cap_border = 0; }
-        HIP_TRY(ctx, hipMalloc((void **)&ctx->d_border, n * sizeof(uint32_t)));
+        HIP_TRY(ctx, device_alloc(ctx, ctx->d_border, n));
         ctx->cap_border = n;
     }
     if (ctx->cap_bcounts < count_words) {
         if (ctx->d_bcounts) { (void)hipFree(ctx->d_bcounts); ctx->d_bcounts = nullptr; ctx->cap_bcounts = 0; }
-        HIP_TRY(ctx, hipMalloc((void **)&ctx->d_bcounts, count_words * sizeof(uint32_t)));
+        HIP_TRY(ctx, device_alloc(ctx, ctx->d_bcounts, count_words));
         ctx->cap_bcounts = count_words;
     }
     return GS_OK;

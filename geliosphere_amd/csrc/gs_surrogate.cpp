@@ -749,7 +749,7 @@ static gs_status predict_pinned(gs_surrogate *s, const float *x, uint32_t n, flo
         if (fallback) std::memcpy(fallback + r0, f, rows);
         return GS_OK;
     };
-    const uint32_t blocks = (n + kHostChunk - 1) / kHostChunk;
+    const uint32_t blocks = (n - 1) / kHostChunk + 1;   // n > 0
     gs_status st = GS_OK;
     for (uint32_t c = 0; c < blocks && st == GS_OK; ++c) {
         if (c >= 2 && (st = take(c - 2)) != GS_OK) break;
