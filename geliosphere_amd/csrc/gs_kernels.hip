@@ -550,7 +550,7 @@ batch_kernel(const DevParams *__restrict__ sims, uint32_t n_sims, const uint64_t
 //    repeated in full steps.  A lone wave pays about 130 cycles for a test (the
 //    compare, the branch, the first normals' LDS latency), so where a wave holds
 //    few particles, whose events are then rare, it looks less often: per step
-//    93 -> 62 ns in 1D at 64 lanes (8 cycles to a test; 4: 66; now 61), 606 -> 566 ns
+//    93 -> 62 ns in 1D at 64 lanes (8 cycles to a test; 4: 66), 606 -> 566 ns
 //    SolarProp, 760 -> 711 ns Geliosphere (4 cycles; 2: 580 and 740; 4 of its
 //    cycles are 50 KB of code, and more would leave the instruction cache).
 //    (About 1 in 5000 lane-cycles of a 1D B-p run has an event.)
