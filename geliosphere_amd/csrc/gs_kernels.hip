@@ -280,6 +280,23 @@ __device__ void run_lanes(const DevParams *__restrict__ sims, uint32_t n_sims, c
         if constexpr (kVecParams) return lp;
         else return P0;
     };
+    // The same, read again from memory (scalar loads, in time for three waves a
+    // SIMD): an empty asm hides that the address is the one of the iteration
+    // before.  Kept over the loop, the 2D models' parameters crowded its constants
+    // out of the scalar registers into vector-register lanes, each written and read
+    // by a vector instruction: 646 of them in two SolarProp steps, now 619.  In ms:
+    // SolarProp 1e7 1556 to 1531, Geliosphere 1e6 367 to 360, 4e6 1035 to 1021.  (As
+    // vector loads: 1546, 383, 1033.)
+    auto params_again = [&]() -> const StepParams & {
+        if constexpr (kVecParams) {
+            return lp;
+        } else {
+            uint64_t at = (uint64_t)&P0;
+            asm volatile("" : "+s"(at));
+            typedef const StepParams __attribute__((address_space(4))) ConstParams;   // scalar loads
+            return *(const StepParams *)(ConstParams *)at;
+        }
+    };
 
     for (;;) {
         // ---- refill idle lanes (wave-uniform control flow)
@@ -399,8 +416,9 @@ __device__ void run_lanes(const DevParams *__restrict__ sims, uint32_t n_sims, c
                 double t[4];
                 if constexpr (!kBatch) asm volatile("" : "+s"(k0), "+s"(k1));   // as above
                 normal_block(pid, blk + (uint32_t)(s >> 1), k0, k1, bm, t);
+                const StepParams &Pm = params_again();
 #pragma unroll
-                for (int h = 0; h < 2; ++h) m.fast_step(params(), &t[2 * h], bm.trig, watch);
+                for (int h = 0; h < 2; ++h) m.fast_step(Pm, &t[2 * h], bm.trig, watch);
             }
         } else {
             // 2D Geliosphere: steps stay rolled (the step body is large).
@@ -430,7 +448,7 @@ __device__ void run_lanes(const DevParams *__restrict__ sims, uint32_t n_sims, c
                         c0 = t[1]; c1 = t[2]; c2 = t[3];
                     }
                 }
-                m.fast_step(params(), z, bm.trig, watch);
+                m.fast_step(params_again(), z, bm.trig, watch);
             }
         }
         const bool again = active & !((int)m.fast_ok(params(), watch, old) & (int)(cap - steps >= (uint32_t)kCycleSteps));
@@ -1103,8 +1121,8 @@ hipError_t gs_scratch_address(int device, void **ptr, size_t *bytes) {
 using namespace gs;
 
 // Waves per SIMD asked of the register allocator, per kernel (1: no request;
-// the 1D kernels reach 4 waves unasked, SolarProp 3).  Measured: SolarProp at
-// 4 waves (128 VGPRs) spills and runs 5 % slower.
+// the 1D kernels reach 4 waves unasked).  Measured: SolarProp at 4 waves (128
+// VGPRs) spills and runs 5 % slower.
 #ifndef GS_BATCH_WAVES_GE
 #define GS_BATCH_WAVES_GE 2   // 227 VGPRs, no spills; at 3 waves 62 spill and the batch ran 12 % slower
 #endif
@@ -1118,7 +1136,7 @@ using namespace gs;
 #define GS_PLAIN_WAVES_GE 3   // 154 VGPRs, no spills
 #endif
 #ifndef GS_PLAIN_WAVES_SP
-#define GS_PLAIN_WAVES_SP 1
+#define GS_PLAIN_WAVES_SP 3   // 163 VGPRs, no spills (169 unasked)
 #endif
 #ifndef GS_BATCH_WAVES_BP
 #define GS_BATCH_WAVES_BP 5   // 96 VGPRs (17 spilled); 4 waves (121, none) ran 0.8 % faster on 32 B-p simulations at 30 % of the batch benchmark's counts, not switched: the tuned batch shapes were measured at 5
