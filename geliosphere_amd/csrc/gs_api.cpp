@@ -167,7 +167,9 @@ DevParams derive(const gs_params &p) {
     d.al = scaled ? al : 1.0;
     d.al2 = d.al * d.al;
     d.kap = scaled ? 1.0 : d.sk2dt;
-    d.s_lo = !scaled ? hi_word(1e17) : p.model == GS_MODEL_1D_BP ? hi_word(d.al * 0.0101) + 1 : 1u;
+    // F-p's fast steps take it that S keeps its sign: (2/3) V dt below every r they allow
+    const bool fast = scaled && !(p.model == GS_MODEL_1D_FP && (2.0 / 3.0) * p.V * p.dt > 1.0);
+    d.s_lo = !fast ? hi_word(1e17) : p.model == GS_MODEL_1D_BP ? hi_word(d.al * 0.0101) + 1 : 1u;
     const double vs = p.model == GS_MODEL_1D_BP ? -p.V : p.V;
     d.vdt = vs * p.dt;
     d.cp = (2.0 / 3.0) * vs * p.dt;

@@ -482,8 +482,10 @@ struct Fp {
     // the cycle included: a crossing looks at both ends of a step; particles
     // start at 100.0001, one unit of the high word above 100, and end at
     // 100.0002, three above) and beta stays above 0.01: P falls from step to
-    // step, so the lowest beta is the last one, or, after a reflection before
-    // the cycle (beta then belongs to a discarded P), the first.
+    // step (a factor 1 - (2/3) V dt / r, positive as (2/3) V dt is at most 1: wider
+    // steps have no fast steps, see s_lo), so the lowest beta is the last one, or,
+    // after a reflection before the cycle (beta then belongs to a discarded P), the
+    // first.
     struct Watch { uint32_t hmax, hmin; };
     static constexpr uint32_t kRLo = hi_word(1.01), kRHi = hi_word(100.0002);
     __device__ __forceinline__ Watch watch() const { return {hi_of(r), hi_of(r)}; }
