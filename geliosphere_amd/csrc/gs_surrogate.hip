@@ -45,13 +45,21 @@ __device__ __forceinline__ bf16x8 frag(const __bf16 *M, int K, int nt, int ks, i
     return *(const bf16x8 *)(M + (((size_t)nt * (size_t)(K >> 5) + (size_t)ks) * 64 + (size_t)lane) * 8);
 }
 
-// bf16(silu(z)), z / (1 + e^-z) with one Newton step in place of the IEEE division (div_fixup
-// keeps its zeros, infinities and NaN): over all 2^32 floats the same bf16 value
-// but for z in (-88.73, -87.33), results under 1e-36.  The division was half of
+// bf16(silu(z)) = bf16(z / (1 + e^-z)) from ez = e^-z and z / 4, with one Newton step in
+// place of the IEEE division (div_fixup keeps its zeros, infinities and NaN): (z / 4) /
+// (1/4 + e^-z / 4), so that the reciprocal stays a normal number up to the largest
+// finite e^-z.  Over all 2^32 floats z the bf16 value of the division but for 512 with
+// |z| < 5e-38, whose subnormal results differ in the last bit.  The division was half of
 // the activation's instructions.
-__device__ __forceinline__ __bf16 silu_act(float z) {
-    const float d = 1.0f + __expf(-z), y = __builtin_amdgcn_rcpf(d), q = z * y;
-    return (__bf16)__builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, z), y, q), d, z);
+__device__ __forceinline__ __bf16 silu_of(float ez, float z4) {
+    const float d = fmaf(ez, 0.25f, 0.25f), y = __builtin_amdgcn_rcpf(d), q = z4 * y;
+    return (__bf16)__builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, z4), y, q), d, z4);
+}
+// (training: dsilu takes the same e^-z)
+__device__ __forceinline__ __bf16 silu_act(float z) { return silu_of(__expf(-z), 0.25f * z); }
+__device__ __forceinline__ __bf16 silu_of_quarter(float z4) {
+    constexpr float kM4Log2E = -4.0f * 1.44269504088896340736f;
+    return silu_of(__builtin_amdgcn_exp2f(z4 * kM4Log2E), z4);
 }
 __device__ __forceinline__ float dsilu(float z) {
     const float s = 1.0f / (1.0f + __expf(-z));
@@ -152,7 +160,7 @@ __global__ void __launch_bounds__(256) gemm_kernel(GemmArgs g) {
 //    their use, across layers, so that the epilogue of a layer hides the first
 //    loads of the next.
 //  - The SiLU is most of the vector work (two transcendentals and seven other
-//    operations per element): see silu_act.
+//    operations per element): see silu_of_quarter.
 // RT row tiles of 16 by NW waves, chosen by sg_launch_mlp_forward.  Four waves per SIMD: two
 // (four waves of 64 columns each) gave 195 us instead of 160 for 65,536 rows of
 // four members.  There the products alone take 114 us, near the rate of a large
@@ -208,11 +216,14 @@ __global__ void __launch_bounds__(NW * 64, 4) mlp_forward_kernel(MlpArgs g) {
         for (int j = 0; j < CJ; ++j) {
             const int n = 16 * (ct0 + j) + 4 * quad;
             const f32x4 b = *(const f32x4 *)(bias + n);
+            float b4[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) b4[v] = 0.25f * b[v];
 #pragma unroll
             for (int i = 0; i < RT; ++i) {
                 bf16x4 a;
 #pragma unroll
-                for (int v = 0; v < 4; ++v) a[v] = silu_act(acc[i][j][v] + b[v]);
+                for (int v = 0; v < 4; ++v) a[v] = silu_of_quarter(fmaf(acc[i][j][v], 0.25f, b4[v]));   // (acc + b) / 4
                 *(bf16x4 *)(act + (16 * i + fr) * FLD + n) = a;
             }
         }
