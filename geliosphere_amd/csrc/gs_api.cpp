@@ -169,7 +169,7 @@ DevParams derive(const gs_params &p) {
     d.kap = scaled ? 1.0 : d.sk2dt;
     // F-p's fast steps take it that S keeps its sign: (2/3) V dt below every r they allow
     const bool fast = scaled && !(p.model == GS_MODEL_1D_FP && (2.0 / 3.0) * p.V * p.dt > 1.0);
-    d.s_lo = !fast ? hi_word(1e17) : p.model == GS_MODEL_1D_BP ? hi_word(d.al * 0.0101) + 1 : 1u;
+    d.s_lo = !fast ? gs::kNoFast : p.model == GS_MODEL_1D_BP ? hi_word(d.al * 0.0101) + 1 : 1u;
     const double vs = p.model == GS_MODEL_1D_BP ? -p.V : p.V;
     d.vdt = vs * p.dt;
     d.cp = (2.0 / 3.0) * vs * p.dt;
@@ -191,6 +191,11 @@ DevParams derive(const gs_params &p) {
     d.max_steps = p.max_steps ? p.max_steps : kDefaultMaxSteps;
     for (uint32_t i = 0; i <= p.n_bins; ++i) d.edges[i] = p.bin_edges[i];
     return d;
+}
+
+// Whether a simulation's kernels are those without fast steps.
+bool full_only(const gs_params &p) {
+    return (p.model == GS_MODEL_1D_FP || p.model == GS_MODEL_1D_BP) && derive(p).s_lo == gs::kNoFast;
 }
 
 // Room for n elements.  Where the device has none, the ordered copy of an earlier
@@ -450,7 +455,7 @@ unsigned throughput_grid(const gs_ctx *ctx, int model, const Resolved &R, uint64
 // word per launch, zeroed.
 // all_lanes: one wave per SIMD of the device.  part of parts: the share of the
 // device that a batch's model group takes once its particles fit there.
-hipError_t queue_tail(uint64_t all_lanes, int part, int parts, int model, bool batch, const DevParams *sims, uint32_t n_sims,
+hipError_t queue_tail(uint64_t all_lanes, int part, int parts, int model, bool full, bool batch, const DevParams *sims, uint32_t n_sims,
                       const uint64_t *offsets, const DevOut &O, uint64_t fresh_n, gs::SpillRec *half0,
                       gs::SpillRec *half1, uint64_t cap, uint64_t *counts, hipStream_t s) {
     const uint64_t most = fresh_n ? fresh_n : cap;
@@ -475,7 +480,7 @@ hipError_t queue_tail(uint64_t all_lanes, int part, int parts, int model, bool b
         A.lanes = (uint32_t)lanes;
         A.xcd_lo = (uint32_t)part * xcds;
         A.xcd_n = xcds;
-        const hipError_t e = gs_launch_tail(model, batch, sims, n_sims, offsets, O, A, grid, s);
+        const hipError_t e = gs_launch_tail(model, full, batch, sims, n_sims, offsets, O, A, grid, s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -589,20 +594,28 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
     // ---- order
     std::vector<uint32_t> order(part);
     double gcost[4] = {0, 0, 0, 0};
-    for (uint32_t i : order) gcost[sims[i].model] += est_cost(sims[i]) * (double)sims[i].n_particles;
+    std::vector<uint8_t> full(*std::max_element(part.begin(), part.end()) + 1);   // by simulation
+    for (uint32_t i : order) {
+        gcost[sims[i].model] += est_cost(sims[i]) * (double)sims[i].n_particles;
+        full[i] = full_only(sims[i]);
+    }
     std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) {
         const int ma = sims[a].model, mb = sims[b].model;
         if (ma != mb) return gcost[ma] != gcost[mb] ? gcost[ma] < gcost[mb] : ma < mb;
+        if (full[a] != full[b]) return full[b] != 0;
         return est_cost(sims[a]) > est_cost(sims[b]);
     });
     // ---- launches: (model, first sim, count)
-    struct Launch { int model; uint32_t base, count; unsigned grid, block, chunk; size_t off_pos; };
+    struct Launch { int model; bool full; uint32_t base, count; unsigned grid, block, chunk; size_t off_pos; };
     std::vector<Launch> launches;
     for (size_t j = 0; j < m;) {
         size_t k = j;
-        while (k < m && sims[order[k]].model == sims[order[j]].model && k - j < (size_t)gs::kBatchMaxSims) ++k;
+        while (k < m && sims[order[k]].model == sims[order[j]].model && full[order[k]] == full[order[j]] &&
+               k - j < (size_t)gs::kBatchMaxSims)
+            ++k;
         Launch L;
         L.model = sims[order[j]].model;
+        L.full = full[order[j]] != 0;
         L.base = (uint32_t)j;
         L.count = (uint32_t)(k - j);
         const Resolved R = resolve_shape(ctx, L.model, true);
@@ -686,7 +699,7 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
     for (size_t l = 0; l < nl; ++l) {
         const Launch &L = launches[l];
         key.push_back(nv[l]);   // slices of the permutation and the records, fresh tail launches
-        key.push_back((uint64_t)L.model);
+        key.push_back((uint64_t)L.model * 2 + L.full);
         key.push_back(L.count);
         key.push_back(L.grid);
         key.push_back(L.block);
@@ -716,7 +729,7 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
         std::vector<int> group_of(nl);
         int n_groups = 0;
         for (size_t l = 0; l < nl; ++l) {
-            if (l == 0 || launches[l].model != launches[l - 1].model) ++n_groups;
+            if (l == 0 || launches[l].model != launches[l - 1].model || launches[l].full != launches[l - 1].full) ++n_groups;
             group_of[l] = n_groups - 1;
         }
         const int parts = n_groups >= 3 ? 4 : n_groups;   // of the device, for tails side by side
@@ -747,21 +760,22 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
             O.ev_off = ctx->d_meta + L.base;
             O.ev_cap = ctx->d_meta + m + L.base;
             O.n_events = ctx->d_meta + 2 * m + L.base;
-            const bool fresh = nv[l] > 0 && nv[l] <= tail_lanes(ctx);
+            const bool fresh = nv[l] > 0 && nv[l] <= tail_lanes(ctx), tail = nv[l] > 0 && (fresh || !L.full);
+            if (!tail) O.spill = nullptr;
             if (!fresh) {
                 // One throughput launch after another (each fills the device; the
                 // tail of one overlaps the next): with all at once the group with
                 // the longest tail got its share of the slots last.
                 if (after) e = hipStreamWaitEvent(sg, ctx->traj[after - 1], 0);
                 if (e == hipSuccess)
-                    e = gs_launch_traj(L.model, true, ctx->d_params + L.base, L.count, ctx->d_meta + L.off_pos, O,
+                    e = gs_launch_traj(L.model, L.full, true, ctx->d_params + L.base, L.count, ctx->d_meta + L.off_pos, O,
                                        L.grid, L.block, sg);
                 if (e == hipSuccess) e = hipEventRecord(ctx->traj[g], sg);
                 after = g + 1;
             }
-            if (e == hipSuccess && nv[l] > 0)
-                e = queue_tail(tail_lanes(ctx), g, parts, L.model, true, ctx->d_params + L.base, L.count, ctx->d_meta + L.off_pos, O,
-                               fresh ? nv[l] : 0, half0, half1, spill_cap[l], counts, sg);
+            if (e == hipSuccess && tail)
+                e = queue_tail(tail_lanes(ctx), g, parts, L.model, L.full, true, ctx->d_params + L.base, L.count,
+                               ctx->d_meta + L.off_pos, O, fresh ? nv[l] : 0, half0, half1, spill_cap[l], counts, sg);
         }
         for (int g = 0; g < 3 && e == hipSuccess; ++g) {
             if (!used[g]) continue;
@@ -859,6 +873,7 @@ gs_status run_plain_core(gs_ctx *ctx, const gs_params &pp, gs_spectrum *out, gs_
     Layout L = layout(B.words, 1);
     HIP_TRY(ctx, gs_launch_zero(B.words, kWordsPerSim, ctx->stream));
     const Resolved RS = resolve_shape(ctx, p->model, false);
+    const bool full = full_only(*p);
     unsigned grid = RS.grid;
     uint64_t kept = 0;   // records stored
     uint64_t total_events = 0;
@@ -919,10 +934,11 @@ gs_status run_plain_core(gs_ctx *ctx, const gs_params &pp, gs_spectrum *out, gs_
         HIP_TRY(ctx, gs_launch_zero(B.meta + 2, 2 + kTailRounds + 1, ctx->stream));   // events, cycles, hand-on counts
         O.events = events;
         // the tail needs the context's record buffer
-        if (B.own) grid = throughput_grid(ctx, q.model, RS, q.n_particles);
+        if (B.own && !full) grid = throughput_grid(ctx, q.model, RS, q.n_particles);
         const uint64_t cap_tail = tail_cap(ctx, q.n_particles, (uint64_t)grid * RS.block);
         const bool fresh = B.own && q.n_particles > 0 && q.n_particles <= tail_lanes(ctx);
-        if (B.own) {
+        const bool tail = B.own && q.n_particles > 0 && (fresh || !full);
+        if (tail) {
             st = ensure_spill(ctx, cap_tail);
             if (st != GS_OK) return st;
             O.spill = ctx->d_spill;
@@ -930,10 +946,10 @@ gs_status run_plain_core(gs_ctx *ctx, const gs_params &pp, gs_spectrum *out, gs_
             O.spill_cap = cap_tail;
         }
         HIP_TRY(ctx, hipEventRecord(ctx->ev0, ctx->stream));
-        if (!fresh) HIP_TRY(ctx, gs_launch_traj(q.model, false, B.params, 1, nullptr, O, grid, RS.block, ctx->stream));
-        if (B.own && q.n_particles > 0)
-            HIP_TRY(ctx, queue_tail(tail_lanes(ctx), 0, 1, q.model, false, B.params, 1, nullptr, O, fresh ? q.n_particles : 0, ctx->d_spill,
-                                    ctx->d_spill + ctx->cap_spill, cap_tail, B.meta + 4, ctx->stream));
+        if (!fresh) HIP_TRY(ctx, gs_launch_traj(q.model, full, false, B.params, 1, nullptr, O, grid, RS.block, ctx->stream));
+        if (tail)
+            HIP_TRY(ctx, queue_tail(tail_lanes(ctx), 0, 1, q.model, full, false, B.params, 1, nullptr, O, fresh ? q.n_particles : 0,
+                                    ctx->d_spill, ctx->d_spill + ctx->cap_spill, cap_tail, B.meta + 4, ctx->stream));
         HIP_TRY(ctx, hipEventRecord(ctx->ev1, ctx->stream));
         uint64_t nev = 0;
         HIP_TRY(ctx, hipMemcpyAsync(&nev, B.meta + 2, sizeof nev, hipMemcpyDeviceToHost, ctx->stream));

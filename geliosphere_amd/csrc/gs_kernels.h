@@ -40,6 +40,7 @@ enum Stat {
     ST_COUNT_
 };
 
+constexpr uint32_t kNoFast = 0x43763457u;   // the high word of 1e17, which no S of a fast step reaches
 // Parameters a model's init/step read (host-derived constants included).
 // Batched runs copy them per lane into registers; plain runs read them
 // wave-uniformly.
@@ -68,7 +69,7 @@ struct StepParams {
     double polthdt;       // pol_theta dt (2D SolarProp theta drift)
     double sq2dt;         // sqrt(2 dt)
     double delta0_rh;     // delta0 / rh
-    uint32_t s_lo;        // 1D fast steps: the high word that alpha P has to reach (that of 1e17: none)
+    uint32_t s_lo;        // 1D fast steps: the high word that alpha P has to reach (kNoFast: no fast steps)
     uint32_t pad_;
 };
 
@@ -206,15 +207,15 @@ hipError_t gs_launch_debug(int fn, const double *x, double *y, uint64_t n, uint6
 bool gs_traj_block_supported(unsigned block_threads);
 // Blocks of `block_threads` a CU holds for the trajectory kernel of `model`.
 hipError_t gs_traj_occupancy(int model, bool batch, unsigned block_threads, int *blocks_per_cu);
-// Trajectories of n_sims simulations of one model.  sims: device array;
-// offsets: device array of n_sims + 1 prefix sums of n_particles (the
+// Trajectories of n_sims simulations of one model.  full: none of them has fast
+// steps (s_lo == kNoFast; 1D).  sims: device array; offsets: device array of n_sims + 1 prefix sums of n_particles (the
 // virtual id space).  batch = false requires n_sims == 1 (uniform parameters).
-hipError_t gs_launch_traj(int model, bool batch, const gs::DevParams *sims, uint32_t n_sims,
+hipError_t gs_launch_traj(int model, bool full, bool batch, const gs::DevParams *sims, uint32_t n_sims,
                           const uint64_t *offsets, const gs::DevOut &O, unsigned grid,
                           unsigned block_threads, hipStream_t s);
 // One tail launch of `model` over `grid` workgroups of kTailThreads; grid must
 // hold one lane per particle.
-hipError_t gs_launch_tail(int model, bool batch, const gs::DevParams *sims, uint32_t n_sims,
+hipError_t gs_launch_tail(int model, bool full, bool batch, const gs::DevParams *sims, uint32_t n_sims,
                           const uint64_t *offsets, const gs::DevOut &O, const gs::TailArgs &A, unsigned grid,
                           hipStream_t s);
 // Scheduling order of the n = sims->n_particles particles of one plain

@@ -221,6 +221,19 @@ __device__ __forceinline__ bool slow_cycle(Model &m, const Prm &P, const Normals
     return active;
 }
 
+// A cycle of full steps (1D) for every lane that holds a particle.
+template <class Model, class Prm, class Emit>
+__device__ __forceinline__ void full_cycle(Model &m, const Prm &P, const double *z, const double *trig, bool &active,
+                                           uint32_t &steps, const Emit &emit) {
+#pragma unroll
+    for (int s = 0; s < kCycleSteps; ++s) {
+        if (active) {
+            ++steps;
+            if (!m.step(P, &z[s], trig, emit)) active = false;
+        }
+    }
+}
+
 // The lanes of one wave integrate particles until the id space is exhausted.
 //
 // kBatch = false: one simulation, parameters read wave-uniformly from sims[0];
@@ -406,6 +419,19 @@ __device__ void run_lanes(const DevParams *__restrict__ sims, uint32_t n_sims, c
                 asm volatile("" : "+s"(k0), "+s"(k1));
             }
             normal_block(pid, blk, k0, k1, bm, z1);
+            if constexpr (Model::kFullOnly) {
+                if (__ballot(active && cap - steps < (uint32_t)kCycleSteps) == 0) {
+                    const bool had = active;
+                    full_cycle(m, params(), z1, bm.trig, active, steps, emit);
+                    if (had && !active) st.ended(m, steps);
+                } else if (active) {
+                    active = slow_cycle<kCycleSteps>(m, params(), [&](int s, double *z) { z[0] = z1[s]; }, bm.trig, cap,
+                                                     steps, st, emit);
+                }
+                stage_flush<kBatch>(stage, O, kStageFlush);
+                blk += (uint32_t)NPS;
+                continue;
+            }
 #pragma unroll
             for (int s = 0; s < kCycleSteps; ++s) m.fast_step(params(), &z1[s], bm.trig, watch);
         } else if constexpr (NPS == 2) {
@@ -689,7 +715,7 @@ __global__ void __launch_bounds__(kTailThreads) tail_kernel(const DevParams *__r
                 const Model old = m;
                 typename Model::Watch watch = m.watch();
 #pragma unroll
-                for (int s = 0; s < kSteps; ++s) {
+                for (int s = 0; s < (Model::kFullOnly ? 0 : kSteps); ++s) {
                     double z[NPS];
                     for (int i = 0; i < NPS; ++i) z[i] = zc[NPS * s + i];
                     // 1D: the normals of one cycle at a time in registers (all 32 at the
@@ -697,7 +723,8 @@ __global__ void __launch_bounds__(kTailThreads) tail_kernel(const DevParams *__r
                     if (NPS == 1 && s % kCycleSteps == kCycleSteps - 1) __builtin_amdgcn_sched_barrier(0);
                     m.template fast_step<kLanes>(lp, z, bm.trig, watch);
                 }
-                const bool again = active & !((int)m.fast_ok(lp, watch, old) & (int)(cap - steps >= (uint32_t)kSteps));
+                const bool again = active & (Model::kFullOnly || !((int)m.fast_ok(lp, watch, old) &
+                                                                   (int)(cap - steps >= (uint32_t)kSteps)));
                 cycles += kAtOnce;
                 if (__ballot(again)) {
                     if (again) {
@@ -1230,14 +1257,16 @@ static void launch_traj_t(bool batch, const DevParams *sims, uint32_t n_sims, co
 }
 
 template <int kThreads>
-static bool launch_traj_b(int model, bool batch, const DevParams *sims, uint32_t n_sims, const uint64_t *offsets,
+static bool launch_traj_b(int model, bool full, bool batch, const DevParams *sims, uint32_t n_sims, const uint64_t *offsets,
                           const DevOut &O, unsigned grid, hipStream_t s) {
     switch (model) {
     case GS_MODEL_1D_FP:
-        launch_traj_t<Fp, kBatchWaves1D, kPlainWaves1D, kThreads>(batch, sims, n_sims, offsets, O, grid, s);
+        if (full) launch_traj_t<FullOnly<Fp>, kBatchWaves1D, kPlainWaves1D, kThreads>(batch, sims, n_sims, offsets, O, grid, s);
+        else launch_traj_t<Fp, kBatchWaves1D, kPlainWaves1D, kThreads>(batch, sims, n_sims, offsets, O, grid, s);
         return true;
     case GS_MODEL_1D_BP:
-        launch_traj_t<Bp, kBatchWavesBp, kPlainWavesBp, kThreads>(batch, sims, n_sims, offsets, O, grid, s);
+        if (full) launch_traj_t<FullOnly<Bp>, kBatchWavesBp, kPlainWavesBp, kThreads>(batch, sims, n_sims, offsets, O, grid, s);
+        else launch_traj_t<Bp, kBatchWavesBp, kPlainWavesBp, kThreads>(batch, sims, n_sims, offsets, O, grid, s);
         return true;
     case GS_MODEL_2D_SOLARPROP:
         launch_traj_t<Sp, kBatchWavesSp, kPlainWavesSp, kThreads>(batch, sims, n_sims, offsets, O, grid, s);
@@ -1249,7 +1278,7 @@ static bool launch_traj_b(int model, bool batch, const DevParams *sims, uint32_t
     }
 }
 
-hipError_t gs_launch_traj(int model, bool batch, const DevParams *sims, uint32_t n_sims,
+hipError_t gs_launch_traj(int model, bool full, bool batch, const DevParams *sims, uint32_t n_sims,
                           const uint64_t *offsets, const DevOut &O, unsigned grid, unsigned block_threads,
                           hipStream_t s) {
     if (n_sims == 0 || grid == 0) return hipSuccess;
@@ -1257,9 +1286,9 @@ hipError_t gs_launch_traj(int model, bool batch, const DevParams *sims, uint32_t
         return hipErrorInvalidValue;
     bool ok;
     switch (block_threads) {
-    case 128: ok = launch_traj_b<128>(model, batch, sims, n_sims, offsets, O, grid, s); break;
-    case 256: ok = launch_traj_b<256>(model, batch, sims, n_sims, offsets, O, grid, s); break;
-    case 512: ok = launch_traj_b<512>(model, batch, sims, n_sims, offsets, O, grid, s); break;
+    case 128: ok = launch_traj_b<128>(model, full, batch, sims, n_sims, offsets, O, grid, s); break;
+    case 256: ok = launch_traj_b<256>(model, full, batch, sims, n_sims, offsets, O, grid, s); break;
+    case 512: ok = launch_traj_b<512>(model, full, batch, sims, n_sims, offsets, O, grid, s); break;
     default: ok = false; break;
     }
     if (!ok) return hipErrorInvalidValue;
@@ -1275,7 +1304,7 @@ static void launch_tail_t(bool batch, const DevParams *sims, uint32_t n_sims, co
         hipLaunchKernelGGL((tail_kernel<Model, false>), dim3(grid), dim3(kTailThreads), 0, s, sims, n_sims, offsets, O, A);
 }
 
-hipError_t gs_launch_tail(int model, bool batch, const DevParams *sims, uint32_t n_sims, const uint64_t *offsets,
+hipError_t gs_launch_tail(int model, bool full, bool batch, const DevParams *sims, uint32_t n_sims, const uint64_t *offsets,
                           const DevOut &O, const TailArgs &A, unsigned grid, hipStream_t s) {
     if (n_sims == 0 || grid == 0) return hipSuccess;
     const uint64_t lanes = (uint64_t)grid * kTailThreads;
@@ -1283,8 +1312,14 @@ hipError_t gs_launch_tail(int model, bool batch, const DevParams *sims, uint32_t
         A.xcd_n == 0 || A.xcd_lo + A.xcd_n > kXcds || (A.in ? !A.n_in || A.cap > lanes : A.fresh_n > lanes) || (A.out && A.cap < (A.in ? A.cap : A.fresh_n)) || (A.out && !A.n_out) || A.budget == 0)
         return hipErrorInvalidValue;
     switch (model) {
-    case GS_MODEL_1D_FP: launch_tail_t<Fp>(batch, sims, n_sims, offsets, O, A, grid, s); break;
-    case GS_MODEL_1D_BP: launch_tail_t<Bp>(batch, sims, n_sims, offsets, O, A, grid, s); break;
+    case GS_MODEL_1D_FP:
+        if (full) launch_tail_t<FullOnly<Fp>>(batch, sims, n_sims, offsets, O, A, grid, s);
+        else launch_tail_t<Fp>(batch, sims, n_sims, offsets, O, A, grid, s);
+        break;
+    case GS_MODEL_1D_BP:
+        if (full) launch_tail_t<FullOnly<Bp>>(batch, sims, n_sims, offsets, O, A, grid, s);
+        else launch_tail_t<Bp>(batch, sims, n_sims, offsets, O, A, grid, s);
+        break;
     case GS_MODEL_2D_SOLARPROP: launch_tail_t<Sp>(batch, sims, n_sims, offsets, O, A, grid, s); break;
     case GS_MODEL_2D_GELIOSPHERE: launch_tail_t<Ge>(batch, sims, n_sims, offsets, O, A, grid, s); break;
     default: return hipErrorInvalidValue;
