@@ -938,6 +938,7 @@ gs_status run_plain_core(gs_ctx *ctx, const gs_params &pp, gs_spectrum *out, gs_
         const uint64_t cap_tail = tail_cap(ctx, q.n_particles, (uint64_t)grid * RS.block);
         const bool fresh = B.own && q.n_particles > 0 && q.n_particles <= tail_lanes(ctx);
         const bool tail = B.own && q.n_particles > 0 && (fresh || !full);
+        O.spill = nullptr;
         if (tail) {
             st = ensure_spill(ctx, cap_tail);
             if (st != GS_OK) return st;

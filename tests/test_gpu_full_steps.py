@@ -59,3 +59,16 @@ def test_no_cycle_is_computed_twice(engine):
         return min(ms)
     with_k, without = best(r_inj=3.0, T_min=0.05), best(**NONE)
     assert without < 1.9 * with_k, (without, with_k)
+
+
+def test_launches_of_changing_size(engine):
+    """Chunks that are cut to fit a small event region and grow again: a launch
+    without a hand-on after one with."""
+    p = abi.make_params(abi.MODEL_1D_FP, N=200_000, seed=3, dt=6e5, K0_cm2s=5e22)
+    whole = engine.run_plain(p)[0]
+    assert whole.n_events > 1000
+    engine.set_plain_limits(max_events=300)
+    try:
+        assert bytes(engine.run_plain(p)[0]) == bytes(whole)
+    finally:
+        engine.set_plain_limits()
