@@ -443,6 +443,13 @@ uint64_t tail_cap(const gs_ctx *ctx, uint64_t n, uint64_t traj_lanes) {
 // any number of waves.  (Plain runs only: a batch's groups fill each other's gaps;
 // there it cost a fifth.)
 constexpr uint64_t kLaneParticles = 16;
+// Few waves, and tail launches after a throughput launch, are for lifetimes that
+// differ; under a step cap most particles end at the cap, at once.  Below kSpreadSteps
+// of cap the launch keeps its shape (dt 500 s, cap 4000, two waves / shape's: B-p
+// 3,000,000 particles 20.9 / 17.6 ms, Geliosphere 86.7 / 80.8), and below kHandOnSteps
+// its particles, for what is left when the ids run out takes less time than the tail
+// launches (cap 500: B-p 3,000,000 6.4 / 4.2 ms, Geliosphere 20.4 / 18.6).
+constexpr uint64_t kSpreadSteps = 16384, kHandOnSteps = 512;
 unsigned throughput_grid(const gs_ctx *ctx, int model, const Resolved &R, uint64_t n) {
     if (model == GS_MODEL_1D_FP || ctx->tuning) return R.grid;
     const uint64_t waves = std::max<uint64_t>(2, n / (kLaneParticles * tail_lanes(ctx)));
@@ -934,10 +941,10 @@ gs_status run_plain_core(gs_ctx *ctx, const gs_params &pp, gs_spectrum *out, gs_
         HIP_TRY(ctx, gs_launch_zero(B.meta + 2, 2 + kTailRounds + 1, ctx->stream));   // events, cycles, hand-on counts
         O.events = events;
         // the tail needs the context's record buffer
-        if (B.own && !full) grid = throughput_grid(ctx, q.model, RS, q.n_particles);
+        if (B.own && !full && hp.max_steps >= kSpreadSteps) grid = throughput_grid(ctx, q.model, RS, q.n_particles);
         const uint64_t cap_tail = tail_cap(ctx, q.n_particles, (uint64_t)grid * RS.block);
         const bool fresh = B.own && q.n_particles > 0 && q.n_particles <= tail_lanes(ctx);
-        const bool tail = B.own && q.n_particles > 0 && (fresh || !full);
+        const bool tail = B.own && q.n_particles > 0 && (fresh || (!full && hp.max_steps >= kHandOnSteps));
         O.spill = nullptr;
         if (tail) {
             st = ensure_spill(ctx, cap_tail);
