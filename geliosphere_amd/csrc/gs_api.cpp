@@ -77,6 +77,7 @@ struct gs_ctx {
     // launch shape per [plain, batch][model]; zero fields take the defaults
     // (256 threads, the occupancy's blocks per CU, kChunk ids per grab)
     gs_launch_shape shape[2][4] = {};
+    bool asked[2][4] = {};          // set by the caller (not by the autotuner or its cache): used as it is
     bool tuning = false;            // the autotuner measures shapes as they are
     double tuned_rate[2][4] = {};   // particle-steps/s of the tuned shapes (0: not tuned)
     std::string arch;               // gcnArchName of the device
@@ -432,6 +433,10 @@ uint64_t tail_cap(const gs_ctx *ctx, uint64_t n, uint64_t traj_lanes) {
     return std::max<uint64_t>(1, std::min<uint64_t>(n, std::max(traj_lanes, tail_lanes(ctx))));
 }
 
+// Whether every run makes the throughput launch, in the launch shape as it is: a
+// caller who sets a shape chooses how the kernel runs; a tuned shape is a default.
+bool shape_rules(const gs_ctx *ctx, int kernel, int model) { return ctx->asked[kernel][model]; }
+
 // Workgroups of the throughput launch for n particles: as the shape says, but no
 // more than two waves per SIMD, or one for every kLaneParticles particles per lane.
 // With few particles per lane the launch's end is the run's: a lane of five waves
@@ -451,7 +456,7 @@ constexpr uint64_t kLaneParticles = 16;
 // launches (cap 500: B-p 3,000,000 6.4 / 4.2 ms, Geliosphere 20.4 / 18.6).
 constexpr uint64_t kSpreadSteps = 16384, kHandOnSteps = 512;
 unsigned throughput_grid(const gs_ctx *ctx, int model, const Resolved &R, uint64_t n) {
-    if (model == GS_MODEL_1D_FP || ctx->tuning) return R.grid;
+    if (model == GS_MODEL_1D_FP || ctx->tuning || shape_rules(ctx, GS_KERNEL_PLAIN, model)) return R.grid;
     const uint64_t waves = std::max<uint64_t>(2, n / (kLaneParticles * tail_lanes(ctx)));
     return (unsigned)std::min<uint64_t>(R.grid, waves * tail_lanes(ctx) / R.block);
 }
@@ -675,10 +680,13 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
         nv[l] = v;
         perm_total += v;
     }
-    // each launch's slice of the hand-on records
+    // launches whose particles go to tail launches alone; each launch's slice of the
+    // hand-on records
+    std::vector<uint8_t> fresh(nl);
     std::vector<uint64_t> spill_at(nl), spill_cap(nl);
     uint64_t spill_total = 0;
     for (size_t l = 0; l < nl; ++l) {
+        fresh[l] = nv[l] > 0 && nv[l] <= tail_lanes(ctx) && !shape_rules(ctx, GS_KERNEL_BATCH, launches[l].model);
         spill_at[l] = spill_total;
         spill_cap[l] = tail_cap(ctx, nv[l], (uint64_t)launches[l].grid * launches[l].block);
         spill_total += spill_cap[l];
@@ -705,7 +713,8 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
                                  (uint64_t)(uintptr_t)ctx->d_spill, ctx->cap_spill};
     for (size_t l = 0; l < nl; ++l) {
         const Launch &L = launches[l];
-        key.push_back(nv[l]);   // slices of the permutation and the records, fresh tail launches
+        key.push_back(nv[l]);   // slices of the permutation and the records
+        key.push_back(fresh[l]);
         key.push_back((uint64_t)L.model * 2 + L.full);
         key.push_back(L.count);
         key.push_back(L.grid);
@@ -767,9 +776,9 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
             O.ev_off = ctx->d_meta + L.base;
             O.ev_cap = ctx->d_meta + m + L.base;
             O.n_events = ctx->d_meta + 2 * m + L.base;
-            const bool fresh = nv[l] > 0 && nv[l] <= tail_lanes(ctx), tail = nv[l] > 0 && (fresh || !L.full);
+            const bool tail = nv[l] > 0 && (fresh[l] || !L.full);
             if (!tail) O.spill = nullptr;
-            if (!fresh) {
+            if (!fresh[l]) {
                 // One throughput launch after another (each fills the device; the
                 // tail of one overlaps the next): with all at once the group with
                 // the longest tail got its share of the slots last.
@@ -782,7 +791,7 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
             }
             if (e == hipSuccess && tail)
                 e = queue_tail(tail_lanes(ctx), g, parts, L.model, L.full, true, ctx->d_params + L.base, L.count,
-                               ctx->d_meta + L.off_pos, O, fresh ? nv[l] : 0, half0, half1, spill_cap[l], counts, sg);
+                               ctx->d_meta + L.off_pos, O, fresh[l] ? nv[l] : 0, half0, half1, spill_cap[l], counts, sg);
         }
         for (int g = 0; g < 3 && e == hipSuccess; ++g) {
             if (!used[g]) continue;
@@ -943,7 +952,8 @@ gs_status run_plain_core(gs_ctx *ctx, const gs_params &pp, gs_spectrum *out, gs_
         // the tail needs the context's record buffer
         if (B.own && !full && hp.max_steps >= kSpreadSteps) grid = throughput_grid(ctx, q.model, RS, q.n_particles);
         const uint64_t cap_tail = tail_cap(ctx, q.n_particles, (uint64_t)grid * RS.block);
-        const bool fresh = B.own && q.n_particles > 0 && q.n_particles <= tail_lanes(ctx);
+        const bool fresh = B.own && q.n_particles > 0 && q.n_particles <= tail_lanes(ctx) &&
+                           !shape_rules(ctx, GS_KERNEL_PLAIN, q.model);
         const bool tail = B.own && q.n_particles > 0 && (fresh || (!full && hp.max_steps >= kHandOnSteps));
         O.spill = nullptr;
         if (tail) {
@@ -1146,6 +1156,7 @@ gs_status gs_set_launch_shape(gs_ctx *ctx, int32_t model, int32_t kernel, const 
     if (shape->chunk > 4096) return fail(ctx, GS_ERR_INVALID_ARG, "chunk above 4096");
     ctx->shape[kernel][model] = *shape;
     ctx->tuned_rate[kernel][model] = 0.0;
+    ctx->asked[kernel][model] = shape->block_threads || shape->blocks_per_cu || shape->chunk;
     return GS_OK;
 }
 
@@ -1243,6 +1254,7 @@ gs_status gs_autotune_shape(gs_ctx *ctx, const gs_params *pilots, uint32_t n_pil
     }
     ctx->shape[kernel][model] = best;
     ctx->tuned_rate[kernel][model] = best_rate;
+    ctx->asked[kernel][model] = false;
     if (best_shape) *best_shape = best;
     if (best_steps_per_s) *best_steps_per_s = best_rate;
     return GS_OK;
@@ -1313,6 +1325,7 @@ gs_status gs_autotune_load(gs_ctx *ctx, const char *path, uint32_t *n_applied) {
         const gs_launch_shape sh{blk, bpcu, chunk};
         if (gs_set_launch_shape(ctx, model, k, &sh) != GS_OK) continue;
         ctx->tuned_rate[k][model] = rate;
+        ctx->asked[k][model] = false;
         ++n;
     }
     std::fclose(in);

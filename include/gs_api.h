@@ -246,10 +246,13 @@ gs_status gs_set_plain_limits(gs_ctx *ctx, uint64_t max_chunk, uint64_t max_even
 /* Launch shape of a trajectory kernel.  block_threads: workgroup size (128,
  * 256 or 512); blocks_per_cu: persistent blocks per CU, so that each lane
  * integrates about N / (blocks_per_cu x CUs x block_threads) particles one
- * after another (capped at the kernel's occupancy; a plain run of fewer than
- * 16 particles per lane launches fewer blocks); chunk: particle ids a wave
+ * after another (capped at the kernel's occupancy); chunk: particle ids a wave
  * takes from the work queue per grab.  0 in a field: the default (256,
- * the occupancy, 64).  Results never depend on the shape. */
+ * the occupancy, 64).  A shape that a caller sets is the one that runs, for any
+ * number of particles.  With defaults and with shapes of the autotuner or its
+ * cache, a plain run of fewer than 16 particles per lane launches fewer blocks,
+ * and particles that fit one wave per SIMD need no such launch at all.  Results
+ * never depend on the shape. */
 typedef struct gs_launch_shape {
     uint32_t block_threads;
     uint32_t blocks_per_cu;
