@@ -850,6 +850,7 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
     }
     for (size_t l = 0; l < nl; ++l) {
         acc.lane_cycles += hmeta[c_base + l] * (uint64_t)gs::kWave * gs::kCycleSteps;
+        if (fresh[l]) continue;
         acc.grid_blocks += launches[l].grid;
         acc.block_threads = launches[l].block;
     }
@@ -890,7 +891,7 @@ gs_status run_plain_core(gs_ctx *ctx, const gs_params &pp, gs_spectrum *out, gs_
     HIP_TRY(ctx, gs_launch_zero(B.words, kWordsPerSim, ctx->stream));
     const Resolved RS = resolve_shape(ctx, p->model, false);
     const bool full = full_only(*p);
-    unsigned grid = RS.grid;
+    unsigned grid = RS.grid, launched = 0;   // workgroups of the throughput launch, and of the last one made
     uint64_t kept = 0;   // records stored
     uint64_t total_events = 0;
     double kernel_ms = 0.0;
@@ -964,7 +965,10 @@ gs_status run_plain_core(gs_ctx *ctx, const gs_params &pp, gs_spectrum *out, gs_
             O.spill_cap = cap_tail;
         }
         HIP_TRY(ctx, hipEventRecord(ctx->ev0, ctx->stream));
-        if (!fresh) HIP_TRY(ctx, gs_launch_traj(q.model, full, false, B.params, 1, nullptr, O, grid, RS.block, ctx->stream));
+        if (!fresh) {
+            HIP_TRY(ctx, gs_launch_traj(q.model, full, false, B.params, 1, nullptr, O, grid, RS.block, ctx->stream));
+            launched = grid;
+        }
         if (tail)
             HIP_TRY(ctx, queue_tail(tail_lanes(ctx), 0, 1, q.model, full, false, B.params, 1, nullptr, O, fresh ? q.n_particles : 0,
                                     ctx->d_spill, ctx->d_spill + ctx->cap_spill, cap_tail, B.meta + 4, ctx->stream));
@@ -1019,8 +1023,8 @@ gs_status run_plain_core(gs_ctx *ctx, const gs_params &pp, gs_spectrum *out, gs_
     ctx->stats.lane_cycles = H.stats[gs::ST_CYCLES] * (uint64_t)gs::kWave * gs::kCycleSteps;
     ctx->stats.max_particle_steps = H.stats[gs::ST_MAX_STEPS];
     ctx->stats.active_cycles = H.stats[gs::ST_STEPS];
-    ctx->stats.grid_blocks = grid;
-    ctx->stats.block_threads = RS.block;
+    ctx->stats.grid_blocks = launched;
+    ctx->stats.block_threads = launched ? RS.block : 0;
     if (out->n_acc_overflow) return fail(ctx, GS_ERR_OVERFLOW, "weight accumulator overflow");
     return GS_OK;
 }

@@ -163,10 +163,12 @@ typedef struct gs_exit_record {
 typedef struct gs_run_stats {
     double kernel_ms;        /* trajectory kernel time (HIP events)          */
     double total_ms;         /* whole call                                   */
-    uint64_t lane_cycles;    /* lane-cycles issued (active + idle)           */
+    uint64_t lane_cycles;    /* lane-cycles issued (active + idle); a tail launch's lanes */
+                             /* beyond one per particle count as idle        */
     uint64_t active_cycles;  /* lane-cycles with a live particle             */
-    uint32_t grid_blocks;
-    uint32_t block_threads;
+    uint32_t grid_blocks;    /* workgroups of the throughput launch (batch: of all of  */
+    uint32_t block_threads;  /* them), and their size; 0: none, tail launches took all */
+                             /* particles                                    */
     uint64_t max_particle_steps; /* plain runs: most steps of one particle     */
 } gs_run_stats;
 

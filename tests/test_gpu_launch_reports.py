@@ -1,5 +1,4 @@
-"""What a run says that it launched, and which launch shapes it uses: those that a
-caller sets and the autotuner measures are the ones that run."""
+"""What a run says that it launched."""
 import pytest
 
 from geliosphere_amd import abi
