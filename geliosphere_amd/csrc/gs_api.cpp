@@ -78,7 +78,7 @@ struct gs_ctx {
     // (256 threads, the occupancy's blocks per CU, kChunk ids per grab)
     gs_launch_shape shape[2][4] = {};
     bool asked[2][4] = {};          // set by the caller (not by the autotuner or its cache): used as it is
-    bool tuning = false;            // the autotuner measures shapes as they are
+    bool tuning = false;            // the autotuner is timing a shape
     double tuned_rate[2][4] = {};   // particle-steps/s of the tuned shapes (0: not tuned)
     std::string arch;               // gcnArchName of the device
     // the device's fixed scratch array (gs_run_plain_noalloc), looked up once
@@ -434,8 +434,9 @@ uint64_t tail_cap(const gs_ctx *ctx, uint64_t n, uint64_t traj_lanes) {
 }
 
 // Whether every run makes the throughput launch, in the launch shape as it is: a
-// caller who sets a shape chooses how the kernel runs; a tuned shape is a default.
-bool shape_rules(const gs_ctx *ctx, int kernel, int model) { return ctx->asked[kernel][model]; }
+// caller who sets a shape chooses how the kernel runs, and the autotuner times the
+// kernel it tunes; a tuned shape is a default.
+bool shape_rules(const gs_ctx *ctx, int kernel, int model) { return ctx->tuning || ctx->asked[kernel][model]; }
 
 // Workgroups of the throughput launch for n particles: as the shape says, but no
 // more than two waves per SIMD, or one for every kLaneParticles particles per lane.
@@ -456,7 +457,7 @@ constexpr uint64_t kLaneParticles = 16;
 // launches (cap 500: B-p 3,000,000 6.4 / 4.2 ms, Geliosphere 20.4 / 18.6).
 constexpr uint64_t kSpreadSteps = 16384, kHandOnSteps = 512;
 unsigned throughput_grid(const gs_ctx *ctx, int model, const Resolved &R, uint64_t n) {
-    if (model == GS_MODEL_1D_FP || ctx->tuning || shape_rules(ctx, GS_KERNEL_PLAIN, model)) return R.grid;
+    if (model == GS_MODEL_1D_FP || shape_rules(ctx, GS_KERNEL_PLAIN, model)) return R.grid;
     const uint64_t waves = std::max<uint64_t>(2, n / (kLaneParticles * tail_lanes(ctx)));
     return (unsigned)std::min<uint64_t>(R.grid, waves * tail_lanes(ctx) / R.block);
 }

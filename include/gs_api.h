@@ -290,7 +290,9 @@ gs_status gs_set_order(gs_ctx *ctx, int32_t mode);
  * gs_run_batch), best of `repeats` runs per shape, rated by particle-steps
  * per second of trajectory-kernel time.  Search: blocks per CU from 1 to the
  * occupancy at 256 threads; then 128 and 512 threads at about the same waves
- * per CU and at their occupancy; then 16, 32, 128 and 256 ids per grab.  The
+ * per CU and at their occupancy; then 16, 32, 128 and 256 ids per grab.  Every
+ * timed run makes the kernel's launch, for any number of particles; its time
+ * includes the tail launches that end the run, so pilots should be large.  The
  * best shape is applied (gs_set_launch_shape) and kept for gs_autotune_save.
  * best_shape / best_steps_per_s may be NULL.  With the environment variable
  * GS_AUTOTUNE_LOG set (not "0"), each measured shape and its rate is printed
