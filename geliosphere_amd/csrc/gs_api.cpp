@@ -1456,7 +1456,7 @@ gs_status gs_run_plain_noalloc(gs_ctx *ctx, const gs_params *p, gs_spectrum *out
 
 gs_status gs_debug_math(gs_ctx *ctx, int32_t fn, const double *x, double *y, uint64_t n) {
     if (!ctx || (!x && fn != GS_DBG_NORMALS) || !y) return GS_ERR_INVALID_ARG;
-    if (fn < GS_DBG_RCP || fn > GS_DBG_RSQRT4) return fail(ctx, GS_ERR_INVALID_ARG, "unknown fn");
+    if (fn < GS_DBG_RCP || fn > GS_DBG_RSQRT4_MID) return fail(ctx, GS_ERR_INVALID_ARG, "unknown fn");
     if (!x) return GS_ERR_INVALID_ARG;
     if (n == 0) return GS_OK;
     HIP_TRY(ctx, hipSetDevice(ctx->device));
