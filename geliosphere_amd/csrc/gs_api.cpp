@@ -430,11 +430,11 @@ const uint64_t kMaxChunk = 1ull << 27;
 const uint64_t kOrderMinParticles = 4096;   // smaller runs keep id order
 // Tail launches (tail_kernel): after the throughput launch of a run, or instead
 // of it where the particles fit one lane each at one wave per SIMD.  Launch r
-// has kTailBudget << r cycles, the last one as many as it takes: lifetimes
-// spread over three decades, and a doubling budget repacks the survivors
-// about every time their number has halved.  Every launch is queued beforehand
-// and takes its particle count from the one before on the device; one that
-// finds none ends at once (about 3 us).
+// has tail_budget(r) cycles, the last one as many as it takes: lifetimes spread over
+// three decades, and a budget that grows by sqrt(2) repacks the survivors about twice
+// each time their number has halved.  Every launch is queued beforehand and takes its
+// particle count from the one before on the device; one that finds none ends at once
+// (about 3 us).
 constexpr int kTailRounds = 21;
 constexpr uint32_t tail_budget(int r) { return (r & 1 ? 181u : 128u) << (r >> 1); }
 
@@ -455,12 +455,13 @@ bool shape_rules(const gs_ctx *ctx, int kernel, int model) { return ctx->tuning 
 // more than two waves per SIMD, or one for every kLaneParticles particles per lane.
 // With few particles per lane the launch's end is the run's: a lane of five waves
 // a SIMD takes a B-p step in 626 ns, one of two in 297, and what is left when the
-// ids run out is as long in steps either way.  B-p, five waves / two, in ms:
-// 500,000 particles 32 / 23, 1,000,000 44.5 / 37.5, 2,000,000 72 / 69; from there on
-// more waves (3,000,000: 98.5, 100.6, three 96.9).  Geliosphere, three / two:
-// 300,000 239 / 224, 1,000,000 83 / 79.  1D F-p ends on a few lone particles with
-// any number of waves.  (Plain runs only: a batch's groups fill each other's gaps;
-// there it cost a fifth.)
+// ids run out is as long in steps either way.  The shape's waves / two, kernel time in
+// ms: B-p (dt 500 s) 200,000 particles 19.5 / 18.6, 500,000 28.8 / 23.5, 1,000,000 43.2 /
+// 37.2, 2,000,000 70.8 / 66.2, 3,000,000 94.5 / 97.0; SolarProp (dt 100 s) 300,000 192 /
+// 184, 1,000,000 289 / 265, 2,000,000 439 / 400; Geliosphere (dt 100 s) 259 / 254, 377 /
+// 359, 599 / 565, and 1,000,000 at dt 500 s 80.7 / 75.5.  1D F-p ends on a few lone
+// particles with any number of waves.  (Plain runs only: a batch's groups fill each
+// other's gaps; there it cost a fifth.)
 constexpr uint64_t kLaneParticles = 16;
 // Few waves, and tail launches after a throughput launch, are for lifetimes that
 // differ; under a step cap most particles end at the cap, at once.  Below kSpreadSteps
@@ -613,9 +614,11 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
 namespace {
 
 // One sub-batch: the simulations of `part` (indices into sims), grouped by
-// model (groups of larger total work first, costlier particles first within
-// a group), one persistent launch per <= kBatchMaxSims simulations, the model
-// groups on concurrent streams, then one fold launch over all simulations.
+// model (groups of less total work first: their tails wait for the others' launches;
+// costlier particles first within a group; 1D simulations without branch-free steps
+// apart), one persistent launch per <= kBatchMaxSims simulations, or tail launches
+// alone for few particles, the groups on concurrent streams, then one fold launch over
+// all simulations.
 // The launch sequence is captured into a hipGraph once per layout and
 // replayed while the layout (counts, grids, buffers) stays the same.
 gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<uint32_t> &part,
@@ -798,7 +801,7 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
             if (!tail) O.spill = nullptr;
             if (!fresh[l]) {
                 // One throughput launch after another (each fills the device; the
-                // tail of one overlaps the next): with all at once the group with
+                // tails of all run side by side as the last one drains): with all at once the group with
                 // the longest tail got its share of the slots last.
                 if (after) e = hipStreamWaitEvent(sg, ctx->traj[after - 1], 0);
                 if (e == hipSuccess)

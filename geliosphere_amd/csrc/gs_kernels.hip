@@ -644,8 +644,9 @@ __global__ void __launch_bounds__(kTailThreads) tail_kernel(const DevParams *__r
     if (threadIdx.x < kWaves) stage.count[threadIdx.x] = 0;
     load_bm_tables(&bm);
     __syncthreads();
-    // A tail runs beside other launches' throughput waves in a batch: its
-    // waves, on the critical path and at most one per SIMD, issue first.
+    // In a batch a tail runs beside what is left of other launches' throughput
+    // waves: its waves, on the critical path and at most one per SIMD, issue first.
+    // (It starts where those have left registers for it.)
     __builtin_amdgcn_s_setprio(3);
     const int sub = lane & (g - 1), group = lane / g;
     const uint64_t idx = (block * kWaves + wave) * per_wave + group;
@@ -1152,22 +1153,22 @@ using namespace gs;
 // the 1D kernels reach 4 waves unasked).  Measured: SolarProp at 4 waves (128
 // VGPRs) spills and runs 5 % slower.
 #ifndef GS_BATCH_WAVES_GE
-#define GS_BATCH_WAVES_GE 2   // 227 VGPRs, no spills; at 3 waves 62 spill and the batch ran 12 % slower
+#define GS_BATCH_WAVES_GE 2   // 235 VGPRs, no spills; at 3 waves 62 spilled and the batch ran 12 % slower (227 VGPRs, before branch-free cycles)
 #endif
 #ifndef GS_PLAIN_WAVES_1D
 #define GS_PLAIN_WAVES_1D 1
 #endif
 #ifndef GS_PLAIN_WAVES_BP
-#define GS_PLAIN_WAVES_BP 5   // 96 VGPRs, no spills: +3 % over the 98-VGPR, 4-wave shape
+#define GS_PLAIN_WAVES_BP 5   // 90 VGPRs, no spills (96 before branch-free cycles, +3 % over 98 VGPRs and 4 waves)
 #endif
 #ifndef GS_PLAIN_WAVES_GE
-#define GS_PLAIN_WAVES_GE 3   // 154 VGPRs, no spills
+#define GS_PLAIN_WAVES_GE 3   // 164 VGPRs, no spills
 #endif
 #ifndef GS_PLAIN_WAVES_SP
 #define GS_PLAIN_WAVES_SP 3   // 163 VGPRs, no spills (169 unasked)
 #endif
 #ifndef GS_BATCH_WAVES_BP
-#define GS_BATCH_WAVES_BP 5   // 96 VGPRs (17 spilled); 4 waves (121, none) ran 0.8 % faster on 32 B-p simulations at 30 % of the batch benchmark's counts, not switched: the tuned batch shapes were measured at 5
+#define GS_BATCH_WAVES_BP 5   // 96 VGPRs (26 spilled); before branch-free cycles 4 waves (121, none spilled; 17 at 5) ran 0.8 % faster on 32 B-p simulations at 30 % of the batch benchmark's counts, not switched: the tuned batch shapes were measured at 5
 #endif
 constexpr int kBatchWaves1D = 1, kBatchWavesBp = GS_BATCH_WAVES_BP, kBatchWavesSp = 2, kBatchWavesGe = GS_BATCH_WAVES_GE;
 constexpr int kPlainWavesBp = GS_PLAIN_WAVES_BP;

@@ -163,8 +163,8 @@ __global__ void __launch_bounds__(256) gemm_kernel(GemmArgs g) {
 //    operations per element): see silu_of_quarter.
 // RT row tiles of 16 by NW waves, chosen by sg_launch_mlp_forward.  Four waves per SIMD: two
 // (four waves of 64 columns each) gave 195 us instead of 160 for 65,536 rows of
-// four members.  There the products alone take 114 us, near the rate of a large
-// matrix product, and the activations 48 us beside them; before, with IEEE
+// four members.  There the products alone take 114 us (947 TFLOP/s; a large matrix
+// product reaches 1,297 on this card) and the activations 48 us; before, with IEEE
 // divisions, 2-byte LDS writes and two k steps of loads, 190 us.  Ping-pong tiles
 // with the activations of one row tile scheduled into the products of the next
 // (twice the LDS, half the rows) gave 174 us, wave priorities nothing.
@@ -389,7 +389,7 @@ __global__ void adam_kernel(float *P, const float *G, float *Mo, float *Ve, __bf
 //    (forward and backward give a lane the same elements).  What the weight
 //    gradients need goes out in their fragment order (frag_at, along the rows).
 //  - train_weights_kernel forms every layer's weight gradient (a wave takes
-//    32 x 32 elements over the whole minibatch, operands straight from L2)
+//    32 x 16 elements over the whole minibatch, operands straight from L2)
 //    and bias gradient, and applies Adam to them where they are: the gradient
 //    never goes to memory.
 // 16 rows: at 512 rows x 4 members 128 workgroups.  16 waves (20.9 us at 8, 38 at
