@@ -72,3 +72,18 @@ def test_launches_of_changing_size(engine):
         assert bytes(engine.run_plain(p)[0]) == bytes(whole)
     finally:
         engine.set_plain_limits()
+
+
+def test_batches_of_more_groups_than_streams(engine):
+    """Six groups: four models, and both 1D models without branch-free steps; in
+    throughput launches (70,000 particles) and in tail launches."""
+    for n in (35_000, 300):
+        sims = []
+        for i in range(2):
+            sims.append(abi.make_params(abi.MODEL_1D_BP, N=n, seed=20 + i, max_steps=300 + i, **NONE))
+            sims.append(abi.make_params(abi.MODEL_1D_FP, N=n, seed=40 + i, dt=6e5))
+            for m in (abi.MODEL_1D_FP, abi.MODEL_1D_BP, abi.MODEL_2D_SOLARPROP, abi.MODEL_2D_GELIOSPHERE):
+                sims.append(abi.make_params(m, N=n + i, seed=60 + 10 * m + i, dt=500.0, r_inj=80.0, T_min=0.3))
+        want = [bytes(engine.run_plain_noalloc(p)) for p in sims]
+        for _ in range(3):   # the captured graph again
+            assert [bytes(o) for o in engine.run_batch(sims)] == want
