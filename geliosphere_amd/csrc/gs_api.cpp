@@ -482,9 +482,10 @@ unsigned throughput_grid(const gs_ctx *ctx, int model, const Resolved &R, uint64
 // word per launch, zeroed.
 // all_lanes: one wave per SIMD of the device.  part of parts: the share of the
 // device that a batch's model group takes once its particles fit there.
-hipError_t queue_tail(uint64_t all_lanes, int part, int parts, int model, bool full, bool batch, const DevParams *sims, uint32_t n_sims,
-                      const uint64_t *offsets, const DevOut &O, uint64_t fresh_n, gs::SpillRec *half0,
-                      gs::SpillRec *half1, uint64_t cap, uint64_t *counts, hipStream_t s) {
+hipError_t queue_tail(uint64_t all_lanes, int part, int parts, int model, bool full, bool batch,
+                      const DevParams *sims, uint32_t n_sims, const uint64_t *offsets, const DevOut &O,
+                      uint64_t fresh_n, gs::SpillRec *half0, gs::SpillRec *half1, uint64_t cap, uint64_t *counts,
+                      hipStream_t s) {
     const uint64_t most = fresh_n ? fresh_n : cap;
     const uint32_t xcds = gs::kXcds / (uint32_t)parts;
     const uint64_t lanes = all_lanes * xcds / gs::kXcds;
@@ -801,8 +802,8 @@ gs_status run_sub_batch(gs_ctx *ctx, const gs_params *sims, const std::vector<ui
             if (!tail) O.spill = nullptr;
             if (!fresh[l]) {
                 // One throughput launch after another (each fills the device; the
-                // tails of all run side by side as the last one drains): with all at once the group with
-                // the longest tail got its share of the slots last.
+                // tails of all run side by side as the last one drains): with all at
+                // once the group with the longest tail got its share of the slots last.
                 if (after) e = hipStreamWaitEvent(sg, ctx->traj[after - 1], 0);
                 if (e == hipSuccess)
                     e = gs_launch_traj(L.model, L.full, true, ctx->d_params + L.base, L.count, ctx->d_meta + L.off_pos, O,
